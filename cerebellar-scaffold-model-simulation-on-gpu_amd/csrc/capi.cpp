@@ -54,6 +54,28 @@ static int check_ready(scaffold_env *env)
 // r < freq/sec*DT with freq a float promoted to double (UserInputFunctions.cu:4-6).
 static double poisson_thr(float hz) { return (double)hz / kSec * kDT; }
 
+// The draws v whose uniform number 2^-32 + v * 2^-32 (rounded to float as the kernel
+// rounds it) lies below thr: it does not fall as v grows, so they are 0 .. *cut.
+// False when there are none.
+static bool draws_below(double thr, uint32_t *cut)
+{
+    const float inv = 2.3283064365386963e-10f;
+    auto below = [&](uint32_t v) {
+        const float p = (float)v * inv;
+        return (double)(inv + p) < thr;
+    };
+    *cut = 0;
+    if (!below(0u)) return false;
+    uint32_t lo = 0u, hi = 0xFFFFFFFFu;  // below(lo); the answer lies in [lo, hi]
+    while (lo < hi) {
+        const uint32_t mid = lo + (hi - lo) / 2 + 1;
+        if (below(mid)) lo = mid;
+        else hi = mid - 1;
+    }
+    *cut = lo;
+    return true;
+}
+
 static ScStim make_dev_stim(const Stimulus &s)
 {
     ScStim d{};
@@ -75,6 +97,8 @@ static ScStim make_dev_stim(const Stimulus &s)
     d.sine_off = s.f.sine_off;
     d.sine_cycle = s.f.sine_cycle_s;
     d.sine_shift = s.f.sine_shift;
+    d.p_any = draws_below(d.p_thr, &d.p_cut) ? 1 : 0;
+    d.b_any = draws_below(d.b_thr, &d.b_cut) ? 1 : 0;
     return d;
 }
 
@@ -505,6 +529,13 @@ int scaffold_set_option(scaffold_env *env, const char *key, int64_t value)
         if (frozen) return frozen_err();
         if (value < -1 || value > 1) return fail(SCAFFOLD_ERR_INVALID_ARG, "nontemporal is -1, 0 or 1");
         o.nontemporal = (int)value;
+    } else if (!strcmp(key, "resident")) {
+        if (frozen) return frozen_err();
+        o.resident = value ? 1 : 0;
+    } else if (!strcmp(key, "run_polls")) {
+        if (frozen) return frozen_err();
+        if (value < 0 || value > (1 << 30)) return fail(SCAFFOLD_ERR_INVALID_ARG, "run_polls in [0, 2^30]");
+        o.run_polls = (int)value;
     } else return fail(SCAFFOLD_ERR_INVALID_ARG, "unknown option %s", key);
     return SCAFFOLD_OK;
 }
@@ -528,6 +559,8 @@ int scaffold_get_option(scaffold_env *env, const char *key, int64_t *value)
     else if (!strcmp(key, "word_groups")) *value = o.word_groups;
     else if (!strcmp(key, "stage_ratio")) *value = o.stage_ratio;
     else if (!strcmp(key, "nontemporal")) *value = o.nontemporal;
+    else if (!strcmp(key, "resident")) *value = o.resident;
+    else if (!strcmp(key, "run_polls")) *value = o.run_polls;
     else return fail(SCAFFOLD_ERR_INVALID_ARG, "unknown option %s", key);
     return SCAFFOLD_OK;
 }

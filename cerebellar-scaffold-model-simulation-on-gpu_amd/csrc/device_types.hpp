@@ -94,6 +94,10 @@ struct ScStim {
     float   sine_max;            // sinusoidal Poisson peak rate, Hz (0 = off)
     double  sine_on, sine_off;
     float   sine_cycle, sine_shift;   // period (s), phase (rad)
+    // the thresholds on the 32-bit draws themselves: a draw v is below p_thr (b_thr)
+    // exactly when v <= p_cut (b_cut); p_any / b_any 0: no draw is
+    uint32_t p_cut, b_cut;
+    int32_t p_any, b_any;
 };
 
 struct ScCtl {
@@ -103,6 +107,8 @@ struct ScCtl {
     int32_t recount;  // 1: the ring changed outside the step sequence (initialization,
                       // reset, a jump of the step count); the plasticity window counts
                       // of the next run are recomputed from the ring, not updated
+    int32_t failed;   // a resident run gave up: the kernels behind it do nothing
+    int32_t skipped;  // steps of the runs skipped since (the host launches them again)
 };
 
 // 64-neuron groups per wavefront of the plasticity window-count class
@@ -173,7 +179,6 @@ struct ScStimTask {        // 64 neurons of an INPUT population
 #define SC_LDS_GLOBAL ((int32_t)0x80000000)
 
 struct ScTeamIn {          // one incoming projection of a team-mode neuron
-    int32_t end;           // end of its segment in the merged row (32-bit form; informational)
     int32_t delay, exc;
     int32_t lds;           // staged blocks: LDS word that stands for word 0 of the ring row,
                            // or SC_LDS_GLOBAL
@@ -203,8 +208,13 @@ struct ScTeamTask {        // one neuron of a team-mode population
     const uint32_t *grp;   // the neuron's word groups (4 words each; nullptr: none)
     int32_t inst, group, bit, pop;
     int32_t n_in, wprec, len, n_grp;
+    // the part of the row (entries; 16-bit form: chunks) and of the word groups that
+    // holds projections of two or more steps of delay; one-step projections follow
+    int32_t len_e, n_grp_e;
     ScTeamIn in[SC_MAX_IN];
+    int32_t pad_[6];
 };
+static_assert(sizeof(ScTeamTask) == 256, "a team descriptor is two whole 128-byte lines");
 
 // Block layout of the step kernel (a kernel argument).  Blocks are grouped in
 // classes: team neurons of width 16, 8, 4, 2, 1 wavefronts (classes 0..4, with
@@ -219,6 +229,53 @@ struct ScLayout {
     int32_t cls_end[SC_CLASSES];    // cumulative block count at the end of each class
     int32_t cls_ntask[SC_CLASSES];  // tasks of each class
     int32_t cls_task0[SC_CLASSES];  // first descriptor index of each class
+    int32_t lane_per, stim_per;     // lane and stimulus groups per block (at most 16)
+};
+
+// What one block of a resident run waits for before step k of the run: each entry
+// names the blocks [b0, b0 + cnt) that own the presynaptic neurons its tasks read
+// and the delay at which they read them (those blocks must have finished step
+// k - delay).  Entries [0, n_early) are waited for before the block's gathers,
+// entries [n_early, n) -- a team block's one-step projections -- only before those
+// gathers.  The first entry of a team block is of the SC_DEP_ONCE kind: before it
+// sets its first spike bit of step 1 those blocks must have finished step 0, in
+// which they cleared its spike words of the run's later rows.
+//
+// Every block has a 128-byte line of its own: word 0 holds its progress (steps since
+// initialization that it has finished), words 1 .. SC_MAIL of a team block the spike
+// bits of its (at most 16) neurons in its last SC_MAIL steps, each with its step:
+// (progress after the step) << 16 | bits, at word 1 + progress % SC_MAIL.  Where
+// `mail` is set, the one-step entries are read from these instead of the ring row:
+// block b0 + i owns the `per` neurons from device bit bit0 + i * per on, and word w
+// of the ring row (32-bit words [w0, w1) are staged) stands at LDS word lds + w.
+#define SC_DEP_ONCE  (-1)
+#define SC_RUN_BLOCKS 256  // blocks of a resident run on a whole MI355X (one per CU)
+// Fewest steps of a call worth a resident run: its start (tables, the first fetch of its
+// code, the cleared rows) and its end (every block waits for all) cost some 25 us, 2.2
+// us a step are gained (48k cells: 8 steps 217 against 207 us, 25 steps 144 against 200).
+#define SC_RUN_MIN   16
+#define SC_MAX_DEP   20
+#define SC_MAIL      4
+#define SC_MAIL_MOST 192  // most blocks whose mail a block reads
+#define SC_TAG_WORDS 16
+struct ScDep {
+    int32_t b0, cnt, delay;
+    int32_t bit0, per, w0, w1, lds;
+};
+struct ScDeps {
+    int32_t n_early, n, mail, pad_;
+    ScDep e[SC_MAX_DEP];
+};
+
+// A resident run (kernel argument): its steps, the blocks' progress tags (SC_TAG_WORDS
+// apart), the count of blocks that finished it (zero before the run; the top bit
+// gives it up), a host word set when it is given up, and the most polls of a wait.
+struct ScRun {
+    const ScDeps *deps;
+    unsigned long long *tags;
+    uint32_t *done;
+    uint32_t *host_failed;
+    int32_t K, polls;
 };
 
 // State of one device neuron: one 16-byte record, read and written by one load

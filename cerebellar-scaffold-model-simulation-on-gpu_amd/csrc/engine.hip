@@ -80,8 +80,19 @@ struct RunGraphs {
     }
 };
 
+// Resident runs of an engine (k_run): what its launches share.
+struct RunSync {
+    const ScDeps *deps = nullptr;        // per block; nullptr: the network's runs launch a kernel per step
+    unsigned long long *tags = nullptr;  // progress of each block, SC_TAG_WORDS apart
+    uint32_t *done = nullptr;
+    uint32_t *failed_h = nullptr, *failed_hd = nullptr;  // host word a given-up run sets, and its device address
+    int max_steps = 0;                   // longest run whose rows the ring holds beside those it reads
+    int polls = 0;                       // most polls of one wait
+};
+
 struct Engine {
     hipStream_t stream = nullptr;
+    RunSync run;
     std::vector<void *> allocs;
     int64_t bytes = 0;
     ScInstance hi{};
@@ -92,6 +103,7 @@ struct Engine {
     std::vector<ScStimTask> h_stims;
     std::vector<ScTeamTask> h_teams;
     std::vector<int> h_team_t;  // team width (wavefronts) of each team task
+    std::vector<int> h_team_b;  // its width in a batch
     std::vector<TaskWin> h_lane_win, h_team_win;
     ScStim *stims = nullptr;
     int n_stims = 0;
@@ -110,6 +122,7 @@ struct Engine {
     uint8_t *out_hd = nullptr;  // the device's address of out_h (mapped pinned memory), nullptr: copy instead
     hipEvent_t train_ev = nullptr;  // recorded once a call's output train is in out_h (with out_hd)
     int n_out = 0, T_out = 0;
+    size_t out_bytes = 0;  // the train's bytes in out_h, in whole 64-byte lines (64 more bytes follow)
     // plastic projections: multiplier array and per-synapse index, for read-back
     struct PlasticView {
         int proj;
@@ -146,13 +159,13 @@ static int scratch_on_current_device(int32_t **out)
 }
 
 template <typename T>
-static int dalloc(std::vector<void *> &allocs, int64_t *bytes, T **p, size_t count)
+static int dalloc(std::vector<void *> &allocs, int64_t *bytes, T **p, size_t count, bool clear = true)
 {
     size_t b = sizeof(T) * (count ? count : 1);
     void *q = nullptr;
     HIP_TRY(hipMalloc(&q, b));
     allocs.push_back(q);
-    HIP_TRY(hipMemset(q, 0, b));
+    if (clear) HIP_TRY(hipMemset(q, 0, b));
     if (bytes) *bytes += (int64_t)b;
     *p = static_cast<T *>(q);
     return SCAFFOLD_OK;
@@ -161,7 +174,7 @@ static int dalloc(std::vector<void *> &allocs, int64_t *bytes, T **p, size_t cou
 template <typename T>
 static int dupload(std::vector<void *> &allocs, int64_t *bytes, T **p, const std::vector<T> &v)
 {
-    int rc = dalloc(allocs, bytes, p, v.size());
+    int rc = dalloc(allocs, bytes, p, v.size(), v.empty());
     if (rc) return rc;
     if (!v.empty()) HIP_TRY(hipMemcpy(*p, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice));
     return SCAFFOLD_OK;
@@ -184,9 +197,12 @@ static int wbytes_of(int wprec) { return wprec == SC_W_F32 ? 4 : wprec == SC_W_B
 // the longest rows start earliest), then lane groups, then stimulus groups, then
 // the plasticity rules' window-count groups, 16 wavefronts per block.  `team_t` lists the team width of every team descriptor,
 // widest first.
-static ScLayout make_layout(const std::vector<int> &team_t, int n_lanes, int n_stims, int n_hist, int *n_blocks)
+static ScLayout make_layout(const std::vector<int> &team_t, int n_lanes, int n_stims, int n_hist, int lane_per,
+                            int stim_per, int *n_blocks)
 {
     ScLayout L{};
+    L.lane_per = lane_per;
+    L.stim_per = stim_per;
     int blocks = 0;
     size_t i = 0;
     for (int c = 0; c < SC_CLASS_LANE; ++c) {
@@ -200,10 +216,10 @@ static ScLayout make_layout(const std::vector<int> &team_t, int n_lanes, int n_s
         i = j;
     }
     L.cls_ntask[SC_CLASS_LANE] = n_lanes;
-    blocks += (n_lanes + SC_LANE_PER_BLOCK - 1) / SC_LANE_PER_BLOCK;
+    blocks += (n_lanes + lane_per - 1) / lane_per;
     L.cls_end[SC_CLASS_LANE] = blocks;
     L.cls_ntask[SC_CLASS_STIM] = n_stims;
-    blocks += (n_stims + SC_STIM_PER_BLOCK - 1) / SC_STIM_PER_BLOCK;
+    blocks += (n_stims + stim_per - 1) / stim_per;
     L.cls_end[SC_CLASS_STIM] = blocks;
     L.cls_ntask[SC_CLASS_HIST] = n_hist;
     blocks += (n_hist + SC_BLOCK / SC_WAVE - 1) / (SC_BLOCK / SC_WAVE);
@@ -234,7 +250,7 @@ static std::vector<ScStage> plan_stages(const ScLayout &L, int n_blocks, std::ve
         const bool lane = c == SC_CLASS_LANE;
         const int b0 = c ? L.cls_end[c - 1] : 0;
         for (int b = b0; b < L.cls_end[c]; ++b) {
-            const int bi = b - b0, per = lane ? SC_LANE_PER_BLOCK : 1 << c;
+            const int bi = b - b0, per = lane ? L.lane_per : 1 << c;
             const int first = (lane ? 0 : L.cls_task0[c]) + bi * per;
             const int count = std::min(per, L.cls_ntask[c] - bi * per);
             ScWin wins[MAXK];
@@ -323,10 +339,140 @@ static std::vector<ScStage> plan_stages(const ScLayout &L, int n_blocks, std::ve
     return st;
 }
 
+// The wait tables of a network's resident runs (one per block): which blocks own the
+// presynaptic neurons of each projection a block reads, from the bit ranges of its
+// tasks (neurons of a population are assigned to tasks, and tasks to blocks, in
+// ascending order, so a bit range belongs to a range of blocks).  Entries past the
+// table's size widen the last one of their kind: waiting for more blocks, or for a
+// later step of them, is always allowed.
+static std::vector<ScDeps> plan_deps(const ScLayout &L, int n_blocks, int Ndev, const std::vector<ScLaneTask> &lanes,
+                                     const std::vector<TaskWin> &lane_win, const std::vector<ScTeamTask> &teams,
+                                     const std::vector<TaskWin> &team_win, const std::vector<ScStimTask> &stims,
+                                     const std::vector<ScStage> &stages)
+{
+    std::vector<int32_t> owner((size_t)Ndev, -1);  // block of each device neuron
+    struct Part { int first, count; };
+    auto part_of = [&](int c, int b) {
+        const int bi = b - (c ? L.cls_end[c - 1] : 0);
+        const int per = c == SC_CLASS_LANE ? L.lane_per : c == SC_CLASS_STIM ? L.stim_per : 1 << c;
+        return Part{(c < SC_CLASS_LANE ? L.cls_task0[c] : 0) + bi * per, std::min(per, L.cls_ntask[c] - bi * per)};
+    };
+    for (int c = 0; c <= SC_CLASS_STIM; ++c)
+        for (int b = c ? L.cls_end[c - 1] : 0; b < L.cls_end[c]; ++b) {
+            const Part p = part_of(c, b);
+            for (int i = p.first; i < p.first + p.count; ++i) {
+                if (c < SC_CLASS_LANE) { owner[teams[i].group * SC_WAVE + teams[i].bit] = b; continue; }
+                const int g = c == SC_CLASS_LANE ? lanes[i].group : stims[i].group;
+                const int nv = c == SC_CLASS_LANE ? lanes[i].nvalid : stims[i].nvalid;
+                for (int l = 0; l < nv; ++l) owner[g * SC_WAVE + l] = b;
+            }
+        }
+    std::vector<ScDeps> deps((size_t)n_blocks);
+    for (int c = 0; c <= SC_CLASS_LANE; ++c)
+        for (int b = c ? L.cls_end[c - 1] : 0; b < L.cls_end[c]; ++b) {
+            const bool lane = c == SC_CLASS_LANE;
+            const Part p = part_of(c, b);
+            std::vector<ScDep> kind[2];  // longer delays, one-step delays of team neurons
+            if (!lane) {
+                int lo = n_blocks, hi = -1;
+                for (int i = p.first; i < p.first + p.count; ++i) {
+                    const int o = owner[teams[i].group * SC_WAVE];
+                    lo = std::min(lo, o);
+                    hi = std::max(hi, o);
+                }
+                kind[0].push_back(ScDep{lo, hi - lo + 1, SC_DEP_ONCE, 0, 0, 0, 0, 0});
+            }
+            for (int i = p.first; i < p.first + p.count; ++i) {
+                const TaskWin &W = lane ? lane_win[i] : team_win[i];
+                for (int r = 0; r < W.n; ++r) {
+                    if (W.lo[r] > W.hi[r]) continue;
+                    const int b0 = owner[W.lo[r]], b1 = owner[W.hi[r]];
+                    std::vector<ScDep> &v = kind[!lane && W.delay[r] < 2];
+                    bool in = false;
+                    for (ScDep &x : v) {
+                        // ranges of one delay that overlap or touch are one entry
+                        if (x.delay != W.delay[r] || b0 > x.b0 + x.cnt || b1 + 1 < x.b0) continue;
+                        const int e = std::max(x.b0 + x.cnt, b1 + 1);
+                        x.b0 = std::min(x.b0, b0);
+                        x.cnt = e - x.b0;
+                        in = true;
+                        break;
+                    }
+                    if (!in) v.push_back(ScDep{b0, b1 - b0 + 1, W.delay[r], 0, 0, 0, 0, 0});
+                }
+            }
+            ScDeps &D = deps[(size_t)b];
+            for (int k = 0; k < 2; ++k) {
+                const int most = SC_MAX_DEP / 2;
+                for (size_t i = 0; i < kind[k].size(); ++i) {
+                    const ScDep &x = kind[k][i];
+                    if ((int)i < most) { D.e[D.n++] = x; continue; }
+                    ScDep &y = D.e[D.n - 1];
+                    const int e = std::max(y.b0 + y.cnt, x.b0 + x.cnt);
+                    y.b0 = std::min(y.b0, x.b0);
+                    y.cnt = e - y.b0;
+                    y.delay = std::min(y.delay, x.delay);
+                }
+                if (k == 0) D.n_early = D.n;
+            }
+            // mail: every one-step entry names team blocks of one width that hold whole
+            // ranges of one population's neurons, and the block's one-step windows are
+            // staged, one per entry
+            D.mail = !lane && D.n > D.n_early && kind[1].size() <= SC_MAX_DEP / 2;
+            int n_late_win = 0;
+            for (int w = 0; w < (stages.empty() ? 0 : stages[b].n); ++w) n_late_win += stages[b].w[w].delay < 2;
+            if (n_late_win != D.n - D.n_early) D.mail = 0;
+            std::vector<char> taken(SC_MAX_WIN, 0);
+            for (int i = D.n_early; i < D.n && D.mail; ++i) {
+                ScDep &x = D.e[i];
+                int cls = -1;
+                for (int j = 0; j < x.cnt && D.mail; ++j) {
+                    int cj = 0;
+                    while (x.b0 + j >= L.cls_end[cj]) ++cj;
+                    if (j == 0) cls = cj;
+                    D.mail = cj == cls && cj < SC_CLASS_LANE;
+                    if (!D.mail) break;
+                    const Part q = part_of(cj, x.b0 + j);
+                    for (int n = q.first; n < q.first + q.count && D.mail; ++n) {
+                        const int bit = teams[n].group * SC_WAVE + teams[n].bit;
+                        if (j == 0 && n == q.first) {
+                            x.bit0 = bit;
+                            x.per = 1 << cj;
+                            D.mail = x.bit0 % x.per == 0;
+                        }
+                        D.mail = D.mail && bit == x.bit0 + j * x.per + (n - q.first);
+                    }
+                }
+                if (!D.mail) break;
+                D.mail = 0;
+                const int lo = x.bit0 >> 5, hi = (x.bit0 + x.cnt * x.per - 1) >> 5;
+                for (int w = 0; w < stages[b].n; ++w) {
+                    const ScWin &win = stages[b].w[w];
+                    if (win.delay >= 2 || taken[w] || win.w0 + win.nw <= lo || win.w0 > hi) continue;
+                    taken[w] = 1;
+                    D.mail = 1;
+                    x.w0 = win.w0;
+                    x.w1 = win.w0 + win.nw;
+                    x.lds = win.off - win.w0;
+                    break;
+                }
+            }
+            int n_mail = 0;
+            for (int i = D.n_early; i < D.n; ++i) n_mail += D.e[i].cnt;
+            if (n_mail > SC_MAIL_MOST) D.mail = 0;
+            // every projection of the block's teams with a one-step delay is staged
+            for (int i = p.first; i < p.first + p.count && D.mail; ++i)
+                for (int r = 0; r < team_win[i].n; ++r)
+                    if (team_win[i].delay[r] < 2 && teams[i].in[r].lds == SC_LDS_GLOBAL) D.mail = 0;
+        }
+    return deps;
+}
+
 static int upload_work(std::vector<void *> &allocs, int64_t *bytes, DevWork &w, const std::vector<int> &team_t,
                        std::vector<ScLaneTask> lanes, const std::vector<ScStimTask> &stims,
                        std::vector<ScTeamTask> teams, const std::vector<TaskWin> &lane_win,
-                       const std::vector<TaskWin> &team_win, bool stage, int ratio, int n_hist)
+                       const std::vector<TaskWin> &team_win, bool stage, int ratio, int n_hist,
+                       int most_blocks)
 {
     for (size_t i = 1; i < team_t.size(); ++i)
         if (team_t[i] > team_t[i - 1]) return fail(SCAFFOLD_ERR_STATE, "team descriptors not ordered by width");
@@ -336,11 +482,24 @@ static int upload_work(std::vector<void *> &allocs, int64_t *bytes, DevWork &w, 
     ScLaneTask *l;
     ScStimTask *s;
     ScTeamTask *t;
-    w.layout = make_layout(team_t, (int)lanes.size(), (int)stims.size(), n_hist, &w.n_blocks);
+    w.layout = make_layout(team_t, (int)lanes.size(), (int)stims.size(), n_hist, SC_LANE_PER_BLOCK, SC_STIM_PER_BLOCK,
+                           &w.n_blocks);
+    // a network that leaves CUs idle is cut into smaller blocks of lane and stimulus
+    // groups (the neuron update and the Philox draws keep the vector units of their
+    // CU busy), as small as still fit the chip at once
+    for (int per = 4; per < SC_LANE_PER_BLOCK && w.n_blocks < most_blocks; per *= 2) {
+        int n = 0;
+        const ScLayout l = make_layout(team_t, (int)lanes.size(), (int)stims.size(), n_hist, per, per, &n);
+        if (n > most_blocks) continue;
+        w.layout = l;
+        w.n_blocks = n;
+        break;
+    }
     int n_staged = 0;
     std::vector<ScStage> st;
     if (stage) st = plan_stages(w.layout, w.n_blocks, lanes, lane_win, teams, team_win, ratio, &n_staged);
     w.stages = nullptr;
+    w.h_stages = st;
     w.n_staged = n_staged;
     if (n_staged > 0) {
         ScStage *ds;
@@ -350,6 +509,7 @@ static int upload_work(std::vector<void *> &allocs, int64_t *bytes, DevWork &w, 
     if ((rc = dupload(allocs, bytes, &l, lanes))) return rc;
     if ((rc = dupload(allocs, bytes, &s, stims))) return rc;
     if ((rc = dupload(allocs, bytes, &t, teams))) return rc;
+    w.h_teams = teams;  // with the staging plan's LDS words
     w.lanes = l;
     w.stims = s;
     w.teams = t;
@@ -357,6 +517,36 @@ static int upload_work(std::vector<void *> &allocs, int64_t *bytes, DevWork &w, 
     w.idx16 = false;
     for (const ScLaneTask &x : lanes) w.idx16 = w.idx16 || x.idx16;
     for (const ScTeamTask &x : teams) w.idx16 = w.idx16 || x.hdr;
+    return SCAFFOLD_OK;
+}
+
+// Sets up resident runs where the network allows them: the option is on, no
+// plasticity rule (its update kernel runs between steps), a grid that the device
+// holds at once, and a ring with room for at least SC_RUN_MIN new rows beside those
+// the steps read.
+static int engine_plan_run(Engine *e, const Plan &P)
+{
+    if (!P.resident || !e->w.plastic.empty() || e->w.n_blocks <= 0) return SCAFFOLD_OK;
+    if ((int64_t)P.Wr * P.R >= (int64_t)1 << 30) return SCAFFOLD_OK;  // ring words are counted in 32 bits
+    e->run.max_steps = P.R - P.max_delay - 2;
+    if (e->run.max_steps < SC_RUN_MIN) return SCAFFOLD_OK;
+    int rc, most = 0;
+    if ((rc = run_capacity(e->w.idx16, &most))) return rc;
+    if (e->w.n_blocks > most) return SCAFFOLD_OK;
+    // the status word follows the output train in its pinned buffer
+    if (!e->out_hd) return SCAFFOLD_OK;  // no device address for host memory: a kernel per step
+    e->run.failed_h = reinterpret_cast<uint32_t *>(e->out_h + e->out_bytes);
+    e->run.failed_hd = reinterpret_cast<uint32_t *>(e->out_hd + e->out_bytes);
+    // (the count of finished blocks has a line of its own after the blocks' lines)
+    if ((rc = dalloc(e->allocs, &e->bytes, &e->run.tags, (size_t)(e->w.n_blocks + 1) * SC_TAG_WORDS))) return rc;  // zeroed
+    e->run.done = reinterpret_cast<uint32_t *>(e->run.tags + (size_t)e->w.n_blocks * SC_TAG_WORDS);
+    ScDeps *d;
+    if ((rc = dupload(e->allocs, &e->bytes, &d,
+                      plan_deps(e->w.layout, e->w.n_blocks, e->Ndev, e->h_lanes, e->h_lane_win, e->w.h_teams,
+                                e->h_team_win, e->h_stims, e->w.h_stages))))
+        return rc;
+    e->run.deps = d;
+    e->run.polls = P.run_polls;
     return SCAFFOLD_OK;
 }
 
@@ -495,7 +685,10 @@ int engine_create(Engine **out, Plan &P)
             d.wprec = T.wprec;
             // 16-bit form: the padded group length; 32-bit: the synapse count
             d.len = T.idx16 ? (int)(T.row_ptr[j + 1] - T.row_ptr[j])  // chunks
-                            : (pp.n_in ? T.seg_end[(size_t)j * pp.n_in + pp.n_in - 1] : 0);
+                            : 0;
+            for (int q = 0; q < pp.n_in && !T.idx16; ++q) d.len = std::max(d.len, T.seg_end[(size_t)j * pp.n_in + q]);
+            d.len_e = T.len_e[j];
+            d.n_grp_e = T.grp_e[j];
             d.n_grp = (int)(T.grp_ptr[j + 1] - T.grp_ptr[j]);
             d.grp = d.n_grp ? tgrp[ti] + 4 * T.grp_ptr[j] : nullptr;
             TaskWin tw;
@@ -509,7 +702,6 @@ int engine_create(Engine **out, Plan &P)
                 tw.qsegs[q] = T.q_seg[(size_t)j * pp.n_in + q];
                 tw.lo[q] = T.q_lo[(size_t)j * pp.n_in + q];
                 tw.hi[q] = T.q_hi[(size_t)j * pp.n_in + q];
-                d.in[q].end = T.seg_end[(size_t)j * pp.n_in + q];
                 d.in[q].delay = sp.delay;
                 d.in[q].exc = sp.exc;
                 d.in[q].W = sp.W;
@@ -517,6 +709,7 @@ int engine_create(Engine **out, Plan &P)
             }
             e->h_teams.push_back(d);
             e->h_team_t.push_back(T.team_waves);
+            e->h_team_b.push_back(T.batch_waves);
             e->h_team_win.push_back(tw);
         } else if (t.kind == SC_TASK_LANE) {
             const ScGroup &G = P.groups[t.group];
@@ -569,8 +762,10 @@ int engine_create(Engine **out, Plan &P)
         const int groups = (P.pops[P.projs[X.rule.target].pre_pop].num + SC_WAVE - 1) / SC_WAVE;
         n_hist += (groups + SC_HIST_GROUPS - 1) / SC_HIST_GROUPS;  // wavefronts of the window-count class
     }
+    int most_blocks = 0;
+    if ((rc = run_capacity(P.index_bits == 16, &most_blocks))) return bail(rc);
     if ((rc = upload_work(A, B, e->w, e->h_team_t, e->h_lanes, e->h_stims, e->h_teams, e->h_lane_win, e->h_team_win,
-                          P.stage != 0, P.stage_ratio, n_hist)))
+                          P.stage != 0, P.stage_ratio, n_hist, most_blocks)))
         return bail(rc);
     // plasticity rules: per-synapse arrays; the multipliers they update are the
     // f32 arrays of the target's lane slices or merged rows
@@ -631,10 +826,11 @@ int engine_create(Engine **out, Plan &P)
         if ((rc = dupload(A, B, &ob, P.out_bits))) return bail(rc);
         e->out_bits = ob;
         const size_t nb = (size_t)e->T_out * (size_t)std::max(1, e->n_out);
+        e->out_bytes = (nb + 63) / 64 * 64;
         if ((rc = dalloc(A, B, &e->out_d, nb))) return bail(rc);
-        if (hipHostMalloc(reinterpret_cast<void **>(&e->out_h), nb, hipHostMallocMapped) != hipSuccess)
+        if (hipHostMalloc(reinterpret_cast<void **>(&e->out_h), e->out_bytes + 64, hipHostMallocMapped) != hipSuccess)
             return bail(fail(SCAFFOLD_ERR_HIP, "hipHostMalloc of the output train failed"));
-        memset(e->out_h, 0, nb);
+        memset(e->out_h, 0, e->out_bytes + 64);
         // the gather writes the train straight into the mapped pinned buffer (no
         // separate device-to-host copy); where the runtime gives no device address
         // for it, the train is gathered on the device and copied
@@ -644,10 +840,43 @@ int engine_create(Engine **out, Plan &P)
         if (e->out_hd && hipEventCreateWithFlags(&e->train_ev, hipEventDisableTiming) != hipSuccess)
             return bail(fail(SCAFFOLD_ERR_HIP, "hipEventCreate failed"));
     }
+    if ((rc = engine_plan_run(e, P))) return bail(rc);
     std::vector<ScInstance> one{I};
     if ((rc = dupload(A, B, &e->di, one))) return bail(rc);
     *out = e;
     return SCAFFOLD_OK;
+}
+
+// Resident runs of different streams of one device follow each other: two of them
+// side by side could each hold CUs the other's blocks need.  The stream of the last
+// run on each device; another stream's next run first waits for the work that stream
+// holds then.
+static std::mutex g_run_mu;
+static hipStream_t g_run_last[kMaxDevices] = {};
+
+static int run_order(hipStream_t s)
+{
+    int dev = 0;
+    HIP_TRY(hipGetDevice(&dev));
+    if (dev < 0 || dev >= kMaxDevices) return fail(SCAFFOLD_ERR_CAPACITY, "device %d beyond the run table", dev);
+    if (g_run_last[dev] && g_run_last[dev] != s) {
+        LocalEvents L;
+        hipEvent_t ev;
+        int rc = L.make(&ev);
+        if (rc) return rc;
+        HIP_TRY(hipEventRecord(ev, g_run_last[dev]));
+        HIP_TRY(hipStreamWaitEvent(s, ev, 0));
+    }
+    g_run_last[dev] = s;
+    return SCAFFOLD_OK;
+}
+
+// The stream is idle and about to be destroyed.
+static void run_order_forget(hipStream_t s)
+{
+    std::lock_guard<std::mutex> lock(g_run_mu);
+    for (hipStream_t &x : g_run_last)
+        if (x == s) x = nullptr;
 }
 
 void engine_destroy(Engine *e)
@@ -657,6 +886,7 @@ void engine_destroy(Engine *e)
     e->graphs.destroy();
     for (void *p : e->allocs) (void)hipFree(p);
     if (e->out_h) (void)hipHostFree(e->out_h);
+    run_order_forget(e->stream);
     if (e->train_ev) (void)hipEventDestroy(e->train_ev);
     for (hipEvent_t x : e->kt.pool) (void)hipEventDestroy(x);
     if (e->stream) (void)hipStreamDestroy(e->stream);
@@ -739,9 +969,9 @@ static void launch_step_kernels(hipStream_t s, const ScInstance *single, const S
 }
 
 static void launch_end(hipStream_t s, const ScInstance *single, const ScInstance *insts, int n_inst, const DevWork &w,
-                       int K, const ScOut *out)
+                       int K, const ScOut *out, const RunSync *res = nullptr)
 {
-    launch_run_end(s, single, insts, n_inst, K, w.max_groups, out, w.end_done);
+    launch_run_end(s, single, insts, n_inst, K, w.max_groups, out, w.end_done, res ? res->done : nullptr);
 }
 
 static bool same_out(const ScOut &a, const ScOut &b)
@@ -811,12 +1041,14 @@ static int timer_pair(KTimer *kt, int K, hipEvent_t *a, hipEvent_t *b)
 static int run_steps(hipStream_t s, RunGraphs &G, const ScInstance *single, const ScInstance *insts, int n_inst,
                      const DevWork &w, int n_steps, int use_graph, int chunk, KTimer *kt = nullptr,
                      const ScOut *out = nullptr, bool *out_taken = nullptr, hipEvent_t train_ev = nullptr,
-                     int out_row0 = 0, bool *train_ev_set = nullptr)
+                     int out_row0 = 0, bool *train_ev_set = nullptr, const RunSync *res = nullptr)
 {
     if (out_taken) *out_taken = false;
     if (train_ev_set) *train_ev_set = false;
     if (n_steps <= 0) return SCAFFOLD_OK;
     const bool timer = kt && kt->on;
+    if (res && res->deps && !use_graph && n_steps >= SC_RUN_MIN) chunk = std::min(chunk, res->max_steps);
+    else res = nullptr;
     const int last_k = n_steps % chunk ? n_steps % chunk : chunk;  // steps of the last run
     const ScOut *last_out = out && out->out && out->T > 0 && out->T <= last_k ? out : nullptr;
     int done = 0;
@@ -839,6 +1071,11 @@ static int run_steps(hipStream_t s, RunGraphs &G, const ScInstance *single, cons
                                &ge);
             if (rc) return rc;
             HIP_TRY(hipGraphLaunch(ge, s));
+        } else if (res) {
+            std::lock_guard<std::mutex> lock(g_run_mu);
+            int rc = run_order(s);
+            if (rc) return rc;
+            launch_run(s, *single, w, ScRun{res->deps, res->tags, res->done, res->failed_hd, K, res->polls});
         } else {
             launch_step_kernels(s, single, insts, w, K);
         }
@@ -847,9 +1084,9 @@ static int run_steps(hipStream_t s, RunGraphs &G, const ScInstance *single, cons
             launch_out_train(s, single->ring, single->Wr, single->R, out_row0, o->T, o->bits, o->n_out, o->out);
             HIP_TRY(hipEventRecord(train_ev, s));
             if (train_ev_set) *train_ev_set = true;
-            launch_end(s, single, insts, n_inst, w, K, nullptr);
+            launch_end(s, single, insts, n_inst, w, K, nullptr, res);
         } else if (timed || !graph) {
-            launch_end(s, single, insts, n_inst, w, K, o);
+            launch_end(s, single, insts, n_inst, w, K, o, res);
         }
         HIP_TRY(hipGetLastError());
         done += K;
@@ -860,9 +1097,33 @@ static int run_steps(hipStream_t s, RunGraphs &G, const ScInstance *single, cons
 
 static int chunk_for(int graph_steps, int R) { return std::max(1, std::min(graph_steps, R - 1)); }
 
+// After a resident run was given up (its blocks were not on the device together in
+// time, e.g. beside another process's): nothing of it or of the runs behind it was
+// stored or counted.  Launches their steps again, a kernel per step, as all later
+// ones of this engine will be.
+static int engine_recover(Engine *e, int graph_steps)
+{
+    HIP_TRY(hipStreamSynchronize(e->stream));
+    ScCtl c;
+    HIP_TRY(hipMemcpy(&c, e->hi.ctl, sizeof(c), hipMemcpyDeviceToHost));
+    const int steps = c.skipped;
+    c.failed = c.skipped = 0;
+    HIP_TRY(hipMemcpy(e->hi.ctl, &c, sizeof(c), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemset(e->run.done, 0, sizeof(uint32_t)));
+    HIP_TRY(hipMemset(e->hi.ring + (size_t)c.row * e->hi.Wr, 0, sizeof(uint64_t) * e->hi.Wr));
+    HIP_TRY(hipDeviceSynchronize());  // the fills above, before the engine's (non-blocking) stream goes on
+    *e->run.failed_h = 0u;
+    e->run.deps = nullptr;
+    int rc = run_steps(e->stream, e->graphs, &e->hi, e->di, 1, e->w, steps, 0, chunk_for(graph_steps, e->hi.R));
+    if (rc) return rc;
+    HIP_TRY(hipStreamSynchronize(e->stream));
+    return SCAFFOLD_OK;
+}
+
 // Waits for the engine's stream (or only for `upto`, an event recorded on it after
-// every timer event), then adds what the step-kernel timer measured.
-static int engine_finish(Engine *e, hipEvent_t upto = nullptr)
+// every timer event), then adds what the step-kernel timer measured.  *recovered:
+// a resident run was given up and its steps were launched again.
+static int engine_finish(Engine *e, int graph_steps, hipEvent_t upto = nullptr, bool *recovered = nullptr)
 {
     if (upto) HIP_TRY(hipEventSynchronize(upto));
     else HIP_TRY(hipStreamSynchronize(e->stream));
@@ -875,15 +1136,19 @@ static int engine_finish(Engine *e, hipEvent_t upto = nullptr)
     }
     kt.piece_k.clear();
     kt.used = 0;
+    if (e->run.failed_h && *const_cast<volatile uint32_t *>(e->run.failed_h)) {
+        if (recovered) *recovered = true;
+        return engine_recover(e, graph_steps);
+    }
     return SCAFFOLD_OK;
 }
 
 int engine_run(Engine *e, int n_steps, int use_graph, int graph_steps)
 {
     int rc = run_steps(e->stream, e->graphs, &e->hi, e->di, 1, e->w, n_steps, use_graph,
-                       chunk_for(graph_steps, e->hi.R), &e->kt);
+                       chunk_for(graph_steps, e->hi.R), &e->kt, nullptr, nullptr, nullptr, 0, nullptr, &e->run);
     if (rc) return rc;
-    return engine_finish(e);
+    return engine_finish(e, graph_steps);
 }
 
 int engine_run_output(Engine *e, int n_steps, int use_graph, int graph_steps, int64_t first_out_step,
@@ -908,7 +1173,7 @@ int engine_run_output(Engine *e, int n_steps, int use_graph, int graph_steps, in
     bool taken = false, early_set = false;
     if (!rec) {
         rc = run_steps(e->stream, e->graphs, &e->hi, e->di, 1, e->w, n_steps, use_graph, chunk, &e->kt,
-                       closes ? &out : nullptr, &taken, early, row0, &early_set);
+                       closes ? &out : nullptr, &taken, early, row0, &early_set, &e->run);
         if (rc) return rc;
     }
     for (int done = 0; rec && done < n_steps;) {
@@ -930,7 +1195,17 @@ int engine_run_output(Engine *e, int n_steps, int use_graph, int graph_steps, in
         if (!e->out_hd && nb) HIP_TRY(hipMemcpyAsync(e->out_h, e->out_d, nb, hipMemcpyDeviceToHost, e->stream));
         *train = e->out_h;  // complete once engine_finish has synchronized the stream
     }
-    return engine_finish(e, early_set ? e->train_ev : nullptr);
+    bool recovered = false;
+    if ((rc = engine_finish(e, graph_steps, early_set ? e->train_ev : nullptr, &recovered))) return rc;
+    if (train && recovered) {  // the train of the steps launched again
+        launch_out_train(e->stream, e->hi.ring, e->hi.Wr, R, row0, e->T_out, e->out_bits, e->n_out, out.out);
+        HIP_TRY(hipGetLastError());
+        if (!e->out_hd && (size_t)e->T_out * (size_t)e->n_out)
+            HIP_TRY(hipMemcpyAsync(e->out_h, e->out_d, (size_t)e->T_out * (size_t)e->n_out, hipMemcpyDeviceToHost,
+                                   e->stream));
+        HIP_TRY(hipStreamSynchronize(e->stream));
+    }
+    return SCAFFOLD_OK;
 }
 
 int engine_record_sync(Engine *e, Recorder *rec)
@@ -959,7 +1234,8 @@ int engine_time(Engine *e, int n_steps, int use_graph, int graph_steps, double *
     const int chunk = chunk_for(graph_steps, e->hi.R);
     if (!ms_kernel_mean) {
         HIP_TRY(hipEventRecord(a, e->stream));
-        rc = run_steps(e->stream, e->graphs, &e->hi, e->di, 1, e->w, n_steps, use_graph, chunk, &e->kt);
+        rc = run_steps(e->stream, e->graphs, &e->hi, e->di, 1, e->w, n_steps, use_graph, chunk, &e->kt, nullptr, nullptr,
+                       nullptr, 0, nullptr, &e->run);
         if (rc) return rc;
         HIP_TRY(hipEventRecord(b, e->stream));
     } else {
@@ -999,7 +1275,7 @@ int engine_time(Engine *e, int n_steps, int use_graph, int graph_steps, double *
     float ms = 0.f;
     HIP_TRY(hipEventElapsedTime(&ms, a, b));
     if (ms_total) *ms_total = ms;
-    return engine_finish(e);  // the step-kernel timer's events of this run
+    return engine_finish(e, graph_steps);  // the step-kernel timer's events of this run
 }
 
 int engine_get_state(Engine *e, float *V, float *g, int32_t *refr)
@@ -1188,7 +1464,7 @@ int batch_build(Batch **out, std::vector<Engine *> &engines, const std::vector<c
         for (size_t j = 0; j < e->h_teams.size(); ++j) {
             ScTeamTask t = e->h_teams[j];
             t.inst = (int)i;
-            teams.push_back({e->h_team_t[j], team_win_u.size(), t});
+            teams.push_back({e->h_team_b[j], team_win_u.size(), t});
             team_win_u.push_back(e->h_team_win[j]);
         }
     }
@@ -1204,7 +1480,7 @@ int batch_build(Batch **out, std::vector<Engine *> &engines, const std::vector<c
     int rc;
     if ((rc = dupload(b->allocs, nullptr, &b->di, insts))) return bail(rc);
     if ((rc = upload_work(b->allocs, nullptr, b->w, tw, lanes, stims, tt, lane_win, team_win, stage != 0,
-                          plans[0]->stage_ratio, 0)))
+                          plans[0]->stage_ratio, 0, 0)))
         return bail(rc);
     for (const ScInstance &x : insts) b->w.max_groups = std::max(b->w.max_groups, x.n_groups);
     b->w.nontemporal = nt_all || algo > ((int64_t)64 << 20);

@@ -104,6 +104,15 @@ __device__ __forceinline__ T ldg(gptr<T> p)
     else return *p;
 }
 
+// A 32-bit half of a spike word.  COH: a word other blocks may have written during
+// this launch (resident runs); the load goes past the caches of this CU and XCD.
+template <bool COH>
+__device__ __forceinline__ uint32_t ldring(gptr<uint32_t> p)
+{
+    if constexpr (COH) return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else return *p;
+}
+
 // 4 and 2 dwords loaded by one 16- / 8-byte load.
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
@@ -130,10 +139,11 @@ __device__ __forceinline__ void store_state(ScState *st, int d, float u, float2 
 // address) to LDS at dst + 16 * l, without passing through registers; dst is
 // wave-uniform.  The copy counts as an outstanding vector-memory load of the
 // wavefront until it has been written to LDS.
+template <bool COH = false>  // COH: at device scope (sc1), as ldring
 __device__ __forceinline__ void lds_load16(const u32x4 *src, u32x4 *dst)
 {
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src,
-                                     (__attribute__((address_space(3))) void *)dst, 16, 0, 0);
+                                     (__attribute__((address_space(3))) void *)dst, 16, 0, COH ? 16 : 0);
 }
 
 // Wave-uniform value in a scalar register (descriptor indices derived from the
@@ -348,11 +358,11 @@ __device__ __forceinline__ int lif_step(const PopT &P, float &u, float &g0, floa
 // The spike word holding device bit c of a lane slice: from the ring row in
 // global memory, or in a staged block from its LDS window (lds: the LDS word that
 // stands for word 0 of the row); padding (bit zb) reads LDS word 0, kept zero.
-template <bool STAGED>
+template <bool STAGED, bool COH>
 __device__ __forceinline__ uint32_t spike_word(gptr<uint32_t> row32, const uint32_t *win, int lds, uint32_t c, uint32_t zb)
 {
     if constexpr (STAGED) return win[c == zb ? 0 : lds + (int)(c >> 5)];
-    else return row32[c >> 5];
+    else return ldring<COH>(row32 + (c >> 5));
 }
 
 // 16-bit slices: lane `lane`'s offsets of columns 2p and 2p+1 share the 32-bit
@@ -369,8 +379,8 @@ __device__ __forceinline__ uint32_t pair_bit(uint32_t word, int hi, uint32_t bas
 // load each; 16-bit: four column pairs) and two vectors of multipliers.  Vector
 // indices past the slice are clamped to its last vector and the entries past
 // its width masked out of the sum.  k0 is a multiple of 4.
-template <int WP, bool IDX16, bool STAGED, bool NT>
-__device__ __forceinline__ double slice_tail(const ScSlice &sl, gptr<uint32_t> row32, const uint32_t *win, uint32_t zb,
+template <int WP, bool IDX16, bool STAGED, bool NT, bool COH, typename Slice>
+__device__ __forceinline__ double slice_tail(const Slice &sl, gptr<uint32_t> row32, const uint32_t *win, uint32_t zb,
                                              int k0, int lane)
 {
     double S = 0.0;
@@ -409,7 +419,7 @@ __device__ __forceinline__ double slice_tail(const ScSlice &sl, gptr<uint32_t> r
             }
         }
 #pragma unroll
-        for (int j = 0; j < 8; ++j) w[j] = spike_word<STAGED>(row32, win, sl.lds, c[j], zb);
+        for (int j = 0; j < 8; ++j) w[j] = spike_word<STAGED, COH>(row32, win, sl.lds, c[j], zb);
 #pragma unroll
         for (int j = 0; j < 8; ++j)
             if (k + j < width && ((w[j] >> (c[j] & 31)) & 1u))
@@ -418,13 +428,118 @@ __device__ __forceinline__ double slice_tail(const ScSlice &sl, gptr<uint32_t> r
     return S;
 }
 
-// One 64-neuron group of a lane-mode population: the first 4 columns of every
-// slice are loaded in one batch (one vector of columns and one of multipliers per
-// slice, then all spike words), the neuron state alongside, then the LIF update.
-// In a staged block the window copies are issued (stage()) once the first loads
-// are under way.
-// Slice widths and pointers are wave-uniform; slices without multipliers (unit
-// weights) skip the multiplier loads.
+// One 64-neuron group of a lane-mode population.  LaneHead: the first 4 columns of
+// every slice (one vector of columns and one of multipliers per slice; 16-bit form:
+// offset pairs, and in lane 2s+p the header of pair p of slice s).  Slice widths and
+// pointers are wave-uniform; slices without multipliers (unit weights) skip the
+// multiplier loads.
+template <int WP, bool IDX16>
+struct LaneHead {
+    uint32_t c[SC_MAX_SLICES][IDX16 ? 2 : 4];
+    Raw4<WP> raw[SC_MAX_SLICES];
+    uint32_t hv;
+};
+template <int WP, bool IDX16, bool NT, typename Task>
+__device__ __forceinline__ void lane_head(const Task &t, uint32_t zb, int lane, LaneHead<WP, IDX16> &H)
+{
+    const int n_sl = t.n_sl;
+    H.hv = 0u;
+    if constexpr (IDX16) {
+        const int hs = lane >> 1, hp = lane & 1;
+        const uint32_t *h = nullptr;
+        int w = 0;
+#pragma unroll
+        for (int q = 0; q < SC_MAX_SLICES; ++q)
+            if (hs == q && q < n_sl) {
+                h = t.sl[q].hdr;
+                w = t.sl[q].width;
+            }
+        if (2 * hp < w) H.hv = ldg<NT>(gbl(h) + hp);
+    }
+#pragma unroll
+    for (int s = 0; s < SC_MAX_SLICES; ++s) {
+        const int width = s < n_sl ? t.sl[s].width : 0;
+        const void *val = t.sl[s].val;
+        H.raw[s].w[0] = 0u;
+        if (WP != SC_W_UNIT && val && width > 0) H.raw[s] = wraw4<WP, NT>(val, lane);
+        if constexpr (IDX16) {
+            H.c[s][0] = H.c[s][1] = 0xFFFFFFFFu;
+            if (width > 0) {
+                const u32x2 x = ldg<NT>(gbl(static_cast<const u32x2 *>(t.sl[s].col)) + lane);
+                H.c[s][0] = x.x;
+                H.c[s][1] = x.y;
+            }
+        } else {
+            H.c[s][0] = H.c[s][1] = H.c[s][2] = H.c[s][3] = zb;
+            if (width > 0) {
+                const u32x4 x = ldg<NT>(gbl(static_cast<const u32x4 *>(t.sl[s].col)) + lane);
+                H.c[s][0] = x.x; H.c[s][1] = x.y; H.c[s][2] = x.z; H.c[s][3] = x.w;
+            }
+        }
+    }
+}
+
+// The ring rows that the group's slices read in the step whose ring row is row_n
+// (wave-uniform, one instance per task: held in scalar registers).
+template <typename Task>
+__device__ __forceinline__ void lane_rows(const Task &t, const ScInstance &I, int row_n,
+                                          gptr<uint32_t> (&row)[SC_MAX_SLICES])
+{
+#pragma unroll
+    for (int s = 0; s < SC_MAX_SLICES; ++s) {
+        const int rb = uniform(s < t.n_sl ? row_back(row_n, t.sl[s].delay, I.R) : 0);
+        row[s] = gbl(reinterpret_cast<const uint32_t *>(I.ring + (int64_t)rb * I.Wr));
+    }
+}
+
+// dg of the group's neurons from those rows: the row sums of
+// the head columns of every slice, then of the wider slices' tails (so the head
+// batch's registers are free while a tail runs).
+template <int WP, bool IDX16, bool STAGED, bool NT, bool COH, typename Task>
+__device__ __forceinline__ void lane_dg(const Task &t, const gptr<uint32_t> (&row)[SC_MAX_SLICES], const uint32_t *win,
+                                        const LaneHead<WP, IDX16> &H, uint32_t zb, int lane, float &dge, float &dgi)
+{
+    const int n_sl = t.n_sl;
+    uint32_t c[SC_MAX_SLICES][4], sw[SC_MAX_SLICES][4];
+#pragma unroll
+    for (int s = 0; s < SC_MAX_SLICES; ++s) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if constexpr (IDX16)
+                c[s][k] = pair_bit(H.c[s][k >> 1], k & 1, __builtin_amdgcn_readlane(H.hv, 2 * s + (k >> 1)), zb);
+            else
+                c[s][k] = H.c[s][k];
+            sw[s][k] = spike_word<STAGED, COH>(row[s], win, t.sl[s].lds, c[s][k], zb);
+        }
+    }
+    double S[SC_MAX_SLICES];
+#pragma unroll
+    for (int s = 0; s < SC_MAX_SLICES; ++s) {
+        const bool unit = WP == SC_W_UNIT || !t.sl[s].val;
+        const int width = s < n_sl ? t.sl[s].width : 0;
+        S[s] = 0.0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (k < width && ((sw[s][k] >> (c[s][k] & 31)) & 1u))
+                S[s] += unit ? 1.0 : (double)wval4<WP>(H.raw[s], k);
+    }
+    dge = dgi = 0.f;
+#pragma unroll
+    for (int s = 0; s < SC_MAX_SLICES; ++s) {
+        if (s >= n_sl) break;
+        if (t.sl[s].width > 4) S[s] += slice_tail<WP, IDX16, STAGED, NT, COH>(t.sl[s], row[s], win, zb, 4, lane);
+        // dg[post] += S * w_bar (Simulation_header.cu:98), projections in index order
+        const float Sf = (float)(S[s] * (double)t.sl[s].scale);
+        const float add = Sf * t.sl[s].W;
+        if (t.sl[s].exc) dge = dge + add;
+        else dgi = dgi + add;
+    }
+}
+
+// One step of the group: the head columns and the neuron state are loaded in one
+// batch; in a staged block the window copies are issued (stage()) with those loads
+// in flight and are complete past the block's barrier, which every wavefront of the
+// block reaches once; then the row sums and the LIF update.
 template <int WP, bool IDX16, bool STAGED, bool NT, typename Stage>
 __device__ __forceinline__ void lane_group(const ScLaneTask &t, const ScInstance &I, const ScPop &P, int row_n,
                                            const Stage &stage, int lane)
@@ -436,89 +551,17 @@ __device__ __forceinline__ void lane_group(const ScLaneTask &t, const ScInstance
     float2 gg = {0.f, 0.f};
     int32_t rf = 0;
     if (valid) load_state(I.st, d, u, gg, rf);
-    uint32_t c[SC_MAX_SLICES][4], sw[SC_MAX_SLICES][4];
-    Raw4<WP> raw[SC_MAX_SLICES];
-    uint32_t pw[SC_MAX_SLICES][2];  // 16-bit form: offset pairs
+    LaneHead<WP, IDX16> H;
     gptr<uint32_t> row[SC_MAX_SLICES];
-    const int n_sl = t.n_sl;
-    uint32_t hv = 0u;  // 16-bit form: lane 2s+p holds the header of pair p of slice s
-    if constexpr (IDX16) {
-        const int hs = lane >> 1, hp = lane & 1;
-        const uint32_t *h = nullptr;
-        int w = 0;
-#pragma unroll
-        for (int q = 0; q < SC_MAX_SLICES; ++q)
-            if (hs == q && q < n_sl) {
-                h = t.sl[q].hdr;
-                w = t.sl[q].width;
-            }
-        if (2 * hp < w) hv = ldg<NT>(gbl(h) + hp);
-    }
-#pragma unroll
-    for (int s = 0; s < SC_MAX_SLICES; ++s) {
-        const bool on = s < n_sl;
-        const int width = on ? t.sl[s].width : 0;
-        // wave-uniform (one instance per task): held in scalar registers
-        const int rb = uniform(on ? row_back(row_n, t.sl[s].delay, I.R) : 0);
-        row[s] = gbl(reinterpret_cast<const uint32_t *>(I.ring + (int64_t)rb * I.Wr));
-        const void *val = t.sl[s].val;
-        raw[s].w[0] = 0u;
-        if (WP != SC_W_UNIT && val && width > 0) raw[s] = wraw4<WP, NT>(val, lane);
-        if constexpr (IDX16) {
-            pw[s][0] = pw[s][1] = 0xFFFFFFFFu;
-            if (width > 0) {
-                const u32x2 x = ldg<NT>(gbl(static_cast<const u32x2 *>(t.sl[s].col)) + lane);
-                pw[s][0] = x.x;
-                pw[s][1] = x.y;
-            }
-        } else {
-            c[s][0] = c[s][1] = c[s][2] = c[s][3] = zb;
-            if (width > 0) {
-                const u32x4 x = ldg<NT>(gbl(static_cast<const u32x4 *>(t.sl[s].col)) + lane);
-                c[s][0] = x.x; c[s][1] = x.y; c[s][2] = x.z; c[s][3] = x.w;
-            }
-        }
-    }
-    // staged block: the window copies are issued now, with the first loads in
-    // flight, and are complete past the block's barrier, which every wavefront
-    // of the block reaches once
+    lane_head<WP, IDX16, NT>(t, zb, lane, H);
+    lane_rows(t, I, row_n, row);
     const uint32_t *win = nullptr;
     if constexpr (STAGED) {
         win = stage();
         __syncthreads();
     }
-#pragma unroll
-    for (int s = 0; s < SC_MAX_SLICES; ++s)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            if constexpr (IDX16)
-                c[s][k] = pair_bit(pw[s][k >> 1], k & 1, __builtin_amdgcn_readlane(hv, 2 * s + (k >> 1)), zb);
-            sw[s][k] = spike_word<STAGED>(row[s], win, t.sl[s].lds, c[s][k], zb);
-        }
-    // row sums of the first 4 columns of every slice, then the wider slices' tails
-    // (so the head batch's registers are free while a tail runs)
-    double S[SC_MAX_SLICES];
-#pragma unroll
-    for (int s = 0; s < SC_MAX_SLICES; ++s) {
-        const bool unit = WP == SC_W_UNIT || !t.sl[s].val;
-        const int width = s < n_sl ? t.sl[s].width : 0;
-        S[s] = 0.0;
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-            if (k < width && ((sw[s][k] >> (c[s][k] & 31)) & 1u))
-                S[s] += unit ? 1.0 : (double)wval4<WP>(raw[s], k);
-    }
-    float dge = 0.f, dgi = 0.f;
-#pragma unroll
-    for (int s = 0; s < SC_MAX_SLICES; ++s) {
-        if (s >= n_sl) break;
-        if (t.sl[s].width > 4) S[s] += slice_tail<WP, IDX16, STAGED, NT>(t.sl[s], row[s], win, zb, 4, lane);
-        // dg[post] += S * w_bar (Simulation_header.cu:98), projections in index order
-        const float Sf = (float)(S[s] * (double)t.sl[s].scale);
-        const float add = Sf * t.sl[s].W;
-        if (t.sl[s].exc) dge = dge + add;
-        else dgi = dgi + add;
-    }
+    float dge, dgi;
+    lane_dg<WP, IDX16, STAGED, NT, false>(t, row, win, H, zb, lane, dge, dgi);
     int spk = 0;
     if (valid) {
         spk = lif_step(P, u, gg.x, gg.y, rf, dge, dgi);
@@ -552,11 +595,16 @@ struct TeamHead {
     const uint32_t *grp;
     int32_t inst, group, bit, pop, n_in, wprec, len, n_grp;
 };
-__device__ __forceinline__ TeamHead team_head(const ScTeamTask *T)
+template <typename Task>
+__device__ __forceinline__ TeamHead team_head(const Task &T)
 {
-    return TeamHead{T->col, T->hdr, T->val, T->grp, T->inst, T->group, T->bit, T->pop, T->n_in, T->wprec, T->len,
-                    T->n_grp};
+    return TeamHead{T.col, T.hdr, T.val, T.grp, T.inst, T.group, T.bit, T.pop, T.n_in, T.wprec, T.len, T.n_grp};
 }
+// The part of a team's row a gather covers: word groups [g0, g1), entries (16-bit
+// form: chunks) [e0, e1).
+struct TeamPart {
+    int32_t g0, g1, e0, e1;
+};
 
 // One multiplier (index i of a row's array) in storage WP.
 template <int WP>
@@ -578,26 +626,31 @@ __device__ __forceinline__ float wone(const void *val, uint32_t i)
 // team's f64 LDS accumulator of the projection, as in the merged rows.
 #define SC_GROUP_BATCH 1
 #define SC_GROUP_LOADS 4
-template <int WP, bool STAGED, bool NT>
-__device__ __forceinline__ void team_groups(const TeamHead &T, gptr<uint32_t> ring32, const uint32_t *win,
-                                            const uint32_t *rowoff, uint32_t gmask, int tid, int TT, double *acc)
+template <int WP, bool STAGED, bool NT, bool COH>
+__device__ __forceinline__ void team_groups(const TeamHead &T, const TeamPart &part, gptr<uint32_t> ring32,
+                                            const uint32_t *win, const uint32_t *rowoff, uint32_t gmask, int tid,
+                                            int TT, double *acc, u32x4 rec0)
 {
     constexpr int GB = SC_GROUP_BATCH;
     gptr<u32x4> grp = gbl(reinterpret_cast<const u32x4 *>(T.grp));
     const void *val = T.val;
-    const int n = T.n_grp;
-    for (int b = tid; b < n; b += TT * GB) {
+    const int n = part.g1;
+    for (int b = part.g0 + tid; b < n; b += TT * GB) {
         u32x4 g[GB];
+        if (COH && b == part.g0 + tid) {
+            g[0] = rec0;  // (a resident run keeps each lane's first record)
+        } else {
 #pragma unroll
-        for (int u = 0; u < GB; ++u) g[u] = ldg<NT>(grp + min(b + u * TT, n - 1));
+            for (int u = 0; u < GB; ++u) g[u] = ldg<NT>(grp + min(b + u * TT, n - 1));
+        }
         uint32_t lo[GB], hi[GB];
 #pragma unroll
         for (int u = 0; u < GB; ++u) {
             const uint32_t q = g[u].x >> SC_Q_SHIFT, wi = rowoff[q] + 2u * (g[u].x & SC_BIT_MASK);
             lo[u] = hi[u] = 0u;
             if (!STAGED || (gmask != 0u && ((gmask >> q) & 1u))) {
-                if (g[u].z) lo[u] = ring32[wi];
-                if (g[u].w) hi[u] = ring32[wi + 1];
+                if (g[u].z) lo[u] = ldring<COH>(ring32 + wi);
+                if (g[u].w) hi[u] = ldring<COH>(ring32 + wi + 1);
             } else {
                 if (g[u].z) lo[u] = win[wi];
                 if (g[u].w) hi[u] = win[wi + 1];
@@ -633,19 +686,19 @@ __device__ __forceinline__ void team_groups(const TeamHead &T, gptr<uint32_t> ri
     }
 }
 
-template <int WP, int U, bool IDX16, bool STAGED, bool NT>
-__device__ __forceinline__ void team_gather(const TeamHead &T, gptr<uint32_t> ring32, const uint32_t *win,
-                                            const uint32_t *rowoff, uint32_t gmask, uint32_t zb, int tid, int TT,
-                                            double *acc)
+template <int WP, int U, bool IDX16, bool STAGED, bool NT, bool COH>
+__device__ __forceinline__ void team_gather(const TeamHead &T, const TeamPart &part, gptr<uint32_t> ring32,
+                                            const uint32_t *win, const uint32_t *rowoff, uint32_t gmask, uint32_t zb,
+                                            int tid, int TT, double *acc)
 {
-    const int len = T.len;
+    const int len = part.e1;
     const void *val = T.val;
     if constexpr (IDX16) {
         // 16-bit form: T.len chunks of 8 entries; a lane takes one chunk a batch
         // (one 16-byte load of offsets, its header word and its multipliers)
         gptr<u32x4> col = gbl(static_cast<const u32x4 *>(T.col));
         gptr<uint32_t> hdr = gbl(T.hdr);
-        for (int b = tid; b < len; b += TT) {
+        for (int b = part.e0 + tid; b < len; b += TT) {
             const u32x4 x = ldg<NT>(col + b);
             const uint32_t h = ldg<NT>(hdr + b);
             const Raw8<WP> raw = wraw8<WP, NT>(val, b);
@@ -662,7 +715,7 @@ __device__ __forceinline__ void team_gather(const TeamHead &T, gptr<uint32_t> ri
             // chunk's projection was left in memory (gmask; one projection per chunk)
             if (!STAGED || (gmask != 0u && ((gmask >> q) & 1u))) {
 #pragma unroll
-                for (int i = 0; i < 8; ++i) s[i] = ring32[ro + (bit[i] >> 5)];
+                for (int i = 0; i < 8; ++i) s[i] = ldring<COH>(ring32 + ro + (bit[i] >> 5));
             } else {
 #pragma unroll
                 for (int i = 0; i < 8; ++i) s[i] = win[pad[i] ? 0u : ro + (bit[i] >> 5)];
@@ -677,7 +730,7 @@ __device__ __forceinline__ void team_gather(const TeamHead &T, gptr<uint32_t> ri
         constexpr int V = U / 4;  // vectors per batch
         gptr<u32x4> col = gbl(static_cast<const u32x4 *>(T.col));
         const int nv = (len + 3) >> 2;
-        for (int b = tid; b < nv; b += TT * V) {
+        for (int b = (part.e0 >> 2) + tid; b < nv; b += TT * V) {
             uint32_t c[V][4], s[V][4];
             Raw4<WP> raw[V];
 #pragma unroll
@@ -692,21 +745,18 @@ __device__ __forceinline__ void team_gather(const TeamHead &T, gptr<uint32_t> ri
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const uint32_t wi = rowoff[c[u][i] >> SC_Q_SHIFT] + ((c[u][i] & SC_BIT_MASK) >> 5);
-                    s[u][i] = STAGED ? win[wi] : ring32[wi];
+                    s[u][i] = STAGED ? win[wi] : ldring<COH>(ring32 + wi);
                 }
 #pragma unroll
             for (int u = 0; u < V; ++u)
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
-                    if (4 * (b + u * TT) + i < len && ((s[u][i] >> (c[u][i] & 31)) & 1u))
+                    if (4 * (b + u * TT) + i < len && (!COH || 4 * (b + u * TT) + i >= part.e0) && ((s[u][i] >> (c[u][i] & 31)) & 1u))
                         atomicAdd(&acc[c[u][i] >> SC_Q_SHIFT], (double)wval4<WP>(raw[u], i));
         }
     }
 }
 
-// Whether one stimulus entry fires in exchange step n (draw index m):
-// InputStimulation (UserInputFunctions.cu:94-118) with the rule of ScStim.  The
-// three Philox blocks of the step run interleaved, round by round.
 // Cosine of a float argument, rounded once to float.  Cody-Waite reduction by
 // pi/2 = HI + LO (HI has 33 significant bits, so k*HI and x - k*HI are exact for
 // |k| < 2^20; pi/2 - HI - LO < 4e-27), then the Taylor series of cos and sin on
@@ -741,6 +791,25 @@ __device__ __forceinline__ double stim_sine_thr(float t, float max, float cycle,
     return (double)rate / kSec * kDT;
 }
 
+// Whether a window [on, off) holds the whole step from sub-step time t0 to t1 (1),
+// none of it (0), or a part (-1).
+__device__ __forceinline__ int window_of_step(double on, double off, double t0, double t1)
+{
+    if (on <= t0 && t1 < off) return 1;
+    return (t1 < on || t0 >= off) ? 0 : -1;
+}
+
+// Whether one stimulus entry fires in exchange step n (draw index m):
+// InputStimulation (UserInputFunctions.cu:94-118) with the rule of ScStim.  The
+// three Philox blocks of the step run interleaved, round by round.  Their 10 draws
+// are the sub-steps' own; an entry fires when one of them is below the threshold of
+// a component active in its sub-step.  In nearly every step the Poisson and burst
+// windows hold all sub-steps or none and no other component is active: then the
+// smallest draw decides, compared as an integer (the thresholds' draws, p_cut and
+// b_cut, come from the host), in about half the instructions.  A launch per step is as
+// fast either way (9.8 us at 96.7k cells); in a resident run, which the stimulus
+// blocks paced at 4-8 us a step, it takes them to 1.5-2 us.  Otherwise the sub-steps
+// are taken one by one.
 __device__ __forceinline__ int stim_fires(const ScStim &S, int entry, int64_t n, int64_t m)
 {
     const uint64_t blk = (uint64_t)(3 * m);
@@ -756,8 +825,18 @@ __device__ __forceinline__ int stim_fires(const ScStim &S, int entry, int64_t n,
         k0 += 0x9E3779B9u;
         k1 += 0xBB67AE85u;
     }
-    int spk = 0;
     const double nf = (double)(float)n;
+    const double t0 = (double)(float)nf, t1 = (double)(float)(nf + (double)(float)(kStepMax - 1) * kDT);
+    const int wp = S.p_any ? window_of_step(S.poisson_on, S.poisson_off, t0, t1) : 0;
+    const int wb = S.b_any ? window_of_step(S.burst_on, S.burst_off, t0, t1) : 0;
+    const bool periodic = S.periodic_hz != 0.f && S.periodic_on <= t1 &&
+                          (S.periodic_incl ? t0 <= S.periodic_off : t0 < S.periodic_off);
+    const bool sine = S.sine_max != 0.f && S.sine_on <= t1 && t0 < S.sine_off;
+    if (wp >= 0 && wb >= 0 && !periodic && !sine) {
+        const uint32_t v = min(min(min(min(a0, a1), min(a2, a3)), min(min(b0, b1), min(b2, b3))), min(c0, c1));
+        return (wp && v <= S.p_cut) || (wb && v <= S.b_cut);
+    }
+    int spk = 0;
 #pragma unroll 1
     for (int k = 0; k < kStepMax; ++k) {
         const float t = (float)(nf + (double)(float)k * kDT);
@@ -820,34 +899,26 @@ __device__ __forceinline__ const ScInstance &inst_of(const ScInstance &I0, const
     else return insts[i];
 }
 
-// Gather of one team: storage form and multiplier type of its row.
-template <bool IDX16, bool STAGED, bool NT>
-__device__ __forceinline__ void team_dispatch(const TeamHead &T, gptr<uint32_t> ring32, const uint32_t *win,
-                                              const uint32_t *rowoff, uint32_t gm, uint32_t zb, int tid, int TT,
-                                              double *acc)
+// Gather of a part of one team's row: storage form and multiplier type of the row.
+template <int WP, bool IDX16, bool STAGED, bool NT, bool COH>
+__device__ __forceinline__ void team_parts(const TeamHead &T, const TeamPart &part, gptr<uint32_t> ring32,
+                                           const uint32_t *win, const uint32_t *rowoff, uint32_t gm, uint32_t zb,
+                                           int tid, int TT, double *acc, u32x4 rec0)
 {
-    if (T.n_grp > 0) {
-        switch (T.wprec) {
-        case SC_W_F32: team_groups<SC_W_F32, STAGED, NT>(T, ring32, win, rowoff, gm, tid, TT, acc); break;
-        case SC_W_BF16: team_groups<SC_W_BF16, STAGED, NT>(T, ring32, win, rowoff, gm, tid, TT, acc); break;
-        case SC_W_FP8: team_groups<SC_W_FP8, STAGED, NT>(T, ring32, win, rowoff, gm, tid, TT, acc); break;
-        default: team_groups<SC_W_UNIT, STAGED, NT>(T, ring32, win, rowoff, gm, tid, TT, acc); break;
-        }
-    }
-    if (IDX16 && T.hdr) {
-        switch (T.wprec) {
-        case SC_W_F32: team_gather<SC_W_F32, 8, true, STAGED, NT>(T, ring32, win, rowoff, gm, zb, tid, TT, acc); break;
-        case SC_W_BF16: team_gather<SC_W_BF16, 8, true, STAGED, NT>(T, ring32, win, rowoff, gm, zb, tid, TT, acc); break;
-        case SC_W_FP8: team_gather<SC_W_FP8, 8, true, STAGED, NT>(T, ring32, win, rowoff, gm, zb, tid, TT, acc); break;
-        default: team_gather<SC_W_UNIT, 8, true, STAGED, NT>(T, ring32, win, rowoff, gm, zb, tid, TT, acc); break;
-        }
-    } else {
-        switch (T.wprec) {
-        case SC_W_F32: team_gather<SC_W_F32, 8, false, STAGED, NT>(T, ring32, win, rowoff, gm, zb, tid, TT, acc); break;
-        case SC_W_BF16: team_gather<SC_W_BF16, 8, false, STAGED, NT>(T, ring32, win, rowoff, gm, zb, tid, TT, acc); break;
-        case SC_W_FP8: team_gather<SC_W_FP8, 8, false, STAGED, NT>(T, ring32, win, rowoff, gm, zb, tid, TT, acc); break;
-        default: team_gather<SC_W_UNIT, 8, false, STAGED, NT>(T, ring32, win, rowoff, gm, zb, tid, TT, acc); break;
-        }
+    if (part.g1 > part.g0) team_groups<WP, STAGED, NT, COH>(T, part, ring32, win, rowoff, gm, tid, TT, acc, rec0);
+    if (IDX16 && T.hdr) team_gather<WP, 8, true, STAGED, NT, COH>(T, part, ring32, win, rowoff, gm, zb, tid, TT, acc);
+    else team_gather<WP, 8, false, STAGED, NT, COH>(T, part, ring32, win, rowoff, gm, zb, tid, TT, acc);
+}
+template <bool IDX16, bool STAGED, bool NT, bool COH>
+__device__ __forceinline__ void team_dispatch(const TeamHead &T, const TeamPart &part, gptr<uint32_t> ring32,
+                                              const uint32_t *win, const uint32_t *rowoff, uint32_t gm, uint32_t zb,
+                                              int tid, int TT, double *acc, u32x4 rec0 = u32x4{0u, 0u, 0u, 0u})
+{
+    switch (T.wprec) {
+    case SC_W_F32: team_parts<SC_W_F32, IDX16, STAGED, NT, COH>(T, part, ring32, win, rowoff, gm, zb, tid, TT, acc, rec0); break;
+    case SC_W_BF16: team_parts<SC_W_BF16, IDX16, STAGED, NT, COH>(T, part, ring32, win, rowoff, gm, zb, tid, TT, acc, rec0); break;
+    case SC_W_FP8: team_parts<SC_W_FP8, IDX16, STAGED, NT, COH>(T, part, ring32, win, rowoff, gm, zb, tid, TT, acc, rec0); break;
+    default: team_parts<SC_W_UNIT, IDX16, STAGED, NT, COH>(T, part, ring32, win, rowoff, gm, zb, tid, TT, acc, rec0); break;
     }
 }
 
@@ -918,8 +989,9 @@ __device__ __forceinline__ void do_team(const ScInstance &I0, const ScInstance *
         gptr<uint32_t> ring32 = gbl(reinterpret_cast<const uint32_t *>(uniform_ptr(I.ring)));
         const int tid = tw * SC_WAVE + lane, TT = t * SC_WAVE;
         const uint32_t zb = (uint32_t)uniform((I.Wr - 1) * SC_WAVE);
-        if (win) team_dispatch<IDX16, true, NT>(h, ring32, win, rowoff[team], gmask, zb, tid, TT, acc[team]);
-        else team_dispatch<IDX16, false, NT>(h, ring32, win, rowoff[team], 0u, zb, tid, TT, acc[team]);
+        const TeamPart all{0, h.n_grp, 0, h.len};
+        if (win) team_dispatch<IDX16, true, NT, false>(h, all, ring32, win, rowoff[team], gmask, zb, tid, TT, acc[team]);
+        else team_dispatch<IDX16, false, NT, false>(h, all, ring32, win, rowoff[team], 0u, zb, tid, TT, acc[team]);
     }
     __syncthreads();
     float dge = 0.f, dgi = 0.f;
@@ -1126,7 +1198,7 @@ __device__ __forceinline__ void step_body(const ScInstance &I0, const ScInstance
         const int first = L.cls_task0[c] + bi * per, count = min(per, L.cls_ntask[c] - bi * per);
         // wavefronts past the block's teams read the last team's descriptor (unused)
         const ScTeamTask *T = &teams[first + min(wave / t, count - 1)];
-        const TeamHead h = team_head(T);
+        const TeamHead h = team_head(*T);
         ScTeamIn pin{};
         if (lane < SC_MAX_IN) pin = T->in[lane];
         do_team<SINGLE, IDX16, NT>(I0, insts, t, count, h, pin, row_single, k, stage);
@@ -1137,7 +1209,7 @@ __device__ __forceinline__ void step_body(const ScInstance &I0, const ScInstance
         if (item < L.cls_ntask[c]) plastic_hist(I0, plastic, item, row_single, lane);
         return;
     }
-    const int per_block = c == SC_CLASS_LANE ? SC_LANE_PER_BLOCK : SC_STIM_PER_BLOCK;
+    const int per_block = c == SC_CLASS_LANE ? L.lane_per : L.stim_per;
     const int idx = uniform(bi * per_block + wave);
     const bool staged = c == SC_CLASS_LANE && __builtin_amdgcn_readlane((int)sd, (int)(offsetof(ScStage, n) / 4)) > 0;
     if (wave >= per_block || idx >= L.cls_ntask[c]) {
@@ -1194,6 +1266,614 @@ __global__ void __launch_bounds__(SC_BLOCK) __attribute__((amdgpu_waves_per_eu(8
                                                          const ScStage *__restrict__ stages, int k)
 {
     step_body<false, IDX16, NT>(ScInstance{}, insts, L, lanes, stt, teams, stages, nullptr, k);
+}
+
+// ---------------------------------------------------------------- resident runs
+// k_run advances one network by a run of K steps in one launch: every block of the
+// step kernel's layout stays on its CU for the whole run (the grid fits the chip at
+// once) and keeps its neurons' state, descriptors and (lane groups) columns in
+// registers and LDS from step to step.  Blocks do not meet at a barrier per step.
+// Each block publishes a progress tag (steps since initialization that it has
+// finished) on a 128-byte line of its own, and before a step waits only for the
+// blocks that own the presynaptic neurons it reads, at the delay it reads them: a
+// network's long delays let most blocks run ahead, and only the one-step
+// projections chain successive steps.  Ring rows written during the launch are
+// read past the caches (device scope); a run writes each of its rows once and reads
+// back at most max_delay rows, so with K + max_delay + 2 <= R no row is overwritten
+// while another block may still read it.
+//
+// Every wait is bounded.  `done` counts the blocks that finished all K steps; a
+// block whose wait runs out sets its top bit, everyone then leaves, and nobody has
+// stored any state: the blocks store their neurons' state only after `done` has
+// reached the grid size, which a run that was given up cannot reach.  The host then
+// launches the same steps one kernel per step.
+//
+// What bounds a run is the chain of one step of a population that projects onto itself
+// with a one-step delay: the neuron update (1.3 us: one lane per neuron, ~300
+// instructions a lane at ~10 cycles each), its spikes to the other blocks (0.5 us),
+// the gathers.  Hence the split: the longer delays' windows are copied by one
+// wavefront while another updates the neurons, one-step spikes travel in the line
+// that is polled for them instead of through the ring, each lane keeps its first
+// synapse record.  Measured per call of 25 steps, against a launch per step of the
+// same build: 125 against 180 us at 5.8k cells, 149 against 184 at 9.9k, 149 against
+// 198 at 24k, 145 against 200 at 48k (253 blocks).
+#define SC_RUN_GIVEN_UP 0x80000000u
+__device__ __forceinline__ uint32_t ld_agent(const uint32_t *p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ unsigned long long ld_agent(const unsigned long long *p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ void st_agent(T *p, T v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Every vector-memory access this wavefront has issued is complete: its loads (the
+// window copies included) have arrived and its device-scope stores are visible.
+__device__ __forceinline__ void drain() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// A wave-uniform descriptor that the launch does not write, through a pointer that
+// the compiler takes for a new one each time: the fields a step reads are loaded at
+// their use (scalar loads, from the scalar cache) and again in the next step,
+// instead of being held in registers over the whole run.
+#ifdef __HIP_DEVICE_COMPILE__
+#define SC_CONST __attribute__((address_space(4)))
+#else
+#define SC_CONST
+#endif
+template <typename T>
+__device__ __forceinline__ const SC_CONST T &afresh(const T *p)
+{
+    p = uniform_ptr(p);
+#ifdef __HIP_DEVICE_COMPILE__
+    asm volatile("" : "+s"(p));
+#endif
+    return *(const SC_CONST T *)p;
+}
+
+// What the wavefronts of one block share about the run.
+struct RunLds {
+    // wait entries: first block, blocks, delay, and the steps of this run that all of
+    // them are known to have finished
+    int4 dep[SC_MAX_DEP];
+    int4 win[SC_MAX_WIN];  // staged windows: delay, first word in the ring row, words, first word in LDS
+    // the blocks whose mail this block reads: block, LDS word << 5 | bit of its first
+    // neuron (< 0: nothing here reads its neurons), that neuron's ring word, neurons
+    int4 mail[SC_MAIL_MOST];
+    int32_t n_early, n_dep, n_win, n_mail;
+    int32_t stop;
+};
+
+// Gives the run up (any lane): no block that has not counted itself finished will.
+__device__ __forceinline__ void run_give_up(const ScInstance &I, const ScRun &r)
+{
+    __hip_atomic_fetch_or(r.done, SC_RUN_GIVEN_UP, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    st_agent(&I.ctl->failed, 1);
+    __hip_atomic_store(r.host_failed, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// Waits (one wavefront) until the blocks of entries [e0, e1) have finished the steps
+// that step k of the run reads, and sets L->stop when the run was given up.  The
+// entries are checked side by side, one lane each, against what is known; only those
+// that fall short are polled.
+__device__ __forceinline__ void run_wait(const ScInstance &I, const ScRun &r, int e0, int e1, int k,
+                                         unsigned long long m0, RunLds *L, int lane)
+{
+    const int e_mine = e0 + lane;
+    int4 x = {0, 0, 0, 0};
+    if (e_mine < e1) x = L->dep[e_mine];
+    const int need_mine = e_mine >= e1 ? 0 : x.z == SC_DEP_ONCE ? 1 : k - x.z + 1;
+    uint64_t pending = __ballot(need_mine > x.w);
+    while (pending) {
+        const int j = __ffsll((long long)pending) - 1;
+        pending &= pending - 1;
+        const int b0 = __builtin_amdgcn_readlane(x.x, j), cnt = __builtin_amdgcn_readlane(x.y, j);
+        const int need = __builtin_amdgcn_readlane(need_mine, j);
+        for (int polls = 0;; ++polls) {
+            int fin = r.K;  // steps of this run finished by the slowest of this lane's blocks
+            for (int i = lane; i < cnt; i += SC_WAVE) {
+                const unsigned long long t = ld_agent(r.tags + (size_t)(b0 + i) * SC_TAG_WORDS);
+                fin = min(fin, t > m0 ? (int)(t - m0) : 0);
+            }
+            if (__all(fin >= need)) {
+                int f = need;
+                while (f < r.K && __all(fin > f)) ++f;
+                if (lane == 0) L->dep[e0 + j].w = f;
+                break;
+            }
+            if ((polls & 15) == 15 && uniform((int)ld_agent(r.done)) < 0) {
+                if (lane == 0) L->stop = 1;
+                return;
+            }
+            if (polls >= r.polls) {
+                if (lane == 0) {
+                    run_give_up(I, r);
+                    L->stop = 1;
+                }
+                return;
+            }
+        }
+    }
+}
+
+// Counts the block finished and waits for every other one (all wavefronts of the
+// block).  True: the run is complete and its state may be stored.  Either the count
+// reaches the grid size and nobody gives up any more, or somebody replaces it
+// first and it never does.
+__device__ __forceinline__ bool run_complete(const ScInstance &I, const ScRun &r, RunLds *L)
+{
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        __hip_atomic_fetch_add(r.done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (int polls = 0;; ++polls) {
+            uint32_t v = ld_agent(r.done);
+            if (v == gridDim.x) break;
+            if (v & SC_RUN_GIVEN_UP) { L->stop = 1; break; }
+            if (polls >= r.polls &&
+                __hip_atomic_compare_exchange_strong(r.done, &v, v | SC_RUN_GIVEN_UP, __ATOMIC_RELAXED,
+                                                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+                run_give_up(I, r);
+                L->stop = 1;
+                break;
+            }
+            __builtin_amdgcn_s_sleep(1);
+        }
+    }
+    __syncthreads();
+    return L->stop == 0;
+}
+
+// The mail of step k - 1 of this lane's j-th block (its slot's word, whatever is there).
+__device__ __forceinline__ unsigned long long mail_load(const ScRun &r, const RunLds *L, unsigned long long want, int j,
+                                                        int lane)
+{
+    const int i = lane + j * SC_WAVE;
+    if (i >= L->n_mail) return want << 16;
+    return ld_agent(r.tags + (size_t)L->mail[i].x * SC_TAG_WORDS + 1 + (int)(want % SC_MAIL));
+}
+
+// Reads the spikes of step k - 1 (k > 0; one wavefront) from the blocks' mail into the
+// LDS windows of one-step delays, which hold zeros; v0: this lane's first block's mail
+// as loaded earlier.  A block that is already so far ahead that its mail of that step
+// is gone has finished it: its word of the ring row is read instead.
+__device__ __forceinline__ void run_mail(const ScInstance &I, const ScRun &r, uint32_t *win, int k, int row_prev,
+                                         unsigned long long m0, RunLds *L, int lane, unsigned long long v0)
+{
+    const unsigned long long want = m0 + (unsigned long long)k;  // progress after step k - 1
+    const int n = (uniform(L->n_mail) + SC_WAVE - 1) / SC_WAVE;
+#pragma unroll 1
+    for (int j = 0; j < n; ++j) {
+        unsigned long long v = j == 0 ? v0 : mail_load(r, L, want, j, lane);
+        for (int polls = 0; !__all((v >> 16) >= want); ++polls) {
+            if (((polls & 15) == 15 && uniform((int)ld_agent(r.done)) < 0) || polls >= r.polls) {
+                if (lane == 0) {
+                    if (polls >= r.polls) run_give_up(I, r);
+                    L->stop = 1;
+                }
+                return;
+            }
+            if ((v >> 16) < want) v = mail_load(r, L, want, j, lane);
+        }
+        const int i = lane + j * SC_WAVE;
+        if (i < L->n_mail) {
+            const int4 x = L->mail[i];
+            const int at = x.y;
+            if (at >= 0) {
+                uint32_t s = (uint32_t)v & 0xFFFFu;
+                if ((v >> 16) != want)
+                    s = (ld_agent(reinterpret_cast<const uint32_t *>(I.ring + (int64_t)row_prev * I.Wr) + x.z) >> (at & 31)) &
+                        ((1u << x.w) - 1u);
+                if (s) atomicOr(&win[at >> 5], s << (at & 31));
+            }
+        }
+    }
+}
+
+// Publishes that this block has finished step k of the run (one lane).
+__device__ __forceinline__ void run_publish(const ScRun &r, unsigned long long m0, int k)
+{
+    st_agent(r.tags + (size_t)blockIdx.x * SC_TAG_WORDS, m0 + (unsigned long long)k + 1ull);
+}
+
+// Issues the copies of the block's windows into LDS for the step whose ring row is
+// row_n: those of one-step delays (late) or of longer ones, or all; wavefront `wave`
+// of the `waves` that share them.  The windows' table is in LDS: one load brings an
+// entry to each lane.
+enum { RUN_ALL, RUN_EARLY, RUN_LATE };
+template <int WHICH>
+__device__ __forceinline__ void run_stage(const RunLds *L, uint32_t *win_lds, const ScInstance &I, int row_n, int wave,
+                                          int waves, int lane)
+{
+    const int n_win = uniform(L->n_win);
+    const int4 x = L->win[lane & (SC_MAX_WIN - 1)];
+    u32x4 *dst = reinterpret_cast<u32x4 *>(win_lds);
+    const u32x4 *ring = reinterpret_cast<const u32x4 *>(I.ring);
+#pragma unroll 1
+    for (int w = 0; w < n_win; ++w) {
+        const int delay = __builtin_amdgcn_readlane(x.x, w);
+        if (WHICH != RUN_ALL && (delay < 2) != (WHICH == RUN_LATE)) continue;
+        const int n4 = __builtin_amdgcn_readlane(x.z, w) >> 2;
+        const uint32_t s4 = (uint32_t)(row_back(row_n, delay, I.R) * (I.Wr >> 1) + (__builtin_amdgcn_readlane(x.y, w) >> 2));
+        u32x4 *to = dst + (__builtin_amdgcn_readlane(x.w, w) >> 2);
+        for (int cb = wave * SC_WAVE; cb < n4; cb += waves * SC_WAVE)
+            if (cb + lane < n4) lds_load16<true>(ring + (s4 + (uint32_t)(cb + lane)), to + cb);
+    }
+}
+// Clears the windows of one-step delays (one wavefront), for run_mail.
+__device__ __forceinline__ void run_clear_late(const RunLds *L, uint32_t *win_lds, int lane)
+{
+    const int n_win = uniform(L->n_win);
+    const int4 x = L->win[lane & (SC_MAX_WIN - 1)];
+    for (int w = 0; w < n_win; ++w) {
+        if (__builtin_amdgcn_readlane(x.x, w) >= 2) continue;
+        u32x4 *to = reinterpret_cast<u32x4 *>(win_lds) + (__builtin_amdgcn_readlane(x.w, w) >> 2);
+        const int n4 = __builtin_amdgcn_readlane(x.z, w) >> 2;
+        for (int i = lane; i < n4; i += SC_WAVE) to[i] = u32x4{0u, 0u, 0u, 0u};
+    }
+}
+
+// A value that the compiler takes for changed: nothing derived from it is kept from
+// step to step beside it (a step's addresses and masks cost a few instructions; held
+// over the run they spill).
+__device__ __forceinline__ int renew(int v)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    asm volatile("" : "+v"(v));
+#endif
+    return v;
+}
+// The same for the registers of a lane head.
+template <int WP, bool IDX16>
+__device__ __forceinline__ void hold(LaneHead<WP, IDX16> &H)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+#pragma unroll
+    for (int s = 0; s < SC_MAX_SLICES; ++s) {
+#pragma unroll
+        for (auto &x : H.c[s]) asm volatile("" : "+v"(x));
+#pragma unroll
+        for (auto &x : H.raw[s].w) asm volatile("" : "+v"(x));
+    }
+#endif
+}
+
+// One wavefront's lane group over the run (has: it has one; the other wavefronts of
+// the block share its barriers and window copies).  The windows of step k + 1 are
+// copied while the neurons of step k are updated, unless one of them is of the step
+// before (a one-step delay).
+template <int WP, bool IDX16, bool STAGED>
+__device__ __forceinline__ void run_lane(const ScLaneTask *tp, bool has, const ScInstance &I, const ScRun &r,
+                                         bool ahead, uint32_t *win, RunLds *L, int row0,
+                                         unsigned long long m0, int wave, const int lane0)
+{
+    int lane = lane0;
+    const bool valid = has && lane < tp->nvalid;
+    float u = 0.f;
+    float2 gg = {0.f, 0.f};
+    int32_t rf = 0;
+    const uint32_t zb = (uint32_t)(I.Wr - 1) * SC_WAVE;
+    LaneHead<WP, IDX16> H;
+    if (valid) load_state(I.st, tp->group * SC_WAVE + lane, u, gg, rf);
+    if (has) lane_head<WP, IDX16, false>(*tp, zb, lane, H);
+    const int n_dep = L->n_dep;
+    int row_n = row0;
+    for (int k = 0; k < r.K; ++k) {
+        const auto &t = afresh(tp);
+        lane = renew(lane0);
+        if (k == 0 || !ahead) {
+            if (wave == 0) run_wait(I, r, 0, n_dep, k, m0, L, lane);
+            __syncthreads();
+            if (L->stop) return;
+            if constexpr (STAGED) {
+                run_stage<RUN_ALL>(L, win, I, row_n, wave, SC_BLOCK / SC_WAVE, lane);
+                drain();
+                __syncthreads();
+            }
+        }
+        const int row_next = row_n + 1 == I.R ? 0 : row_n + 1;
+        float dge = 0.f, dgi = 0.f;
+        hold(H);
+        if (has) {
+            gptr<uint32_t> row[SC_MAX_SLICES];
+            lane_rows(t, I, row_n, row);
+            lane_dg<WP, IDX16, STAGED, false, true>(t, row, win, H, zb, lane, dge, dgi);
+        }
+        if (ahead && k + 1 < r.K) {
+            if (wave == 0) run_wait(I, r, 0, n_dep, k + 1, m0, L, lane);
+            __syncthreads();
+            if (L->stop) return;
+            if constexpr (STAGED) run_stage<RUN_ALL>(L, win, I, row_next, wave, SC_BLOCK / SC_WAVE, lane);
+        }
+        if (has) {
+            const int spk = valid ? lif_step(afresh(I.pops + t.pop), u, gg.x, gg.y, rf, dge, dgi) : 0;
+            const unsigned long long word = __ballot(spk != 0);
+            if (lane == 0) st_agent(reinterpret_cast<unsigned long long *>(I.ring) + (int64_t)row_n * I.Wr + t.group, word);
+        }
+        drain();
+        __syncthreads();
+        if (threadIdx.x == 0) run_publish(r, m0, k);
+        row_n = row_next;
+    }
+    if (run_complete(I, r, L) && valid) store_state(I.st, tp->group * SC_WAVE + lane, u, gg, rf);
+}
+
+// The team neurons of one block over the run: as do_team, with the first wavefront
+// running the neuron updates of all its teams, the gathers of the one-step
+// projections after the others, and the neuron state in LDS.  The windows of step
+// k + 1 (but for one-step delays) are copied while the neurons of step k are updated.
+template <bool IDX16, bool STAGED>
+__device__ __forceinline__ void run_team(const ScInstance &I, const ScTeamTask *__restrict__ teams, int t, int count,
+                                         const ScRun &r, uint32_t *win, RunLds *L, int row0,
+                                         unsigned long long m0)
+{
+    constexpr int NTEAM = SC_BLOCK / SC_WAVE;
+    constexpr int PW = (SC_POP_WORDS + 1) / 2 * 2;
+    __shared__ double acc[NTEAM][SC_MAX_IN];
+    __shared__ uint32_t rowoff[NTEAM][SC_MAX_IN];
+    __shared__ alignas(8) uint32_t par[NTEAM][PW];
+    __shared__ ScTeamIn pin[NTEAM][SC_MAX_IN];
+    __shared__ ScState sv[NTEAM];
+    const int wave = uniform(threadIdx.x / SC_WAVE);
+    int lane = threadIdx.x & (SC_WAVE - 1);
+    const int team = wave / t, tw = wave - team * t;
+    const bool active = team < count;
+    const bool upd = wave == 0 && lane < count;  // this lane owns the neuron of team `lane`
+    const ScTeamTask *tp = teams + min(team, count - 1);  // this wavefront's team
+    int dj = 0, n_in = 0;
+    if (upd) {
+        const ScTeamTask *T = teams + lane;
+        dj = T->group * SC_WAVE + T->bit;
+        n_in = T->n_in;
+        sv[lane] = I.st[dj];
+        // the owner of a word's first neuron clears the word in the run's other rows
+        // and in the row after the run (its row of the first step is clear already)
+        if (T->bit == 0)
+            for (int k = 1, row = row0; k <= r.K; ++k) {
+                row = row + 1 == I.R ? 0 : row + 1;
+                st_agent(reinterpret_cast<unsigned long long *>(I.ring) + (int64_t)row * I.Wr + T->group, 0ull);
+            }
+    }
+    if (active && tw == 0) {
+        if (lane < SC_MAX_IN) {
+            acc[team][lane] = 0.0;
+            pin[team][lane] = tp->in[lane];
+        }
+        if (lane < SC_POP_WORDS) par[team][lane] = gbl(reinterpret_cast<const uint32_t *>(&I.pops[tp->pop]))[lane];
+    }
+    const TeamHead h = team_head(afresh(tp));
+    const int g_e = afresh(tp).n_grp_e, len_e = afresh(tp).len_e;
+    const int n_early = L->n_early, n_dep = L->n_dep, phases = n_dep > n_early ? 2 : 1;
+    const uint32_t gmask =
+        STAGED ? (uint32_t)__ballot(lane < h.n_in && lane < SC_MAX_IN && tp->in[lane & (SC_MAX_IN - 1)].lds == SC_LDS_GLOBAL) : 0u;
+    const int TT = t * SC_WAVE;
+    gptr<uint32_t> ring32 = gbl(reinterpret_cast<const uint32_t *>(uniform_ptr(I.ring)));
+    const uint32_t zb = (uint32_t)uniform((I.Wr - 1) * SC_WAVE);
+    const bool use_mail = STAGED && L->n_mail > 0;
+    // each lane's first record of both parts of its row stays in registers
+    u32x4 rec[2];
+#pragma unroll
+    for (int ph = 0; ph < 2; ++ph) {
+        const int i = (ph ? g_e : 0) + tw * SC_WAVE + lane, end = ph ? h.n_grp : g_e;
+        rec[ph] = active && i < end ? gbl(reinterpret_cast<const u32x4 *>(h.grp))[i] : u32x4{0u, 0u, 0u, 0u};
+    }
+    int row_n = row0;
+    if (wave == 1) {
+        run_wait(I, r, 1, n_early, 0, m0, L, lane);
+        if constexpr (STAGED) {
+            run_stage<RUN_EARLY>(L, win, I, row_n, 0, 1, lane);
+            if (use_mail) run_stage<RUN_LATE>(L, win, I, row_n, 0, 1, lane);
+        }
+    }
+    for (int k = 0; k < r.K; ++k) {
+        lane = renew((int)threadIdx.x & (SC_WAVE - 1));
+        if (active && tw == 0 && lane < SC_MAX_IN) {
+            const ScTeamIn &x = pin[team][lane];
+            rowoff[team][lane] = lane >= h.n_in ? 0u
+                                 : (STAGED && x.lds != SC_LDS_GLOBAL)
+                                     ? (uint32_t)x.lds
+                                     : (uint32_t)row_back(row_n, x.delay, I.R) * (uint32_t)(2 * I.Wr);
+        }
+        if (wave == 1) drain();
+        __syncthreads();  // the windows of the longer delays are in LDS, the sums are zero
+        if (L->stop) return;
+        const unsigned long long mail0 = use_mail && wave == 0 ? mail_load(r, L, m0 + (unsigned long long)k, 0, lane) : 0ull;
+#pragma unroll 1
+        for (int ph = 0; ph < phases; ++ph) {
+            if (ph) {
+                if (wave == 0) {
+                    // (the one-step windows of the run's first step are staged from the ring)
+                    if (use_mail) {
+                        if (k > 0) run_mail(I, r, win, k, row_back(row_n, 1, I.R), m0, L, lane, mail0);
+                    } else {
+                        run_wait(I, r, n_early, n_dep, k, m0, L, lane);
+                        if constexpr (STAGED) {
+                            run_stage<RUN_LATE>(L, win, I, row_n, 0, 1, lane);
+                            drain();
+                        }
+                    }
+                }
+                __syncthreads();
+                if (L->stop) return;
+            }
+            if (active) {
+                const TeamPart part = ph ? TeamPart{g_e, h.n_grp, len_e, h.len} : TeamPart{0, g_e, 0, len_e};
+                team_dispatch<IDX16, STAGED, false, true>(h, part, ring32, win, rowoff[team], gmask, zb,
+                                                          tw * SC_WAVE + renew(lane), TT, acc[team], ph ? rec[1] : rec[0]);
+            }
+            // the spikes of the step before are in the ring by now
+            if (ph == 0 && wave == 0 && k > 0) {
+                drain();
+                if (lane == 0) run_publish(r, m0, k - 1);
+            }
+        }
+        const int row_next = row_n + 1 == I.R ? 0 : row_n + 1;
+        __syncthreads();  // the sums are complete, the windows no longer read
+        if (wave == 1 && k + 1 < r.K) {
+            // meanwhile the next step's windows
+            run_wait(I, r, 1, n_early, k + 1, m0, L, lane);
+            if constexpr (STAGED) {
+                run_stage<RUN_EARLY>(L, win, I, row_next, 0, 1, lane);
+                if (use_mail) run_clear_late(L, win, lane);
+            }
+        }
+        if (wave == 0) {
+            // other blocks clear this block's words of the run's later rows in step 0
+            if (k == 1) run_wait(I, r, 0, 1, k, m0, L, lane);
+            lane = renew(lane);
+            int spk = 0;
+            if (upd) {
+                // dg[post] += S * w_bar (Simulation_header.cu:98), projections in index order
+                float dge = 0.f, dgi = 0.f;
+#pragma unroll 1
+                for (int q = 0; q < n_in; ++q) {
+                    const ScTeamIn &x = pin[lane][q];
+                    const float add = (float)(acc[lane][q] * (double)x.scale) * x.W;
+                    acc[lane][q] = 0.0;
+                    if (x.exc) dge = dge + add;
+                    else dgi = dgi + add;
+                }
+                ScState x = sv[lane];
+                spk = lif_step(*reinterpret_cast<const ScPop *>(par[lane]), x.V, x.g_exc, x.g_inh, x.refr, dge, dgi);
+                sv[lane] = x;
+            }
+            const uint32_t bits = (uint32_t)__ballot(spk != 0);
+            const unsigned long long after = m0 + (unsigned long long)k + 1ull;
+            if (lane == 0)
+                st_agent(r.tags + (size_t)blockIdx.x * SC_TAG_WORDS + 1 + (int)(after % SC_MAIL), after << 16 | bits);
+            if (spk)
+                atomicOr(reinterpret_cast<unsigned long long *>(I.ring) + (int64_t)row_n * I.Wr + dj / SC_WAVE,
+                         1ull << (dj & (SC_WAVE - 1)));
+        }
+        row_n = row_next;
+    }
+    if (wave == 0) {
+        drain();
+        if (lane == 0) run_publish(r, m0, r.K - 1);
+    }
+    if (run_complete(I, r, L) && upd) I.st[dj] = sv[lane];
+}
+
+template <bool IDX16, bool STAGED>
+__device__ __forceinline__ void run_lane_dispatch(const ScLaneTask *t, bool has, const ScInstance &I, const ScRun &r,
+                                                  bool ahead, uint32_t *win, RunLds *L, int row0,
+                                                  unsigned long long m0, int wave, int lane)
+{
+    if (IDX16 && t->idx16) {
+        switch (t->wp) {
+        case SC_W_F32: run_lane<SC_W_F32, true, STAGED>(t, has, I, r, ahead, win, L, row0, m0, wave, lane); break;
+        case SC_W_BF16: run_lane<SC_W_BF16, true, STAGED>(t, has, I, r, ahead, win, L, row0, m0, wave, lane); break;
+        case SC_W_FP8: run_lane<SC_W_FP8, true, STAGED>(t, has, I, r, ahead, win, L, row0, m0, wave, lane); break;
+        default: run_lane<SC_W_UNIT, true, STAGED>(t, has, I, r, ahead, win, L, row0, m0, wave, lane); break;
+        }
+    } else {
+        switch (t->wp) {
+        case SC_W_F32: run_lane<SC_W_F32, false, STAGED>(t, has, I, r, ahead, win, L, row0, m0, wave, lane); break;
+        case SC_W_BF16: run_lane<SC_W_BF16, false, STAGED>(t, has, I, r, ahead, win, L, row0, m0, wave, lane); break;
+        case SC_W_FP8: run_lane<SC_W_FP8, false, STAGED>(t, has, I, r, ahead, win, L, row0, m0, wave, lane); break;
+        default: run_lane<SC_W_UNIT, false, STAGED>(t, has, I, r, ahead, win, L, row0, m0, wave, lane); break;
+        }
+    }
+}
+
+// 128 VGPRs and one block per CU (256 blocks).  With 64 VGPRs two blocks share a CU
+// and networks of up to 512 blocks fit, but the loop-carried values spill and the
+// blocks of a CU share its issue slots: at 96.7k cells (501 blocks) such a run took
+// 241 us per 25-step call against 248 with a launch per step, not worth a second
+// instantiation; at 9.9k cells 172 against 154 with 128 VGPRs.
+template <bool IDX16>
+__global__ void __launch_bounds__(SC_BLOCK) __attribute__((amdgpu_waves_per_eu(4, 4)))
+k_run(ScInstance I0, ScLayout L, const ScLaneTask *__restrict__ lanes,
+      const ScStimTask *__restrict__ stt, const ScTeamTask *__restrict__ teams, const ScStage *__restrict__ stages,
+      ScRun r)
+{
+    __shared__ __attribute__((aligned(16))) uint32_t win_lds[SC_WIN_WORDS];
+    __shared__ RunLds run_lds;
+    if (I0.ctl->failed) return;  // an earlier run was given up: the host launches this one's steps again
+    const int row0 = I0.ctl->row;
+    const unsigned long long m0 = (unsigned long long)I0.ctl->m;
+    const int b = blockIdx.x;
+    int c = 0;
+#pragma unroll
+    for (int j = 0; j < SC_CLASSES - 1; ++j) c += (b >= L.cls_end[j]) ? 1 : 0;
+    const int bi = b - (c ? L.cls_end[c - 1] : 0);
+    const int wave = uniform(threadIdx.x / SC_WAVE), lane = threadIdx.x & (SC_WAVE - 1);
+    const ScDeps *dp = r.deps + b;
+    bool one_step = false;  // (one lane per wait entry)
+    if (lane < SC_MAX_DEP) {
+        const ScDep x = dp->e[lane];
+        one_step = lane < dp->n && x.delay == 1;
+        if (wave == 0) run_lds.dep[lane] = int4{x.b0, x.cnt, x.delay, 0};
+    }
+    int n_mail = 0;
+    if (dp->mail)
+        for (int e = dp->n_early; e < dp->n; ++e) {
+            const ScDep x = dp->e[e];
+            const int i = (int)threadIdx.x - n_mail;
+            if (i >= 0 && i < x.cnt) {
+                const int bit = x.bit0 + i * x.per, w = bit >> 5;
+                run_lds.mail[threadIdx.x] =
+                    int4{x.b0 + i, w >= x.w0 && w < x.w1 ? (x.lds + w) << 5 | (bit & 31) : -1, w, x.per};
+            }
+            n_mail += x.cnt;
+        }
+    if (threadIdx.x == 0) {
+        run_lds.n_mail = n_mail;
+        run_lds.n_early = dp->n_early;
+        run_lds.n_dep = dp->n;
+        run_lds.stop = 0;
+        *reinterpret_cast<u32x4 *>(win_lds) = u32x4{0u, 0u, 0u, 0u};
+    }
+    const bool ahead = __ballot(one_step) == 0ull;
+    const int n_win = stages ? stages[b].n : 0;
+    if ((int)threadIdx.x < n_win) {
+        const ScWin x = stages[b].w[threadIdx.x];
+        run_lds.win[threadIdx.x] = int4{x.delay, x.w0, x.nw, x.off};
+    }
+    if (threadIdx.x == 0) run_lds.n_win = n_win;
+    __syncthreads();
+    if (c < SC_CLASS_LANE) {
+        const int t = SC_MAX_TEAM >> c, per = 1 << c;
+        const int first = L.cls_task0[c] + bi * per, count = min(per, L.cls_ntask[c] - bi * per);
+        if (n_win) run_team<IDX16, true>(I0, teams + first, t, count, r, win_lds, &run_lds, row0, m0);
+        else run_team<IDX16, false>(I0, teams + first, t, count, r, win_lds, &run_lds, row0, m0);
+        return;
+    }
+    if (c == SC_CLASS_LANE) {
+        const int idx = uniform(bi * L.lane_per + wave);
+        const bool has = wave < L.lane_per && idx < L.cls_ntask[c];
+        const ScLaneTask *t = lanes + (has ? idx : L.cls_ntask[c] - 1);
+        if (n_win) run_lane_dispatch<IDX16, true>(t, has, I0, r, ahead, win_lds, &run_lds, row0, m0, wave, lane);
+        else run_lane_dispatch<IDX16, false>(t, has, I0, r, ahead, win_lds, &run_lds, row0, m0, wave, lane);
+        return;
+    }
+    // stimulus groups read nothing of the run: they run ahead of everyone
+    const int idx = uniform(bi * L.stim_per + wave);
+    const bool has = wave < L.stim_per && idx < L.cls_ntask[SC_CLASS_STIM];
+    const ScStimTask t = stt[has ? idx : 0];
+    const int d = t.group * SC_WAVE + lane;
+    int s = -1, entry = 0;
+    if (has && lane < t.nvalid) {
+        s = I0.stim_s[d];
+        entry = I0.stim_e[d];
+    }
+    const int64_t n0 = I0.ctl->n;
+    int row_n = row0;
+    for (int k = 0; k < r.K; ++k) {
+        if (has) {
+            const int spk = s >= 0 ? stim_fires(I0.stims[s], entry, n0 + k, (int64_t)m0 + k) : 0;
+            const unsigned long long word = __ballot(spk != 0);
+            if (lane == 0)
+                st_agent(reinterpret_cast<unsigned long long *>(I0.ring) + (int64_t)row_n * I0.Wr + t.group, word);
+        }
+        drain();
+        __syncthreads();
+        if (threadIdx.x == 0) run_publish(r, m0, k);
+        row_n = row_n + 1 == I0.R ? 0 : row_n + 1;
+    }
+    (void)run_complete(I0, r, &run_lds);
 }
 
 // Per-population spike counts and synaptic events of K consecutive steps.  The
@@ -1289,14 +1969,21 @@ __device__ __forceinline__ void stats_block(const ScInstance &I0, const ScInstan
 // step counters (the run's ring rows); once it no longer does, it counts itself in
 // *done, and the last block to arrive advances the counters of every instance by K
 // (n, m, ring row; the window-count recount flag cleared) and resets *done for the
-// next launch.
+// next launch (run_done, the resident run's count of finished blocks, as well).
+// After a resident run that was given up nothing is counted or advanced; the run's
+// steps are added to those the host has to launch again.
 template <bool SINGLE>
 __global__ void __launch_bounds__(SC_STATS_CHUNK / 2) k_run_end(ScInstance I0, const ScInstance *__restrict__ insts,
                                                                  int n_inst, int K, int nchunk, int n_stats, ScOut O,
-                                                                 unsigned int *__restrict__ done)
+                                                                 unsigned int *__restrict__ done,
+                                                                 unsigned int *__restrict__ run_done)
 {
     __shared__ int last;
     const int b = blockIdx.x;
+    if (SINGLE && run_done && I0.ctl->failed) {
+        if (b == 0 && threadIdx.x == 0) I0.ctl->skipped += K;
+        return;
+    }
     if (b < n_stats) {
         stats_block<SINGLE>(I0, insts, K, nchunk, b);
     } else {
@@ -1323,7 +2010,10 @@ __global__ void __launch_bounds__(SC_STATS_CHUNK / 2) k_run_end(ScInstance I0, c
         c->row = (c->row + K) % I.R;
         c->recount = 0;
     }
-    if (threadIdx.x == 0) *done = 0u;
+    if (threadIdx.x == 0) {
+        *done = 0u;
+        if (run_done) *run_done = 0u;
+    }
 }
 
 __global__ void k_set_ctl(ScCtl *ctl, int64_t n, int64_t m, int row)
@@ -1333,6 +2023,8 @@ __global__ void k_set_ctl(ScCtl *ctl, int64_t n, int64_t m, int row)
         ctl->m = m;
         ctl->row = row;
         ctl->recount = 1;
+        ctl->failed = 0;
+        ctl->skipped = 0;
     }
 }
 
@@ -1529,8 +2221,25 @@ void launch_step(hipStream_t s, const ScInstance *single, const ScInstance *inst
     else launch_step_nt<false>(s, single, insts, w, k);
 }
 
+int run_capacity(bool idx16, int *blocks)
+{
+    int dev = 0, cus = 0, per_cu = 0;
+    HIP_TRY(hipGetDevice(&dev));
+    HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    HIP_TRY(idx16 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_run<true>, SC_BLOCK, 0)
+                  : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_run<false>, SC_BLOCK, 0));
+    *blocks = per_cu * cus;
+    return SCAFFOLD_OK;
+}
+
+void launch_run(hipStream_t s, const ScInstance &I, const DevWork &w, const ScRun &r)
+{
+    if (w.idx16) k_run<true><<<w.n_blocks, SC_BLOCK, 0, s>>>(I, w.layout, w.lanes, w.stims, w.teams, w.stages, r);
+    else k_run<false><<<w.n_blocks, SC_BLOCK, 0, s>>>(I, w.layout, w.lanes, w.stims, w.teams, w.stages, r);
+}
+
 void launch_run_end(hipStream_t s, const ScInstance *single, const ScInstance *insts, int n_inst, int K,
-                    int max_groups, const ScOut *out, unsigned int *done)
+                    int max_groups, const ScOut *out, unsigned int *done, unsigned int *run_done)
 {
     if (K <= 0 || n_inst <= 0) return;
     const int nchunk = std::max(1, (max_groups + SC_STATS_CHUNK - 1) / SC_STATS_CHUNK);
@@ -1544,10 +2253,11 @@ void launch_run_end(hipStream_t s, const ScInstance *single, const ScInstance *i
     }
     if (single) {
         if (nchunk > 1) k_stats_zero<true><<<K, 256, 0, s>>>(*single, insts, K);
-        k_run_end<true><<<n_stats + n_out_blocks, bs, 0, s>>>(*single, insts, 1, K, nchunk, n_stats, o, done);
+        k_run_end<true><<<n_stats + n_out_blocks, bs, 0, s>>>(*single, insts, 1, K, nchunk, n_stats, o, done, run_done);
     } else {
         if (nchunk > 1) k_stats_zero<false><<<K * n_inst, 256, 0, s>>>(ScInstance{}, insts, K);
-        k_run_end<false><<<n_stats, bs, 0, s>>>(ScInstance{}, insts, n_inst, K, nchunk, n_stats, o, done);
+        k_run_end<false><<<n_stats, bs, 0, s>>>(ScInstance{}, insts, n_inst, K, nchunk, n_stats, o, done,
+                                                                     nullptr);
     }
 }
 

@@ -22,6 +22,8 @@ struct DevWork {
     const ScTeamTask *teams = nullptr;
     bool idx16 = false;  // some descriptor holds 16-bit column offsets
     bool nontemporal = false;  // synapse streams loaded as nontemporal (networks beyond the L2)
+    std::vector<ScTeamTask> h_teams;  // host copies: the team descriptors as uploaded, the staging plan
+    std::vector<ScStage> h_stages;
     const ScStage *stages = nullptr;  // per block: spike windows staged in LDS (nullptr: none)
     int n_staged = 0;                 // blocks with staged windows
     int max_groups = 0;               // most 64-neuron groups of one instance (statistics grid)
@@ -48,7 +50,11 @@ void launch_step(hipStream_t s, const ScInstance *single, const ScInstance *inst
 // `done` is a zeroed device counter kept for this launch sequence (the kernel
 // leaves it zero again).
 void launch_run_end(hipStream_t s, const ScInstance *single, const ScInstance *insts, int n_inst, int K,
-                    int max_groups, const ScOut *out, unsigned int *done);
+                    int max_groups, const ScOut *out, unsigned int *done, unsigned int *run_done = nullptr);
+// Blocks of a resident run that the current device holds at once, and the run (one
+// network, no plasticity rules).  launch_run_end follows with run_done = r.done.
+int run_capacity(bool idx16, int *blocks);
+void launch_run(hipStream_t s, const ScInstance &I, const DevWork &w, const ScRun &r);
 void launch_set_ctl(hipStream_t s, ScCtl *ctl, int64_t n, int64_t m, int row);
 void launch_init_params(hipStream_t s, const ScInstance *di, int n_threads, uint64_t seed, uint64_t off);
 void launch_compact(hipStream_t s, const uint64_t *row, int n_groups, const ScGroup *groups, const ScPop *pops,

@@ -78,6 +78,8 @@ struct Options {
     int reset_g = 0;
     int stage_spikes = 1;
     int stage_ratio = 0;      // stage a block when window words <= stage_ratio x its gathers' 64-byte segments (0: by size)
+    int resident = 1;         // 1: runs of networks that fit the chip are one launch (0: a launch per step)
+    int run_polls = 1 << 20;  // resident runs: most polls of one wait before the run is given up
     int nontemporal = -1;     // synapse streams as nontemporal loads: -1 when they exceed the L2, 0 never, 1 always
 };
 
@@ -114,6 +116,8 @@ struct HostProjArrays {
 struct TeamPop {
     int pop = -1;
     int team_waves = 1;
+    int batch_waves = 1;  // the width in a batch (whose blocks fill the chip together)
+    double work = 0.0;  // mean row length (merged entries and word-group synapses)
     int wprec = SC_W_UNIT;
     std::vector<int64_t> row_ptr;   // num + 1
     std::vector<int32_t> seg_end;   // num x n_in: end of each projection's segment, relative to the row
@@ -137,6 +141,9 @@ struct TeamPop {
     std::vector<int64_t> grp_ptr;
     int64_t n_grp = 0;
     int64_t n_gval = 0;  // synapses in word groups (their multipliers end val)
+    // per neuron: entries (16-bit form: chunks) of the merged row and word groups
+    // that belong to projections of two or more steps of delay (they come first)
+    std::vector<int32_t> len_e, grp_e;
 };
 
 // A plasticity rule lowered to the device layout: per synapse of the target
@@ -178,6 +185,9 @@ struct Plan {
     int lane_synapses = 8;  // team width target in effect
     int group_min = 0;      // word-group threshold in effect (0: none)
     bool nontemporal = false;  // load the synapse streams nontemporal
+    int index_bits = 32;
+    bool resident = false;     // resident runs allowed
+    int run_polls = 0;
     int64_t syn16 = 0;  // synapses stored as 16-bit column offsets
     int64_t n_grp = 0, grp_syn = 0;  // word groups of the team rows and the synapses they hold
     // bytes the stored layout streams per step: every column / header / multiplier

@@ -521,11 +521,23 @@ int plan_build(scaffold_env *env, Plan &P)
             }
             dense[q] = !src.col.empty() && (int64_t)src.col.size() >= (int64_t)group_min * words;
         }
+        // rows hold the projections of two or more steps of delay first, the
+        // one-step ones after them (a resident run gathers the former before it
+        // waits for the previous step); the sums are exact, so the order is free
+        int ord[SC_MAX_IN], n_ord = 0;
+        bool late[SC_MAX_IN] = {};
+        for (int q = 0; q < d.n_in; ++q) late[q] = P.projs[d.in_proj[q]].delay < 2;
+        for (int l = 0; l < 2; ++l)
+            for (int q = 0; q < d.n_in; ++q)
+                if (late[q] == (l == 1)) ord[n_ord++] = q;
         T.row_ptr.assign(d.num + 1, 0);
         T.seg_end.assign((size_t)d.num * d.n_in, 0);
+        T.len_e.assign(d.num, 0);
+        T.grp_e.assign(d.num, 0);
         for (int j = 0; j < d.num; ++j) {
             int64_t len = 0;
-            for (int q = 0; q < d.n_in; ++q) {
+            for (int o = 0; o < n_ord; ++o) {
+                const int q = ord[o];
                 const Projection &src = env->projs[d.in_proj[q]];
                 if (dense[q]) {  // repeated columns only
                     sort_row(src, j);
@@ -534,6 +546,7 @@ int plan_build(scaffold_env *env, Plan &P)
                     len += src.row_ptr[j + 1] - src.row_ptr[j];
                 }
                 T.seg_end[(size_t)j * d.n_in + q] = (int32_t)len;
+                if (!late[q]) T.len_e[j] = (int32_t)len;
             }
             // 32-bit form: rows padded to whole 4-entry vectors (16-byte loads)
             T.row_ptr[j + 1] = T.row_ptr[j] + (want16 ? len : (len + 3) / 4 * 4);
@@ -546,8 +559,8 @@ int plan_build(scaffold_env *env, Plan &P)
         int64_t n_gval = 0;
         for (int j = 0; j < d.num; ++j) {
             int64_t pos = T.row_ptr[j];
-            for (int q = 0; q < d.n_in; ++q) {
-                const int pi = d.in_proj[q];
+            for (int o = 0; o < n_ord; ++o) {
+                const int q = ord[o], pi = d.in_proj[q];
                 const Projection &src = env->projs[pi];
                 const ScPop &pre = P.pops[src.pre];
                 if (dense[q]) {
@@ -587,6 +600,7 @@ int plan_build(scaffold_env *env, Plan &P)
                         if (plastic_proj[pi]) vpos[pi][e] = pos;
                     }
                 }
+                if (!late[q]) T.grp_e[j] = (int32_t)((int64_t)T.grp.size() / 4 - T.grp_ptr[j]);
             }
             // padding repeats the last entry (a bit the row reads anyway) with a
             // zero multiplier; the kernel masks it by the row length as well
@@ -600,8 +614,9 @@ int plan_build(scaffold_env *env, Plan &P)
         T.row_seg.assign(d.num, 0);
         T.q_seg.assign((size_t)d.num * d.n_in, 0);
         for (int j = 0; j < d.num; ++j)
-            for (int q = 0; q < d.n_in; ++q) {
-                const int64_t s0 = T.row_ptr[j] + (q ? T.seg_end[(size_t)j * d.n_in + q - 1] : 0);
+            for (int o = 0; o < n_ord; ++o) {
+                const int q = ord[o];
+                const int64_t s0 = T.row_ptr[j] + (o ? T.seg_end[(size_t)j * d.n_in + ord[o - 1]] : 0);
                 const int64_t s1 = T.row_ptr[j] + T.seg_end[(size_t)j * d.n_in + q];
                 uint32_t &qlo = T.q_lo[(size_t)j * d.n_in + q], &qhi = T.q_hi[(size_t)j * d.n_in + q];
                 for (int64_t a = s0; a < s1; a += SC_WAVE) {
@@ -654,7 +669,11 @@ int plan_build(scaffold_env *env, Plan &P)
                 // row sums are exact, so the order cannot change them)
                 perm.resize(T.row_ptr[j + 1] - T.row_ptr[j]);
                 for (size_t i = 0; i < perm.size(); ++i) perm[i] = T.row_ptr[j] + (int64_t)i;
-                std::stable_sort(perm.begin(), perm.end(), [&](int64_t x, int64_t y) { return T.col[x] < T.col[y]; });
+                const auto by_col = [&](int64_t x, int64_t y) { return T.col[x] < T.col[y]; };
+                std::stable_sort(perm.begin(), perm.begin() + T.len_e[j], by_col);
+                std::stable_sort(perm.begin() + T.len_e[j], perm.end(), by_col);
+                const size_t n_early = (size_t)T.len_e[j];
+                T.len_e[j] = 0;
                 size_t e = 0;
                 while (e < perm.size()) {
                     const int64_t c0 = (int64_t)c16.size();
@@ -670,6 +689,7 @@ int plan_build(scaffold_env *env, Plan &P)
                         if (wb) memcpy(&v16[(c0 + n) * wb], &T.val[perm[e] * wb], wb);
                         if (!newpos.empty()) newpos[perm[e]] = c0 + n;
                     }
+                    if (e <= n_early) T.len_e[j] = (int32_t)((int64_t)h.size() - rp[j]);  // whole chunks so far
                 }
                 rp[j + 1] = (int64_t)h.size();
             }
@@ -708,13 +728,41 @@ int plan_build(scaffold_env *env, Plan &P)
         // counting the synapses of the word groups (narrower teams for rows of
         // groups ran faster at low firing rates but up to 2x slower at high ones:
         // a lane's spiking bits are added one after another)
-        const double work = (double)tot + (double)n_gval;
-        const double per_lane = work / std::max(1, d.num) / SC_WAVE / std::max(1, P.lane_synapses);
-        int t = 1;
-        while (t < SC_MAX_TEAM && t < per_lane) t <<= 1;
-        T.team_waves = t;
+        T.work = ((double)tot + (double)n_gval) / std::max(1, d.num);
         P.team_of[p] = (int)P.teams.size();
         P.teams.push_back(std::move(T));
+    }
+    auto width_for = [](const TeamPop &T, double lane_synapses) {
+        const double per_lane = T.work / SC_WAVE / std::max(1.0, lane_synapses);
+        int t = 1;
+        while (t < SC_MAX_TEAM && t < per_lane) t <<= 1;
+        return t;
+    };
+    // A network whose runs can stay resident (a block per CU, 256 at most) takes wider
+    // teams where they still fit, at three quarters of the synapses per lane: 6
+    // instead of 8 measured 141 against 149 us per 25-step call at 9.9k cells, 139
+    // against 149 at 24k, 146 against 166 at 39k (rule-text density), 125 against 125
+    // at 5.8k.
+    double per_lane = P.lane_synapses;
+    if (!large && opt.resident && env->plast.empty()) {
+        int blocks = 0;
+        for (const TeamPop &T : P.teams) {
+            const int per = SC_MAX_TEAM / width_for(T, 0.75 * per_lane);
+            blocks += (P.pops[T.pop].num + per - 1) / per;
+        }
+        int lanes = 0, stims = 0;
+        for (int p = 0; p < npop; ++p) {
+            const ScPop &d = P.pops[p];
+            if (d.kind == SCAFFOLD_INPUT) stims += (d.num + SC_WAVE - 1) / SC_WAVE;
+            else if (!team_pop[p]) lanes += (d.num + SC_WAVE - 1) / SC_WAVE;
+        }
+        blocks += (lanes + SC_LANE_PER_BLOCK - 1) / SC_LANE_PER_BLOCK;
+        blocks += (stims + SC_STIM_PER_BLOCK - 1) / SC_STIM_PER_BLOCK;
+        if (blocks <= SC_RUN_BLOCKS) per_lane *= 0.75;
+    }
+    for (TeamPop &T : P.teams) {
+        T.team_waves = width_for(T, per_lane);
+        T.batch_waves = width_for(T, P.lane_synapses);
     }
     // plasticity rules lowered to the layout (rules in table order)
     P.plastic.clear();
@@ -854,6 +902,9 @@ int plan_build(scaffold_env *env, Plan &P)
         P.stream_bytes += (int64_t)(T.col.size() * 4 + T.col16.size() * 2 + T.hdr.size() * 4 + T.grp.size() * 4 +
                                     T.val.size()) - T.n_gval * wbytes_of(T.wprec);
     P.stage = opt.stage_spikes;
+    P.index_bits = opt.index_bits;
+    P.resident = opt.resident != 0;
+    P.run_polls = opt.run_polls;
     // the synapse streams of one step beyond 64 MB (twice the aggregate L2) are
     // loaded nontemporal, so they do not evict descriptors and spike rows
     P.nontemporal = opt.nontemporal < 0 ? P.algo_bytes > ((int64_t)64 << 20) : opt.nontemporal != 0;

@@ -243,7 +243,9 @@ int scaffold_set_input_stim_ids(scaffold_env *env, int neuron_index,
  *   "lane_synapses"     team mode: target synapses per lane (sets the team width);
  *                       0 (default): 8 when one step's synapse and state streams
  *                       fit in 64 MB (the step is latency-bound: wide teams),
- *                       else 64 (throughput-bound: more synapses per block)
+ *                       else 64 (throughput-bound: more synapses per block).
+ *                       Three quarters of the value where the network's runs then
+ *                       still stay resident (see "resident")
  *   "graph"             0 (default): launch every step kernel directly; 1: replay
  *                       captured hipGraphs of whole runs (on ROCm 7 the direct
  *                       launches measured as fast or faster at every size: the
