@@ -79,7 +79,7 @@ struct ScGroup {
     int32_t pop;
     int32_t first_local;   // population-local id of lane 0
     int32_t nvalid;        // valid lanes
-    int32_t self_final;
+    int32_t ref_first;     // reference global id of lane 0
 };
 
 struct ScStim {
@@ -321,6 +321,14 @@ struct ScPlastic {
     float coef[4];             // A0, A1_I, A1_J, A2_JI
     int32_t affine;            // bit c: coefficient c is (float)(ac[c] + aa[c] * (ab[c] - (double)w))
     double ac[4], aa[4], ab[4];
+};
+
+// Tells the host that what it waits for is in the engine's mapped host memory: the
+// work's last block stores `seq` to *ready once the data is there (nullptr: nobody
+// waits).  Sequence numbers of an engine ascend in stream order.
+struct ScSignal {
+    unsigned long long *ready;
+    unsigned long long seq;
 };
 
 // Fired-list queries without allocation: ids at most, and the word offset of the

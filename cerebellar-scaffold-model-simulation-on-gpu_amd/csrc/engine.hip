@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
@@ -90,6 +91,20 @@ struct RunSync {
     int polls = 0;                       // most polls of one wait
 };
 
+// Mapped host memory that kernels of one engine hand results over in (its calls are
+// one after another, so it holds one result at a time).  `ready` is the sequence
+// number of the last result that is complete (ScSignal).  The data's size follows the
+// network's (16 bytes a neuron, within bounds): pinning costs 1.5 ms a megabyte when
+// the network is set up; larger results are handed over in parts.
+constexpr size_t kHandLeast = 64 << 10, kHandMost = 1 << 20;
+struct HandOff {
+    uint32_t run_failed;  // a resident run was given up
+    int32_t count;
+    unsigned long long ready;
+    unsigned long long pad_[6];
+};
+static_assert(sizeof(HandOff) == 64, "the data starts on a line of its own");
+
 struct Engine {
     hipStream_t stream = nullptr;
     RunSync run;
@@ -108,21 +123,23 @@ struct Engine {
     ScStim *stims = nullptr;
     int n_stims = 0;
     int n_pops = 0;
-    int32_t *cnt_buf = nullptr;  // compaction count
     int32_t *scratch = nullptr;  // the static scratch on this engine's device (no-allocation queries)
     std::vector<int32_t> dev_to_ref;
     int Ndev = 0, total_ref = 0;
     RunGraphs graphs;
     KTimer kt;
-    // output spike train: device bits of the OUTPUT neurons, the T_out x n_out
-    // byte buffer on the device and its pinned host copy
+    // output spike train: device bits of the OUTPUT neurons, T_out x n_out bytes in
+    // mapped pinned memory
     const int32_t *out_bits = nullptr;
-    uint8_t *out_d = nullptr;
     uint8_t *out_h = nullptr;
-    uint8_t *out_hd = nullptr;  // the device's address of out_h (mapped pinned memory), nullptr: copy instead
-    hipEvent_t train_ev = nullptr;  // recorded once a call's output train is in out_h (with out_hd)
+    uint8_t *out_hd = nullptr;      // the device's address of out_h
+    hipEvent_t train_ev = nullptr;  // recorded once a call's output train is in out_h
     int n_out = 0, T_out = 0;
-    size_t out_bytes = 0;  // the train's bytes in out_h, in whole 64-byte lines (64 more bytes follow)
+    size_t out_bytes = 0;  // the train's bytes in out_h, in whole 64-byte lines
+    HandOff *hand = nullptr, *hand_d = nullptr;  // behind them, and the device's address of it
+    uint8_t *data = nullptr, *data_d = nullptr;  // behind that: hand_bytes of data
+    size_t hand_bytes = 0;
+    unsigned long long seq = 0;                  // of the last signal asked for
     // plastic projections: multiplier array and per-synapse index, for read-back
     struct PlasticView {
         int proj;
@@ -533,10 +550,8 @@ static int engine_plan_run(Engine *e, const Plan &P)
     int rc, most = 0;
     if ((rc = run_capacity(e->w.idx16, &most))) return rc;
     if (e->w.n_blocks > most) return SCAFFOLD_OK;
-    // the status word follows the output train in its pinned buffer
-    if (!e->out_hd) return SCAFFOLD_OK;  // no device address for host memory: a kernel per step
-    e->run.failed_h = reinterpret_cast<uint32_t *>(e->out_h + e->out_bytes);
-    e->run.failed_hd = reinterpret_cast<uint32_t *>(e->out_hd + e->out_bytes);
+    e->run.failed_h = &e->hand->run_failed;
+    e->run.failed_hd = &e->hand_d->run_failed;
     // (the count of finished blocks has a line of its own after the blocks' lines)
     if ((rc = dalloc(e->allocs, &e->bytes, &e->run.tags, (size_t)(e->w.n_blocks + 1) * SC_TAG_WORDS))) return rc;  // zeroed
     e->run.done = reinterpret_cast<uint32_t *>(e->run.tags + (size_t)e->w.n_blocks * SC_TAG_WORDS);
@@ -816,28 +831,31 @@ int engine_create(Engine **out, Plan &P)
     }
     e->w.max_groups = P.n_groups;
     e->w.nontemporal = P.nontemporal;
-    if ((rc = dalloc(A, B, &e->cnt_buf, 1))) return bail(rc);
     if ((rc = scratch_on_current_device(&e->scratch))) return bail(rc);
-    // output spike train (T_out steps x n_out neurons), copied to pinned host memory
+    // output spike train (T_out steps x n_out neurons)
     e->n_out = P.n_output;
     e->T_out = std::max(1, P.T_out);
     {
         int32_t *ob;
         if ((rc = dupload(A, B, &ob, P.out_bits))) return bail(rc);
         e->out_bits = ob;
-        const size_t nb = (size_t)e->T_out * (size_t)std::max(1, e->n_out);
-        e->out_bytes = (nb + 63) / 64 * 64;
-        if ((rc = dalloc(A, B, &e->out_d, nb))) return bail(rc);
-        if (hipHostMalloc(reinterpret_cast<void **>(&e->out_h), e->out_bytes + 64, hipHostMallocMapped) != hipSuccess)
-            return bail(fail(SCAFFOLD_ERR_HIP, "hipHostMalloc of the output train failed"));
-        memset(e->out_h, 0, e->out_bytes + 64);
-        // the gather writes the train straight into the mapped pinned buffer (no
-        // separate device-to-host copy); where the runtime gives no device address
-        // for it, the train is gathered on the device and copied
+        // the gather writes the train straight into mapped pinned memory (no separate
+        // device-to-host copy); the hand-off buffer of the queries lies behind it
+        e->out_bytes = ((size_t)e->T_out * (size_t)std::max(1, e->n_out) + 63) / 64 * 64;
         void *dp = nullptr;
-        if (hipHostGetDevicePointer(&dp, e->out_h, 0) == hipSuccess && dp) e->out_hd = static_cast<uint8_t *>(dp);
-        else (void)hipGetLastError();
-        if (e->out_hd && hipEventCreateWithFlags(&e->train_ev, hipEventDisableTiming) != hipSuccess)
+        e->hand_bytes = std::min(kHandMost, std::max(kHandLeast, (size_t)P.Ndev * 16));
+        if (hipHostMalloc(reinterpret_cast<void **>(&e->out_h), e->out_bytes + sizeof(HandOff) + e->hand_bytes,
+                          hipHostMallocMapped) != hipSuccess)
+            return bail(fail(SCAFFOLD_ERR_HIP, "hipHostMalloc of the hand-off memory failed"));
+        if (hipHostGetDevicePointer(&dp, e->out_h, 0) != hipSuccess || !dp)
+            return bail(fail(SCAFFOLD_ERR_HIP, "no device address for the hand-off memory"));
+        e->out_hd = static_cast<uint8_t *>(dp);
+        memset(e->out_h, 0, e->out_bytes + sizeof(HandOff));
+        e->hand = reinterpret_cast<HandOff *>(e->out_h + e->out_bytes);
+        e->hand_d = reinterpret_cast<HandOff *>(e->out_hd + e->out_bytes);
+        e->data = reinterpret_cast<uint8_t *>(e->hand + 1);
+        e->data_d = reinterpret_cast<uint8_t *>(e->hand_d + 1);
+        if (hipEventCreateWithFlags(&e->train_ev, hipEventDisableTiming) != hipSuccess)
             return bail(fail(SCAFFOLD_ERR_HIP, "hipEventCreate failed"));
     }
     if ((rc = engine_plan_run(e, P))) return bail(rc);
@@ -1161,7 +1179,7 @@ int engine_run_output(Engine *e, int n_steps, int use_graph, int graph_steps, in
     // holds all of it; otherwise by a launch of its own after the runs
     ScOut out;
     out.bits = e->out_bits;
-    out.out = e->out_hd ? e->out_hd : e->out_d;
+    out.out = e->out_hd;
     out.T = e->T_out;
     out.n_out = e->n_out;
     const bool closes = train && out.T * out.n_out > 0 && first_out_step + out.T == step0 + n_steps;
@@ -1169,7 +1187,7 @@ int engine_run_output(Engine *e, int n_steps, int use_graph, int graph_steps, in
     const int row0 = (int)(((first_out_step % R) + R) % R);
     // the call returns once the train is in host memory (mapped pinned memory:
     // written by the gather itself), not after the last run's statistics
-    hipEvent_t early = e->out_hd ? e->train_ev : nullptr;
+    hipEvent_t early = e->train_ev;
     bool taken = false, early_set = false;
     if (!rec) {
         rc = run_steps(e->stream, e->graphs, &e->hi, e->di, 1, e->w, n_steps, use_graph, chunk, &e->kt,
@@ -1187,12 +1205,10 @@ int engine_run_output(Engine *e, int n_steps, int use_graph, int graph_steps, in
         done += K;
     }
     if (train) {
-        const size_t nb = (size_t)e->T_out * (size_t)e->n_out;
         if (!taken) {
             launch_out_train(e->stream, e->hi.ring, e->hi.Wr, R, row0, e->T_out, e->out_bits, e->n_out, out.out);
             HIP_TRY(hipGetLastError());
         }
-        if (!e->out_hd && nb) HIP_TRY(hipMemcpyAsync(e->out_h, e->out_d, nb, hipMemcpyDeviceToHost, e->stream));
         *train = e->out_h;  // complete once engine_finish has synchronized the stream
     }
     bool recovered = false;
@@ -1200,9 +1216,6 @@ int engine_run_output(Engine *e, int n_steps, int use_graph, int graph_steps, in
     if (train && recovered) {  // the train of the steps launched again
         launch_out_train(e->stream, e->hi.ring, e->hi.Wr, R, row0, e->T_out, e->out_bits, e->n_out, out.out);
         HIP_TRY(hipGetLastError());
-        if (!e->out_hd && (size_t)e->T_out * (size_t)e->n_out)
-            HIP_TRY(hipMemcpyAsync(e->out_h, e->out_d, (size_t)e->T_out * (size_t)e->n_out, hipMemcpyDeviceToHost,
-                                   e->stream));
         HIP_TRY(hipStreamSynchronize(e->stream));
     }
     return SCAFFOLD_OK;
@@ -1335,32 +1348,53 @@ int engine_get_totals(Engine *e, unsigned long long *totals)
     return SCAFFOLD_OK;
 }
 
-int engine_get_fired(Engine *e, int row, int32_t *ids, int32_t cap, int32_t *n)
+// The next signal of the engine's stream.
+static ScSignal hand_signal(Engine *e) { return ScSignal{&e->hand_d->ready, ++e->seq}; }
+
+// Waits until signal `seq` is in.  The host reads the word for about as long as short
+// work takes (a read of the word is seen 3-8 us sooner than the runtime's wait returns), then
+// leaves the wait to the runtime, which also reports what went wrong on the stream.
+static int hand_wait(Engine *e, unsigned long long seq)
 {
-    int32_t *dout = nullptr;
-    const int c = std::max(cap, 1);
-    HIP_TRY(hipMalloc(&dout, sizeof(int32_t) * c));
-    launch_compact(e->stream, e->hi.ring + (size_t)row * e->hi.Wr, e->hi.n_groups, e->hi.groups, e->hi.pops, dout,
-                   cap, e->cnt_buf);
-    hipError_t err = hipGetLastError();
-    if (err == hipSuccess) err = hipStreamSynchronize(e->stream);
-    if (err == hipSuccess) err = hipMemcpy(n, e->cnt_buf, sizeof(int32_t), hipMemcpyDeviceToHost);
-    if (err == hipSuccess && cap > 0)
-        err = hipMemcpy(ids, dout, sizeof(int32_t) * std::min(cap, *n), hipMemcpyDeviceToHost);
-    (void)hipFree(dout);
-    if (err != hipSuccess) return fail(SCAFFOLD_ERR_HIP, "fired-list compaction: %s", hipGetErrorString(err));
+    const auto arrived = [&] { return __atomic_load_n(&e->hand->ready, __ATOMIC_ACQUIRE) >= seq; };
+    const auto t0 = std::chrono::steady_clock::now();
+    while (!arrived()) {
+        for (int i = 0; i < 64 && !arrived(); ++i) __builtin_ia32_pause();
+        if (std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) break;
+    }
+    if (!arrived()) HIP_TRY(hipStreamSynchronize(e->stream));
     return SCAFFOLD_OK;
 }
 
-// engine_get_fired without allocating: the compaction writes its count and ids
-// into the static scratch of the engine's device, then both are copied out.
+int engine_get_fired(Engine *e, int row, int32_t *ids, int32_t cap, int32_t *n)
+{
+    const int32_t most = (int32_t)(e->hand_bytes / sizeof(int32_t));  // ids handed over at a time
+    int32_t first = 0;
+    do {
+        const int32_t len = std::min(most, std::max(cap, 0) - first);
+        const ScSignal sig = hand_signal(e);
+        launch_fired(e->stream, e->hi.ring + (size_t)row * e->hi.Wr, e->hi.n_groups, e->hi.groups,
+                     reinterpret_cast<int32_t *>(e->data_d), first, len, &e->hand_d->count, sig);
+        HIP_TRY(hipGetLastError());
+        int rc = hand_wait(e, sig.seq);
+        if (rc) return rc;
+        *n = e->hand->count;
+        const int32_t k = std::min(len, *n - first);
+        if (k > 0) memcpy(ids + first, e->data, sizeof(int32_t) * (size_t)k);
+        first += len;
+    } while (first < std::min(cap, *n));
+    return SCAFFOLD_OK;
+}
+
+// engine_get_fired through the static scratch of the engine's device: the compaction
+// writes its count and ids there, then both are copied out.
 int engine_get_fired_noalloc(Engine *e, int row, int32_t *ids, int32_t cap, int32_t *n)
 {
     if (cap < 0 || cap > SC_FIRED_NOALLOC_MAX)
         return fail(SCAFFOLD_ERR_CAPACITY, "cap %d: the static scratch holds at most %d ids", cap, SC_FIRED_NOALLOC_MAX);
     int32_t *count = e->scratch, *out = e->scratch + SC_SCRATCH_IDS;
-    launch_compact(e->stream, e->hi.ring + (size_t)row * e->hi.Wr, e->hi.n_groups, e->hi.groups, e->hi.pops, out, cap,
-                   count);
+    launch_fired(e->stream, e->hi.ring + (size_t)row * e->hi.Wr, e->hi.n_groups, e->hi.groups, out, 0, cap, count,
+                 ScSignal{});
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(e->stream));
     HIP_TRY(hipMemcpy(n, count, sizeof(int32_t), hipMemcpyDeviceToHost));

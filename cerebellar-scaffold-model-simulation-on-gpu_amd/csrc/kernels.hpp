@@ -57,8 +57,9 @@ int run_capacity(bool idx16, int *blocks);
 void launch_run(hipStream_t s, const ScInstance &I, const DevWork &w, const ScRun &r);
 void launch_set_ctl(hipStream_t s, ScCtl *ctl, int64_t n, int64_t m, int row);
 void launch_init_params(hipStream_t s, const ScInstance *di, int n_threads, uint64_t seed, uint64_t off);
-void launch_compact(hipStream_t s, const uint64_t *row, int n_groups, const ScGroup *groups, const ScPop *pops,
-                    int32_t *out, int cap, int32_t *count);
+// Ids [first, first + len) of the fired-neuron list of one ring row and its length.
+void launch_fired(hipStream_t s, const uint64_t *row, int n_groups, const ScGroup *groups, int32_t *out, int first,
+                  int len, int32_t *count, const ScSignal &sig);
 void launch_copy(hipStream_t s, const void *src, void *dst, int64_t n16, int grid);
 // Output spike train: T steps from ring row row0 (wrapping at R), one byte per
 // (step, output neuron), output neurons at device bits bits[0..n_out).

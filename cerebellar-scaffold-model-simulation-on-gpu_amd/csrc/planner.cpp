@@ -226,7 +226,7 @@ int plan_build(scaffold_env *env, Plan &P)
             g.pop = p;
             g.first_local = gi * SC_WAVE;
             g.nvalid = std::min(SC_WAVE, d.num - gi * SC_WAVE);
-            g.self_final = 1;
+            g.ref_first = d.ref_base + g.first_local;
             P.groups.push_back(g);
         }
     }
@@ -908,7 +908,6 @@ int plan_build(scaffold_env *env, Plan &P)
     // the synapse streams of one step beyond 64 MB (twice the aggregate L2) are
     // loaded nontemporal, so they do not evict descriptors and spike rows
     P.nontemporal = opt.nontemporal < 0 ? P.algo_bytes > ((int64_t)64 << 20) : opt.nontemporal != 0;
-    for (auto &g : P.groups) g.self_final = 1;
 
     // work list: team neurons (widest teams first), lane groups, stimulus groups
     P.tasks.clear();
