@@ -100,6 +100,12 @@ struct ScStim {
     int32_t p_any, b_any;
 };
 
+// Stimulus descriptors that one launch of the upload kernel carries (kernel argument).
+#define SC_STIMS_PER_LAUNCH 8
+struct ScStimBlock {
+    ScStim s[SC_STIMS_PER_LAUNCH];
+};
+
 struct ScCtl {
     int64_t n;      // trial-relative step of launch offset k = 0
     int64_t m;      // stimulus draws since init (3 Philox blocks per draw)
@@ -350,5 +356,8 @@ struct ScInstance {
     const int32_t *stim_e;     // entry index
     const uint32_t *outdeg;    // per device index
     ScCtl   *ctl;
+    // copies of counts, events and totals in mapped host memory, as of the last run
+    int32_t *h_counts;
+    unsigned long long *h_events, *h_totals;
     int32_t R, Wr, n_groups, n_pops, n_stims, Ndev, pad0, pad1;
 };

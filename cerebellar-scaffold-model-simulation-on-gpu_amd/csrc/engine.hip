@@ -97,6 +97,7 @@ struct RunSync {
 // network's (16 bytes a neuron, within bounds): pinning costs 1.5 ms a megabyte when
 // the network is set up; larger results are handed over in parts.
 constexpr size_t kHandLeast = 64 << 10, kHandMost = 1 << 20;
+constexpr unsigned long long kNoSignal = ~0ull;
 struct HandOff {
     uint32_t run_failed;  // a resident run was given up
     int32_t count;
@@ -133,13 +134,17 @@ struct Engine {
     const int32_t *out_bits = nullptr;
     uint8_t *out_h = nullptr;
     uint8_t *out_hd = nullptr;      // the device's address of out_h
-    hipEvent_t train_ev = nullptr;  // recorded once a call's output train is in out_h
     int n_out = 0, T_out = 0;
     size_t out_bytes = 0;  // the train's bytes in out_h, in whole 64-byte lines
     HandOff *hand = nullptr, *hand_d = nullptr;  // behind them, and the device's address of it
     uint8_t *data = nullptr, *data_d = nullptr;  // behind that: hand_bytes of data
     size_t hand_bytes = 0;
-    unsigned long long seq = 0;                  // of the last signal asked for
+    unsigned long long seq = 0;  // of the last signal asked for
+    // the statistics of the last run are in host memory once this signal is in
+    // (kNoSignal: once the stream is idle)
+    unsigned long long stats_seq = 0;
+    const int32_t *counts_h = nullptr;  // R x n_pops, R, n_pops + 1: the host copies
+    const unsigned long long *events_h = nullptr, *totals_h = nullptr;
     // plastic projections: multiplier array and per-synapse index, for read-back
     struct PlasticView {
         int proj;
@@ -530,7 +535,7 @@ static int upload_work(std::vector<void *> &allocs, int64_t *bytes, DevWork &w, 
     w.lanes = l;
     w.stims = s;
     w.teams = t;
-    if ((rc = dalloc(allocs, bytes, &w.end_done, 1))) return rc;  // zeroed
+    if ((rc = dalloc(allocs, bytes, &w.end_done, 2))) return rc;  // zeroed
     w.idx16 = false;
     for (const ScLaneTask &x : lanes) w.idx16 = w.idx16 || x.idx16;
     for (const ScTeamTask &x : teams) w.idx16 = w.idx16 || x.hdr;
@@ -843,8 +848,10 @@ int engine_create(Engine **out, Plan &P)
         // device-to-host copy); the hand-off buffer of the queries lies behind it
         e->out_bytes = ((size_t)e->T_out * (size_t)std::max(1, e->n_out) + 63) / 64 * 64;
         void *dp = nullptr;
-        e->hand_bytes = std::min(kHandMost, std::max(kHandLeast, (size_t)P.Ndev * 16));
-        if (hipHostMalloc(reinterpret_cast<void **>(&e->out_h), e->out_bytes + sizeof(HandOff) + e->hand_bytes,
+        e->hand_bytes = std::min(kHandMost, std::max(kHandLeast, (size_t)P.Ndev * 16));  // whole lines
+        const size_t stat_bytes = ((size_t)P.R + I.n_pops + 1) * 8 + (size_t)P.R * I.n_pops * 4;
+        if (hipHostMalloc(reinterpret_cast<void **>(&e->out_h),
+                          e->out_bytes + sizeof(HandOff) + e->hand_bytes + stat_bytes,
                           hipHostMallocMapped) != hipSuccess)
             return bail(fail(SCAFFOLD_ERR_HIP, "hipHostMalloc of the hand-off memory failed"));
         if (hipHostGetDevicePointer(&dp, e->out_h, 0) != hipSuccess || !dp)
@@ -855,8 +862,17 @@ int engine_create(Engine **out, Plan &P)
         e->hand_d = reinterpret_cast<HandOff *>(e->out_hd + e->out_bytes);
         e->data = reinterpret_cast<uint8_t *>(e->hand + 1);
         e->data_d = reinterpret_cast<uint8_t *>(e->hand_d + 1);
-        if (hipEventCreateWithFlags(&e->train_ev, hipEventDisableTiming) != hipSuccess)
-            return bail(fail(SCAFFOLD_ERR_HIP, "hipEventCreate failed"));
+        // the statistics' copies close it
+        const size_t n64 = (size_t)P.R + I.n_pops + 1;
+        auto *st = reinterpret_cast<unsigned long long *>(e->data + e->hand_bytes);
+        memset(st, 0, stat_bytes);
+        e->events_h = st;
+        e->totals_h = st + P.R;
+        e->counts_h = reinterpret_cast<const int32_t *>(st + n64);
+        st = reinterpret_cast<unsigned long long *>(e->data_d + e->hand_bytes);
+        I.h_events = st;
+        I.h_totals = st + P.R;
+        I.h_counts = reinterpret_cast<int32_t *>(st + n64);
     }
     if ((rc = engine_plan_run(e, P))) return bail(rc);
     std::vector<ScInstance> one{I};
@@ -905,7 +921,6 @@ void engine_destroy(Engine *e)
     for (void *p : e->allocs) (void)hipFree(p);
     if (e->out_h) (void)hipHostFree(e->out_h);
     run_order_forget(e->stream);
-    if (e->train_ev) (void)hipEventDestroy(e->train_ev);
     for (hipEvent_t x : e->kt.pool) (void)hipEventDestroy(x);
     if (e->stream) (void)hipStreamDestroy(e->stream);
     delete e;
@@ -967,8 +982,8 @@ int engine_upload_stims(Engine *e, const std::vector<ScStim> &stims)
 {
     if ((int)stims.size() != e->n_stims) return fail(SCAFFOLD_ERR_STATE, "stimulus table size changed");
     if (stims.empty()) return SCAFFOLD_OK;
-    HIP_TRY(hipStreamSynchronize(e->stream));
-    HIP_TRY(hipMemcpy(e->stims, stims.data(), sizeof(ScStim) * stims.size(), hipMemcpyHostToDevice));
+    launch_set_stims(e->stream, e->stims, stims.data(), (int)stims.size());
+    HIP_TRY(hipGetLastError());
     return SCAFFOLD_OK;
 }
 
@@ -987,9 +1002,9 @@ static void launch_step_kernels(hipStream_t s, const ScInstance *single, const S
 }
 
 static void launch_end(hipStream_t s, const ScInstance *single, const ScInstance *insts, int n_inst, const DevWork &w,
-                       int K, const ScOut *out, const RunSync *res = nullptr)
+                       int K, const ScOut *out, const ScSignal &stats = ScSignal{}, const RunSync *res = nullptr)
 {
-    launch_run_end(s, single, insts, n_inst, K, w.max_groups, out, w.end_done, res ? res->done : nullptr);
+    launch_run_end(s, single, insts, n_inst, K, w.max_groups, out, stats, w.end_done, res ? res->done : nullptr);
 }
 
 static bool same_out(const ScOut &a, const ScOut &b)
@@ -1047,26 +1062,49 @@ static int timer_pair(KTimer *kt, int K, hipEvent_t *a, hipEvent_t *b)
     return SCAFFOLD_OK;
 }
 
+// The next signal of the engine's stream.
+static ScSignal hand_signal(Engine *e) { return ScSignal{&e->hand_d->ready, ++e->seq}; }
+
+// Waits until signal `seq` is in.  The host reads the word for about as long as short
+// work takes (a read of the word is seen 3-8 us sooner than the runtime's wait returns), then
+// leaves the wait to the runtime, which also reports what went wrong on the stream.
+static int hand_wait(Engine *e, unsigned long long seq)
+{
+    if (seq == kNoSignal) {
+        HIP_TRY(hipStreamSynchronize(e->stream));
+        return SCAFFOLD_OK;
+    }
+    const auto arrived = [&] { return __atomic_load_n(&e->hand->ready, __ATOMIC_ACQUIRE) >= seq; };
+    const auto t0 = std::chrono::steady_clock::now();
+    while (!arrived()) {
+        for (int i = 0; i < 64 && !arrived(); ++i) __builtin_ia32_pause();
+        if (std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) break;
+    }
+    if (!arrived()) HIP_TRY(hipStreamSynchronize(e->stream));
+    return SCAFFOLD_OK;
+}
+
 // n_steps steps in runs: graph replays of `chunk` steps, then direct launches for
 // the rest (every run direct without graphs).  With the timer on, each run's step
 // kernels lie between two events and its end is launched after them.  `out`: the
 // output train of the last out->T steps, gathered by the last run's end when that
 // run holds them all (*out_taken then set; otherwise the caller gathers it).
-// With `train_ev` (one instance), a last run launched directly gathers the train
-// by a launch of its own (its first ring row out_row0), records train_ev after it
-// and only then launches its end, so a caller that waits for the train alone
-// does not wait for the run's statistics (*train_ev_set then set).
+// `e` (one instance, resident runs where it has them): the end of its last run, if
+// launched directly, signals the train (*train_seq; 0: no signal) and then the run's
+// statistics (e->stats_seq), so a caller that waits for the train alone does not wait
+// for the statistics.
 static int run_steps(hipStream_t s, RunGraphs &G, const ScInstance *single, const ScInstance *insts, int n_inst,
                      const DevWork &w, int n_steps, int use_graph, int chunk, KTimer *kt = nullptr,
-                     const ScOut *out = nullptr, bool *out_taken = nullptr, hipEvent_t train_ev = nullptr,
-                     int out_row0 = 0, bool *train_ev_set = nullptr, const RunSync *res = nullptr)
+                     Engine *e = nullptr, const ScOut *out = nullptr, bool *out_taken = nullptr,
+                     unsigned long long *train_seq = nullptr, bool resident = true)
 {
     if (out_taken) *out_taken = false;
-    if (train_ev_set) *train_ev_set = false;
+    if (train_seq) *train_seq = 0;
     if (n_steps <= 0) return SCAFFOLD_OK;
     const bool timer = kt && kt->on;
-    if (res && res->deps && !use_graph && n_steps >= SC_RUN_MIN) chunk = std::min(chunk, res->max_steps);
-    else res = nullptr;
+    const RunSync *res =
+        e && resident && e->run.deps && !use_graph && n_steps >= SC_RUN_MIN ? &e->run : nullptr;
+    if (res) chunk = std::min(chunk, res->max_steps);
     const int last_k = n_steps % chunk ? n_steps % chunk : chunk;  // steps of the last run
     const ScOut *last_out = out && out->out && out->T > 0 && out->T <= last_k ? out : nullptr;
     int done = 0;
@@ -1098,13 +1136,20 @@ static int run_steps(hipStream_t s, RunGraphs &G, const ScInstance *single, cons
             launch_step_kernels(s, single, insts, w, K);
         }
         if (timed) HIP_TRY(hipEventRecord(b, s));
-        if (!graph && o && train_ev && single) {
-            launch_out_train(s, single->ring, single->Wr, single->R, out_row0, o->T, o->bits, o->n_out, o->out);
-            HIP_TRY(hipEventRecord(train_ev, s));
-            if (train_ev_set) *train_ev_set = true;
-            launch_end(s, single, insts, n_inst, w, K, nullptr, res);
-        } else if (timed || !graph) {
-            launch_end(s, single, insts, n_inst, w, K, o, res);
+        if (timed || !graph) {
+            ScOut train = o ? *o : ScOut{};
+            ScSignal stats{};
+            if (e && last) {
+                if (o && train_seq) {
+                    train.sig = hand_signal(e);
+                    *train_seq = train.sig.seq;
+                }
+                stats = hand_signal(e);
+                e->stats_seq = stats.seq;
+            }
+            launch_end(s, single, insts, n_inst, w, K, o ? &train : nullptr, stats, res);
+        } else if (e && last) {
+            e->stats_seq = kNoSignal;
         }
         HIP_TRY(hipGetLastError());
         done += K;
@@ -1138,23 +1183,24 @@ static int engine_recover(Engine *e, int graph_steps)
     return SCAFFOLD_OK;
 }
 
-// Waits for the engine's stream (or only for `upto`, an event recorded on it after
-// every timer event), then adds what the step-kernel timer measured.  *recovered:
-// a resident run was given up and its steps were launched again.
-static int engine_finish(Engine *e, int graph_steps, hipEvent_t upto = nullptr, bool *recovered = nullptr)
+// Waits for signal `upto` (kNoSignal: for the engine's stream), then adds what the
+// step-kernel timer measured.  *recovered: a resident run was given up and its steps
+// were launched again.
+static int engine_finish(Engine *e, int graph_steps, unsigned long long upto, bool *recovered = nullptr)
 {
-    if (upto) HIP_TRY(hipEventSynchronize(upto));
-    else HIP_TRY(hipStreamSynchronize(e->stream));
+    int rc = hand_wait(e, upto);
+    if (rc) return rc;
     KTimer &kt = e->kt;
     float x = 0.f;
     for (size_t i = 0; i < kt.piece_k.size(); ++i) {
+        HIP_TRY(hipEventSynchronize(kt.pool[2 * i + 1]));
         HIP_TRY(hipEventElapsedTime(&x, kt.pool[2 * i], kt.pool[2 * i + 1]));
         kt.ms += x;
         kt.launches += kt.piece_k[i];
     }
     kt.piece_k.clear();
     kt.used = 0;
-    if (e->run.failed_h && *const_cast<volatile uint32_t *>(e->run.failed_h)) {
+    if (__atomic_load_n(&e->hand->run_failed, __ATOMIC_ACQUIRE)) {
         if (recovered) *recovered = true;
         return engine_recover(e, graph_steps);
     }
@@ -1164,9 +1210,9 @@ static int engine_finish(Engine *e, int graph_steps, hipEvent_t upto = nullptr, 
 int engine_run(Engine *e, int n_steps, int use_graph, int graph_steps)
 {
     int rc = run_steps(e->stream, e->graphs, &e->hi, e->di, 1, e->w, n_steps, use_graph,
-                       chunk_for(graph_steps, e->hi.R), &e->kt, nullptr, nullptr, nullptr, 0, nullptr, &e->run);
+                       chunk_for(graph_steps, e->hi.R), &e->kt, e);
     if (rc) return rc;
-    return engine_finish(e, graph_steps);
+    return engine_finish(e, graph_steps, e->stats_seq);
 }
 
 int engine_run_output(Engine *e, int n_steps, int use_graph, int graph_steps, int64_t first_out_step,
@@ -1185,13 +1231,13 @@ int engine_run_output(Engine *e, int n_steps, int use_graph, int graph_steps, in
     const bool closes = train && out.T * out.n_out > 0 && first_out_step + out.T == step0 + n_steps;
     const int R = e->hi.R;
     const int row0 = (int)(((first_out_step % R) + R) % R);
-    // the call returns once the train is in host memory (mapped pinned memory:
-    // written by the gather itself), not after the last run's statistics
-    hipEvent_t early = e->train_ev;
-    bool taken = false, early_set = false;
+    // the call returns once the train is in host memory (written there by the gather
+    // itself), not after the last run's statistics
+    bool taken = false;
+    unsigned long long early = 0;
     if (!rec) {
         rc = run_steps(e->stream, e->graphs, &e->hi, e->di, 1, e->w, n_steps, use_graph, chunk, &e->kt,
-                       closes ? &out : nullptr, &taken, early, row0, &early_set, &e->run);
+                       e, closes ? &out : nullptr, &taken, &early);
         if (rc) return rc;
     }
     for (int done = 0; rec && done < n_steps;) {
@@ -1199,7 +1245,7 @@ int engine_run_output(Engine *e, int n_steps, int use_graph, int graph_steps, in
         const int K = (int)std::min<int64_t>(n_steps - done, (s / rec_T + 1) * rec_T - s);
         if ((rc = recorder_before(rec, e->stream, s + K))) return rc;
         rc = run_steps(e->stream, e->graphs, &e->hi, e->di, 1, e->w, K, use_graph, chunk, &e->kt,
-                       closes && done + K == n_steps ? &out : nullptr, &taken, early, row0, &early_set);
+                       e, closes && done + K == n_steps ? &out : nullptr, &taken, &early, false);
         if (rc) return rc;
         if ((s + K) % rec_T == 0 && (rc = recorder_window(rec, e->stream, e->hi.ring, s + K))) return rc;
         done += K;
@@ -1212,7 +1258,8 @@ int engine_run_output(Engine *e, int n_steps, int use_graph, int graph_steps, in
         *train = e->out_h;  // complete once engine_finish has synchronized the stream
     }
     bool recovered = false;
-    if ((rc = engine_finish(e, graph_steps, early_set ? e->train_ev : nullptr, &recovered))) return rc;
+    const unsigned long long upto = !train ? e->stats_seq : early ? early : kNoSignal;
+    if ((rc = engine_finish(e, graph_steps, upto, &recovered))) return rc;
     if (train && recovered) {  // the train of the steps launched again
         launch_out_train(e->stream, e->hi.ring, e->hi.Wr, R, row0, e->T_out, e->out_bits, e->n_out, out.out);
         HIP_TRY(hipGetLastError());
@@ -1247,8 +1294,7 @@ int engine_time(Engine *e, int n_steps, int use_graph, int graph_steps, double *
     const int chunk = chunk_for(graph_steps, e->hi.R);
     if (!ms_kernel_mean) {
         HIP_TRY(hipEventRecord(a, e->stream));
-        rc = run_steps(e->stream, e->graphs, &e->hi, e->di, 1, e->w, n_steps, use_graph, chunk, &e->kt, nullptr, nullptr,
-                       nullptr, 0, nullptr, &e->run);
+        rc = run_steps(e->stream, e->graphs, &e->hi, e->di, 1, e->w, n_steps, use_graph, chunk, &e->kt, e);
         if (rc) return rc;
         HIP_TRY(hipEventRecord(b, e->stream));
     } else {
@@ -1288,7 +1334,7 @@ int engine_time(Engine *e, int n_steps, int use_graph, int graph_steps, double *
     float ms = 0.f;
     HIP_TRY(hipEventElapsedTime(&ms, a, b));
     if (ms_total) *ms_total = ms;
-    return engine_finish(e, graph_steps);  // the step-kernel timer's events of this run
+    return engine_finish(e, graph_steps, kNoSignal);  // the step-kernel timer's events of this run
 }
 
 int engine_get_state(Engine *e, float *V, float *g, int32_t *refr)
@@ -1333,36 +1379,18 @@ int engine_get_ring_row(Engine *e, int row, uint64_t *words)
 
 int engine_get_counts(Engine *e, int row, int32_t *counts, unsigned long long *events)
 {
-    HIP_TRY(hipStreamSynchronize(e->stream));
-    if (counts)
-        HIP_TRY(hipMemcpy(counts, e->hi.counts + (size_t)row * e->n_pops, sizeof(int32_t) * e->n_pops,
-                          hipMemcpyDeviceToHost));
-    if (events) HIP_TRY(hipMemcpy(events, e->hi.events + row, sizeof(unsigned long long), hipMemcpyDeviceToHost));
+    int rc = hand_wait(e, e->stats_seq);
+    if (rc) return rc;
+    if (counts) memcpy(counts, e->counts_h + (size_t)row * e->n_pops, sizeof(int32_t) * e->n_pops);
+    if (events) *events = e->events_h[row];
     return SCAFFOLD_OK;
 }
 
 int engine_get_totals(Engine *e, unsigned long long *totals)
 {
-    HIP_TRY(hipStreamSynchronize(e->stream));
-    HIP_TRY(hipMemcpy(totals, e->hi.totals, sizeof(unsigned long long) * (e->n_pops + 1), hipMemcpyDeviceToHost));
-    return SCAFFOLD_OK;
-}
-
-// The next signal of the engine's stream.
-static ScSignal hand_signal(Engine *e) { return ScSignal{&e->hand_d->ready, ++e->seq}; }
-
-// Waits until signal `seq` is in.  The host reads the word for about as long as short
-// work takes (a read of the word is seen 3-8 us sooner than the runtime's wait returns), then
-// leaves the wait to the runtime, which also reports what went wrong on the stream.
-static int hand_wait(Engine *e, unsigned long long seq)
-{
-    const auto arrived = [&] { return __atomic_load_n(&e->hand->ready, __ATOMIC_ACQUIRE) >= seq; };
-    const auto t0 = std::chrono::steady_clock::now();
-    while (!arrived()) {
-        for (int i = 0; i < 64 && !arrived(); ++i) __builtin_ia32_pause();
-        if (std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) break;
-    }
-    if (!arrived()) HIP_TRY(hipStreamSynchronize(e->stream));
+    int rc = hand_wait(e, e->stats_seq);
+    if (rc) return rc;
+    memcpy(totals, e->totals_h, sizeof(unsigned long long) * (e->n_pops + 1));
     return SCAFFOLD_OK;
 }
 
@@ -1443,6 +1471,7 @@ int engine_copy_probe(int64_t bytes, int iters, double *ms)
 struct Batch {
     hipStream_t stream = nullptr;
     std::vector<void *> allocs;
+    std::vector<hipStream_t> inst_streams;  // the engines' own
     ScInstance *di = nullptr;
     int n_inst = 0;
     int min_R = 0;
@@ -1491,6 +1520,7 @@ int batch_build(Batch **out, std::vector<Engine *> &engines, const std::vector<c
     for (size_t i = 0; i < engines.size(); ++i) {
         const Engine *e = engines[i];
         insts.push_back(e->hi);
+        b->inst_streams.push_back(e->stream);
         b->min_R = std::min(b->min_R, e->hi.R);
         for (ScLaneTask t : e->h_lanes) { t.inst = (int)i; lanes.push_back(t); }
         lane_win.insert(lane_win.end(), e->h_lane_win.begin(), e->h_lane_win.end());
@@ -1530,6 +1560,8 @@ int batch_run(Batch *b, int n_steps, int graph_steps, double *ms)
     int rc = L.make(&e0);
     if (!rc) rc = L.make(&e1);
     if (rc) return rc;
+    // what calls on the networks themselves left queued: new rates, the end of a run
+    for (hipStream_t x : b->inst_streams) HIP_TRY(hipStreamSynchronize(x));
     HIP_TRY(hipEventRecord(e0, b->stream));
     rc = run_steps(b->stream, b->graphs, nullptr, b->di, b->n_inst, b->w, n_steps, 1,
                    chunk_for(graph_steps, b->min_R));

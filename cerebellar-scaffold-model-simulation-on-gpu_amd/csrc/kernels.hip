@@ -1876,6 +1876,13 @@ k_run(ScInstance I0, ScLayout L, const ScLaneTask *__restrict__ lanes,
     (void)run_complete(I0, r, &run_lds);
 }
 
+// The caller's data in mapped host memory is complete (its stores before the block's
+// last barrier, each thread's own fenced at system scope): tells the host.
+__device__ __forceinline__ void signal_host(const ScSignal &sig)
+{
+    __hip_atomic_store(sig.ready, sig.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Per-population spike counts and synaptic events of K consecutive steps.  The
 // ring row of each (instance, step) is cut into chunks of SC_STATS_CHUNK spike
 // words, one block each: popcounts per population and the out-degrees of the set
@@ -1961,47 +1968,81 @@ __device__ __forceinline__ void stats_block(const ScInstance &I0, const ScInstan
     }
 }
 
-// The end of a run of K steps in one launch: blocks [0, n_stats) are the
-// statistics blocks above; the blocks after them (one instance, O.out set) write
-// the output spike train of the run's last O.T steps: byte (s, c) is the spike of
-// output neuron c (device bit O.bits[c]) at step s, row-major by step, as
-// loop_n_steps hands it over (GPUScaffoldSimulation.cu:777).  Every block reads the
+// The end of a run of K steps in one launch: blocks [0, n_out) (one instance, O.out
+// set) write the output spike train of the run's last O.T steps: byte (s, c) is the
+// spike of output neuron c (device bit O.bits[c]) at step s, row-major by step, as
+// loop_n_steps hands it over (GPUScaffoldSimulation.cu:777), and signal O.sig; the
+// blocks after them are the statistics blocks above.  Every block reads the
 // step counters (the run's ring rows); once it no longer does, it counts itself in
-// *done, and the last block to arrive advances the counters of every instance by K
-// (n, m, ring row; the window-count recount flag cleared) and resets *done for the
+// done[0] (the train's blocks count themselves in done[1] before), and the last block
+// to arrive copies the run's counts and events and the totals to their places in host
+// memory, signals `stats`, advances the counters of every instance by K
+// (n, m, ring row; the window-count recount flag cleared) and resets the counts for the
 // next launch (run_done, the resident run's count of finished blocks, as well).
 // After a resident run that was given up nothing is counted or advanced; the run's
 // steps are added to those the host has to launch again.
+//
+// The train in a launch of its own before this one, an event behind it, and copies of
+// the statistics on request took a one-step exchange of a 9.9k-cell network 72 us (the
+// rates' copy included), this way 27.
 template <bool SINGLE>
 __global__ void __launch_bounds__(SC_STATS_CHUNK / 2) k_run_end(ScInstance I0, const ScInstance *__restrict__ insts,
-                                                                 int n_inst, int K, int nchunk, int n_stats, ScOut O,
-                                                                 unsigned int *__restrict__ done,
+                                                                 int n_inst, int K, int nchunk, int n_out, ScOut O,
+                                                                 ScSignal stats, unsigned int *__restrict__ done,
                                                                  unsigned int *__restrict__ run_done)
 {
     __shared__ int last;
     const int b = blockIdx.x;
     if (SINGLE && run_done && I0.ctl->failed) {
-        if (b == 0 && threadIdx.x == 0) I0.ctl->skipped += K;
+        if (b == 0 && threadIdx.x == 0) {
+            I0.ctl->skipped += K;
+            if (O.sig.ready) signal_host(O.sig);
+            if (stats.ready) signal_host(stats);
+        }
         return;
     }
-    if (b < n_stats) {
-        stats_block<SINGLE>(I0, insts, K, nchunk, b);
+    if (b >= n_out) {
+        stats_block<SINGLE>(I0, insts, K, nchunk, b - n_out);
     } else {
-        const int i = (b - n_stats) * (int)blockDim.x + (int)threadIdx.x;
+        const int i = b * (int)blockDim.x + (int)threadIdx.x;
         if (i < O.T * O.n_out) {
             const int st = i / O.n_out, c = i - st * O.n_out;
             const int row = run_row(I0, K - O.T + st);
             const int bit = O.bits[c];
             O.out[i] = (uint8_t)((I0.ring[(int64_t)row * I0.Wr + (bit >> 6)] >> (bit & 63)) & 1ull);
         }
+        if (O.sig.ready) {
+            __threadfence_system();
+            __syncthreads();
+            if (threadIdx.x == 0 && atomicAdd(done + 1, 1u) == (unsigned)n_out - 1u) {
+                done[1] = 0u;
+                signal_host(O.sig);
+            }
+        }
     }
     __syncthreads();  // every read of the counters in this block is done
-    if (threadIdx.x == 0) {
+    if (threadIdx.x == 0) {  // (the block's statistics were stored by this wavefront)
         __threadfence();
         last = atomicAdd(done, 1u) == gridDim.x - 1;
     }
     __syncthreads();
     if (!last) return;
+    constexpr int COPY = 256;  // the threads that copy: each of their wavefronts ends with a fence
+    for (int inst = 0; inst < n_inst && threadIdx.x < COPY; ++inst) {
+        const ScInstance &I = inst_of<SINGLE>(I0, insts, inst);
+        const int np = I.n_pops;
+        for (int i = threadIdx.x; i < K * np; i += COPY) {
+            const int kk = i / np, at = run_row(I, kk) * np + (i - kk * np);
+            I.h_counts[at] = (int32_t)ld_agent(reinterpret_cast<const uint32_t *>(I.counts) + at);
+        }
+        for (int kk = threadIdx.x; kk < K; kk += COPY) {
+            const int row = run_row(I, kk);
+            I.h_events[row] = ld_agent(I.events + row);
+        }
+        if ((int)threadIdx.x <= np) I.h_totals[threadIdx.x] = ld_agent(I.totals + threadIdx.x);
+    }
+    if (stats.ready && threadIdx.x < COPY) __threadfence_system();
+    __syncthreads();
     for (int i = threadIdx.x; i < n_inst; i += blockDim.x) {
         const ScInstance &I = inst_of<SINGLE>(I0, insts, i);
         ScCtl *c = I.ctl;
@@ -2011,9 +2052,20 @@ __global__ void __launch_bounds__(SC_STATS_CHUNK / 2) k_run_end(ScInstance I0, c
         c->recount = 0;
     }
     if (threadIdx.x == 0) {
-        *done = 0u;
+        done[0] = 0u;
         if (run_done) *run_done = 0u;
+        if (stats.ready) signal_host(stats);
     }
+}
+
+// New stimulus descriptors, brought as a kernel argument: the launch takes its place in
+// the stream behind the steps already queued and nobody waits for it (a copy from host
+// memory had to wait for those steps, and took 15 us of the caller's time itself).
+__global__ void k_set_stims(ScStim *__restrict__ dst, ScStimBlock B, int n)
+{
+    constexpr int W = (int)(sizeof(ScStim) / 4);
+    const uint32_t *src = reinterpret_cast<const uint32_t *>(&B);
+    for (int i = threadIdx.x; i < n * W; i += blockDim.x) reinterpret_cast<uint32_t *>(dst)[i] = src[i];
 }
 
 __global__ void k_set_ctl(ScCtl *ctl, int64_t n, int64_t m, int row)
@@ -2137,13 +2189,6 @@ __global__ void __launch_bounds__(256) k_plastic(ScInstance I, ScPlastic P, int 
     // the window counts of this step are complete (the step kernel ran before this
     // launch): the next step updates them from these
     if (c == 0 && lane == 0) I.ctl->recount = 0;
-}
-
-// The caller's data in mapped host memory is complete (its stores before the block's
-// last barrier, each thread's own fenced at system scope): tells the host.
-__device__ __forceinline__ void signal_host(const ScSignal &sig)
-{
-    __hip_atomic_store(sig.ready, sig.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Fired-neuron list of one ring row: the spike words are the ballots of spike
@@ -2274,25 +2319,34 @@ void launch_run(hipStream_t s, const ScInstance &I, const DevWork &w, const ScRu
 }
 
 void launch_run_end(hipStream_t s, const ScInstance *single, const ScInstance *insts, int n_inst, int K,
-                    int max_groups, const ScOut *out, unsigned int *done, unsigned int *run_done)
+                    int max_groups, const ScOut *out, const ScSignal &stats, unsigned int *done, unsigned int *run_done)
 {
     if (K <= 0 || n_inst <= 0) return;
     const int nchunk = std::max(1, (max_groups + SC_STATS_CHUNK - 1) / SC_STATS_CHUNK);
     const int n_stats = K * n_inst * nchunk;
     constexpr int bs = SC_STATS_CHUNK / 2;
     ScOut o{};
-    int n_out_blocks = 0;
+    int n_out = 0;
     if (single && out && out->out && out->T * out->n_out > 0) {
         o = *out;
-        n_out_blocks = (o.T * o.n_out + bs - 1) / bs;
+        n_out = (o.T * o.n_out + bs - 1) / bs;
     }
     if (single) {
         if (nchunk > 1) k_stats_zero<true><<<K, 256, 0, s>>>(*single, insts, K);
-        k_run_end<true><<<n_stats + n_out_blocks, bs, 0, s>>>(*single, insts, 1, K, nchunk, n_stats, o, done, run_done);
+        k_run_end<true><<<n_stats + n_out, bs, 0, s>>>(*single, insts, 1, K, nchunk, n_out, o, stats, done, run_done);
     } else {
         if (nchunk > 1) k_stats_zero<false><<<K * n_inst, 256, 0, s>>>(ScInstance{}, insts, K);
-        k_run_end<false><<<n_stats, bs, 0, s>>>(ScInstance{}, insts, n_inst, K, nchunk, n_stats, o, done,
-                                                                     nullptr);
+        k_run_end<false><<<n_stats, bs, 0, s>>>(ScInstance{}, insts, n_inst, K, nchunk, 0, o, stats, done, nullptr);
+    }
+}
+
+void launch_set_stims(hipStream_t s, ScStim *dst, const ScStim *src, int n)
+{
+    for (int i = 0; i < n; i += SC_STIMS_PER_LAUNCH) {
+        const int k = std::min(n - i, SC_STIMS_PER_LAUNCH);
+        ScStimBlock B{};
+        std::copy(src + i, src + i + k, B.s);
+        k_set_stims<<<1, 256, 0, s>>>(dst + i, B, k);
     }
 }
 

@@ -29,7 +29,7 @@ struct DevWork {
     int max_groups = 0;               // most 64-neuron groups of one instance (statistics grid)
     std::vector<ScPlastic> plastic;   // plasticity rules, applied in order after each step
     const ScPlastic *d_plastic = nullptr;  // the rules on the device (window-count blocks of the step kernel)
-    unsigned int *end_done = nullptr;      // arrival counter of the run-end kernel (zero between launches)
+    unsigned int *end_done = nullptr;      // arrival counters of the run-end kernel (zero between launches)
 };
 
 // Output spike train of a run's last T steps: n_out output neurons at device bits
@@ -38,6 +38,7 @@ struct ScOut {
     const int32_t *bits = nullptr;
     uint8_t *out = nullptr;
     int T = 0, n_out = 0;
+    ScSignal sig{};  // once it is there (the run's end only)
 };
 
 // All launchers are asynchronous on stream s.  `single` != nullptr selects the
@@ -46,11 +47,15 @@ void launch_step(hipStream_t s, const ScInstance *single, const ScInstance *inst
 // The end of a run of K steps, one launch (plus a zeroing launch when a ring row
 // spans several statistics chunks): per-population counts and synaptic events of
 // the run's rows, the output spike train of its last out->T steps when out is set
-// (one instance only), then the advance of every instance's step counters by K.
-// `done` is a zeroed device counter kept for this launch sequence (the kernel
-// leaves it zero again).
+// (one instance only), then the statistics' copies in host memory (signalled by
+// `stats`) and the advance of every instance's step counters by K.
+// `done` are two zeroed device counters kept for this launch sequence (the kernel
+// leaves them zero again).
 void launch_run_end(hipStream_t s, const ScInstance *single, const ScInstance *insts, int n_inst, int K,
-                    int max_groups, const ScOut *out, unsigned int *done, unsigned int *run_done = nullptr);
+                    int max_groups, const ScOut *out, const ScSignal &stats, unsigned int *done,
+                    unsigned int *run_done = nullptr);
+// The stimulus descriptors dst[0..n) := src[0..n) (host memory, read by the call).
+void launch_set_stims(hipStream_t s, ScStim *dst, const ScStim *src, int n);
 // Blocks of a resident run that the current device holds at once, and the run (one
 // network, no plasticity rules).  launch_run_end follows with run_done = r.done.
 int run_capacity(bool idx16, int *blocks);

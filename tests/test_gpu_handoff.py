@@ -1,9 +1,12 @@
-"""Results that kernels hand over in mapped host memory, at the sizes where the hand-over
-splits: fired-neuron lists against the spike rows."""
+"""What kernels hand over in mapped host memory and take as arguments, at the sizes where
+that splits: fired-neuron lists, output trains and counts against the spike rows, rates
+against the spikes they set."""
 import math
 
 import numpy as np
 import pytest
+
+from conftest import new_env
 
 pytestmark = pytest.mark.gpu
 
@@ -40,3 +43,73 @@ def test_fired_lists_match_rows(pkg, n_input, hz):
             got, n = env.fired(step, cap=cap)
             assert n == want.size and np.array_equal(got, want[:cap])
     env.finalize()
+
+
+@pytest.mark.parametrize("n_stims", [1, 8, 9, 17])
+def test_rates_take_their_place_between_runs(pkg, n_stims):
+    """Stimulus i fires all its neurons or none, as the rates of each window say."""
+    env = pkg.NetworkEnvironment(1, n_stims + 1, 0, n_stims)
+    env.set_neuron_params(0, "cell", 0, 1, 10.0, -65.0, 2.0, 0.0, -70.0, -50.0, 1.0, pkg.NORMAL,
+                          [1.0, 0.0, 0.1, 5.0])
+    pops = []
+    for i in range(n_stims):
+        index = env.set_neuron_params(1 + i, f"in{i}", 0, 3 + i, 0, 0, 0, 0, 0, 0, 0, pkg.INPUT, [])
+        f = pkg.StimFunc()
+        f.poisson_hz, f.poisson_on, f.poisson_off, f.seed = 0.0, 0.0, math.inf, 5 + i
+        f.poisson_hz_from_freq = 1
+        env.set_input_stim_ids(index, np.arange(3 + i), f)
+        pops.append(index)
+    env.initialize(50, 25)
+    rng = np.random.default_rng(n_stims)
+    t = 0
+    for _ in range(4):
+        on = rng.integers(0, 2, n_stims)
+        env.set_input_freq([10000.0 * x for x in on])
+        env.loop_n_steps(t, 2, want_output=False)
+        t += 2
+        for step in (t - 2, t - 1):
+            counts, _ = env.counts(step)
+            assert [counts[p] for p in pops] == [x * (3 + i) for i, x in enumerate(on)]
+    spikes, _ = env.totals()
+    assert spikes.sum() == sum(env.counts(s)[0].sum() for s in range(t))
+    env.finalize()
+
+
+@pytest.mark.parametrize("T", [1, 40, 47, 100])
+def test_trains_match_rows(pkg, T):
+    """Trains of one and of several blocks, handed over by calls of one window and of several."""
+    env = new_env(pkg, 0)
+    env.initialize(2 * T, T)
+    t = 0
+    for n in (T, T, 2 * T if T > 1 else 30):
+        out = np.array(env.loop_n_steps(t, n))
+        t += n
+        rows = np.stack([env.spike_row(s) for s in range(t - T, t)])
+        base = [env.population(i).base_id for i in range(env.info().n_populations)
+                if env.population(i).device_type == pkg.OUTPUT]
+        assert np.array_equal(out, rows[:, base[0]:base[0] + out.shape[1]])
+    env.finalize()
+
+
+def test_rates_set_before_a_batch_runs(pkg):
+    """A batch runs on a stream of its own: the rates set on its networks come first."""
+    def rates(env, hz):
+        env.set_input_freq([hz] * env.info().n_stimuli)
+
+    one, alone = new_env(pkg, 0), new_env(pkg, 0)
+    for e in (one, alone):
+        e.initialize(50, 25)
+    batch = pkg.Batch([one])
+    for w, hz in enumerate((3.0, 25.0, 1.0)):
+        rates(one, hz)
+        batch.run(25)
+        rates(alone, hz)
+        alone.loop_n_steps(25 * w, 25, want_output=False)
+    assert np.array_equal(one.totals()[0], alone.totals()[0]) and one.totals()[1] == alone.totals()[1]
+    for s in range(60, 75):
+        assert np.array_equal(one.counts(s)[0], alone.counts(s)[0])
+    for x, y in zip(one.state(), alone.state()):
+        assert np.array_equal(x.view(np.uint32), y.view(np.uint32))
+    batch.destroy()
+    one.finalize()
+    alone.finalize()
