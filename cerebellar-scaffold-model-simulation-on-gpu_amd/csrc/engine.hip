@@ -4,10 +4,12 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
+#include <thread>
 #include <vector>
 
 #include "kernels.hpp"
@@ -1337,18 +1339,84 @@ int engine_time(Engine *e, int n_steps, int use_graph, int graph_steps, double *
     return engine_finish(e, graph_steps, kNoSignal);  // the step-kernel timer's events of this run
 }
 
+// The state in reference order.  A kernel reorders it on its way into the hand-off
+// buffer, part by part (kParts of them in the buffer), and the host copies each part
+// to the caller's arrays while the next ones come; above kCopyAlone neurons a few
+// threads share the copying, which the page faults of newly allocated arrays bound.
+// One copy of the records, reordered by the host, took 4.0 ms at 1.55M neurons; 1.5 ms
+// this way.
+constexpr int kParts = 4, kCopyAlone = 1 << 17, kCopyThreads = 4;
+
 int engine_get_state(Engine *e, float *V, float *g, int32_t *refr)
 {
-    HIP_TRY(hipStreamSynchronize(e->stream));
-    const size_t N = (size_t)e->Ndev;
-    std::vector<ScState> hs(N);
-    HIP_TRY(hipMemcpy(hs.data(), e->hi.st, sizeof(ScState) * N, hipMemcpyDeviceToHost));
-    for (size_t d = 0; d < N; ++d) {
-        const int r = e->dev_to_ref[d];
-        if (r < 0) continue;
-        if (V) V[r] = hs[d].V;
-        if (g) { g[2 * (size_t)r] = hs[d].g_exc; g[2 * (size_t)r + 1] = hs[d].g_inh; }
-        if (refr) refr[r] = hs[d].refr;
+    const int N = e->total_ref;
+    if (N <= 0) return SCAFFOLD_OK;
+    // (the buffer holds at least 4096 neurons, and all of a network of up to 65536)
+    const int room = (int)(e->hand_bytes / sizeof(ScState)), parts = N <= std::min(room, 16384) ? 1 : kParts;
+    const int cap = parts == 1 ? (N + 1) & ~1 : room / kParts & ~1, n_chunks = (N + cap - 1) / cap;
+    const size_t part_bytes = (size_t)cap * sizeof(ScState);
+    const unsigned long long seq0 = e->seq + 1;  // signal of chunk c: seq0 + c
+    const auto launch = [&](int c) {
+        launch_state(e->stream, e->hi, c * cap, std::min(cap, N - c * cap), cap, e->data_d + (c % parts) * part_bytes,
+                     e->w.end_done, hand_signal(e));
+        return hipGetLastError();
+    };
+    const auto copy = [&](int c) {
+        const size_t r0 = (size_t)c * cap, n = std::min((size_t)cap, (size_t)N - r0);
+        const float *from = reinterpret_cast<const float *>(e->data + (c % parts) * part_bytes);
+        if (V) memcpy(V + r0, from, n * sizeof(float));
+        if (g) memcpy(g + 2 * r0, from + cap, 2 * n * sizeof(float));
+        if (refr) memcpy(refr + r0, from + 3 * (size_t)cap, n * sizeof(int32_t));
+    };
+    int launched = 0;
+    for (; launched < std::min(parts, n_chunks); ++launched) HIP_TRY(launch(launched));
+    if (N < kCopyAlone) {
+        for (int c = 0; c < n_chunks; ++c) {
+            int rc = hand_wait(e, seq0 + c);
+            if (rc) return rc;
+            copy(c);
+            if (launched < n_chunks) HIP_TRY(launch(launched++));
+        }
+        return SCAFFOLD_OK;
+    }
+    // chunks are taken in order; copied[p]: chunks that left part p
+    std::atomic<int> next{0}, copied[kParts] = {};
+    std::atomic<bool> stop{false};
+    const auto arrived = [&](int c) { return __atomic_load_n(&e->hand->ready, __ATOMIC_ACQUIRE) >= seq0 + c; };
+    const auto work = [&] {
+        for (int c = next++; c < n_chunks; c = next++) {
+            for (int i = 0; !arrived(c); ++i) {
+                if (stop) return;
+                if (i < 4096) __builtin_ia32_pause();
+                else std::this_thread::yield();
+            }
+            copy(c);
+            copied[c % kParts].fetch_add(1);
+        }
+    };
+    std::thread helpers[kCopyThreads];
+    int n_helpers = 0;
+    try {
+        for (; n_helpers < kCopyThreads; ++n_helpers) helpers[n_helpers] = std::thread(work);
+    } catch (...) {  // no more threads: the ones that started do
+    }
+    hipError_t err = hipSuccess;
+    while (n_helpers && err == hipSuccess && launched < n_chunks) {
+        for (int i = 1; err == hipSuccess && copied[launched % kParts] < launched / kParts; ++i) {
+            __builtin_ia32_pause();
+            if ((i & 0xFFFFF) == 0 && (err = hipStreamQuery(e->stream)) == hipErrorNotReady) err = hipSuccess;
+        }
+        if (err == hipSuccess) err = launch(launched++);
+    }
+    if (err == hipSuccess && n_helpers) err = hipStreamSynchronize(e->stream);
+    if (err != hipSuccess) stop = true;
+    for (int i = 0; i < n_helpers; ++i) helpers[i].join();
+    if (err != hipSuccess) return fail(SCAFFOLD_ERR_HIP, "state read-back: %s", hipGetErrorString(err));
+    for (int c = next; c < n_chunks; ++c) {  // no thread could be started
+        int rc = hand_wait(e, seq0 + c);
+        if (rc) return rc;
+        copy(c);
+        if (launched < n_chunks) HIP_TRY(launch(launched++));
     }
     return SCAFFOLD_OK;
 }

@@ -2104,6 +2104,39 @@ __global__ void k_init_params(const ScInstance *__restrict__ ip, uint32_t k0, ui
     I.st[d].refr = 0;
 }
 
+// State of the neurons of reference ids [r0, r0 + n), in that order, into host memory:
+// `cap` potentials, 2 cap conductances, cap counters at `out`.  Each thread finds its
+// neuron through the few populations.  Bound by the bus (16 bytes a neuron).
+__global__ void __launch_bounds__(256) k_state(const ScState *__restrict__ st, const ScPop *__restrict__ pops, int n_pops,
+                                               int r0, int n, int cap, void *__restrict__ out,
+                                               unsigned int *__restrict__ done, ScSignal sig)
+{
+    const int i = blockIdx.x * (int)blockDim.x + (int)threadIdx.x;
+    if (i < n) {
+        int d = -1;
+        for (int p = 0; p < n_pops; ++p) {
+            const int at = r0 + i - pops[p].ref_base;
+            if (at >= 0 && at < pops[p].num) d = pops[p].dev_base + at;
+        }
+        if (d >= 0) {
+            float u;
+            float2 g;
+            int32_t refr;
+            load_state(st, d, u, g, refr);
+            float *V = static_cast<float *>(out);
+            V[i] = u;
+            reinterpret_cast<float2 *>(V + cap)[i] = g;
+            reinterpret_cast<int32_t *>(V + 3 * cap)[i] = refr;
+        }
+    }
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0 && atomicAdd(done, 1u) == gridDim.x - 1) {
+        *done = 0u;
+        signal_host(sig);
+    }
+}
+
 // Conductances of every device neuron set to zero (the other fields kept).
 __global__ void k_zero_g(ScState *st, int n)
 {
@@ -2364,6 +2397,12 @@ void launch_fired(hipStream_t s, const uint64_t *row, int n_groups, const ScGrou
                   int len, int32_t *count, const ScSignal &sig)
 {
     k_fired<<<1, 1024, 0, s>>>(row, n_groups, groups, out, first, len, count, sig);
+}
+
+void launch_state(hipStream_t s, const ScInstance &I, int r0, int n, int cap, void *out, unsigned int *done,
+                  const ScSignal &sig)
+{
+    if (n > 0) k_state<<<(n + 255) / 256, 256, 0, s>>>(I.st, I.pops, I.n_pops, r0, n, cap, out, done, sig);
 }
 
 void launch_zero_g(hipStream_t s, ScState *st, int n)

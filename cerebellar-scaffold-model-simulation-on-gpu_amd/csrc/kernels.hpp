@@ -71,6 +71,11 @@ void launch_copy(hipStream_t s, const void *src, void *dst, int64_t n16, int gri
 void launch_out_train(hipStream_t s, const uint64_t *ring, int Wr, int R, int row0, int T, const int32_t *bits,
                       int n_out, uint8_t *out);
 void launch_zero_g(hipStream_t s, ScState *st, int n);
+// State of n > 0 neurons from reference id r0 on into mapped host memory: potentials,
+// conductances and counters, with room for cap (even) neurons each.  `done`: a zeroed
+// counter (left zero).
+void launch_state(hipStream_t s, const ScInstance &I, int r0, int n, int cap, void *out, unsigned int *done,
+                  const ScSignal &sig);
 // The plasticity rules of one network after step k of a run (single instance).
 void launch_plastic(hipStream_t s, const ScInstance &I, const DevWork &w, int k);
 

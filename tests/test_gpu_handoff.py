@@ -113,3 +113,18 @@ def test_rates_set_before_a_batch_runs(pkg):
     batch.destroy()
     one.finalize()
     alone.finalize()
+
+
+@pytest.mark.parametrize("n_input", [1, 16382, 16384, 65537, 131070, 131071, 300001])
+def test_state_read_back_in_parts(pkg, n_input):
+    """The state that was set, read back whole, in parts, and in parts copied by threads."""
+    env = input_env(pkg, n_input, 0.0)
+    n = n_input + 1
+    rng = np.random.default_rng(n)
+    V, g = rng.standard_normal(n).astype(np.float32), rng.standard_normal(2 * n).astype(np.float32)
+    refr = rng.integers(0, 1 << 30, n).astype(np.int32)
+    env.set_state(V, g, refr)
+    for _ in range(2):
+        for got, want in zip(env.state(), (V, g, refr)):
+            assert np.array_equal(got, want)
+    env.finalize()
