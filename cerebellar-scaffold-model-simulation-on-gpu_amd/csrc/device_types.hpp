@@ -301,7 +301,9 @@ struct alignas(16) ScState {
 // synapses (source order, grouped by post row) in
 // chunks of at most SC_PLASTIC_CHUNK entries of one row, one wavefront each; a
 // chunk carries its row's trigger: the postsynaptic device bit (Hebb) or the
-// teacher's device bit (Teacher; -1: none).  Per synapse: the presynaptic
+// teacher's device bit (Teacher; -1: none).  Where rows average fewer synapses than a
+// wavefront has lanes they are packed instead: a wavefront takes 64 synapses of any
+// rows, each with its own trigger.  Per synapse: the presynaptic
 // population-local id and the index of its multiplier in `val` (the f32
 // multiplier array of the layout that holds the projection).  skip_quiet: a
 // synapse whose trigger did not spike keeps its multiplier (no A0 term, a zero
@@ -315,10 +317,12 @@ struct ScPlastic {
     const uint32_t *pre;       // population-local presynaptic id
     const uint32_t *vidx;
     const uint32_t *ch_begin;  // n_chunks + 1 synapse offsets
-    const int32_t  *ch_trig;   // per chunk
+    const int32_t  *ch_trig;   // per chunk (packed: per synapse)
     float *val;
     uint8_t *hist;             // per presynaptic neuron (groups x 64 bytes)
     int32_t n_chunks;
+    int32_t packed;
+    uint32_t n_syn;            // packed: chunk c holds synapses [64 c, 64 c + 64) of n_syn, of any rows
     int32_t pre_group0, pre_groups;  // the presynaptic population's 64-neuron groups
     int32_t rule, delay, t_delay, window;
     int32_t present;           // bit c: coefficient c is set (A0, A1_I, A1_J, A2_JI)

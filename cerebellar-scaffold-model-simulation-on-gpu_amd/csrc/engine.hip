@@ -813,7 +813,9 @@ int engine_create(Engine **out, Plan &P)
         d.ch_begin = cb;
         d.ch_trig = ct;
         d.val = const_cast<float *>(reinterpret_cast<const float *>(v));
-        d.n_chunks = (int32_t)X.ch_trig.size();
+        d.packed = X.packed ? 1 : 0;
+        d.n_syn = X.packed ? (uint32_t)X.pre.size() : 0u;
+        d.n_chunks = (int32_t)(X.packed ? (X.pre.size() + SC_WAVE - 1) / SC_WAVE : X.ch_trig.size());
         d.skip_quiet = X.skip_quiet ? 1 : 0;
         d.rule = X.rule.rule;
         d.delay = X.delay;

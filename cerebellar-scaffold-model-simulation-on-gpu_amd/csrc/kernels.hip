@@ -2162,13 +2162,18 @@ __global__ void k_zero_g(ScState *st, int n)
 // (Hebb to [0, 1], Teacher to >= 0) and rounded to a multiple of 2^grid_exp,
 // which keeps every row sum of the projection exact in f64 (so the order of the
 // gather's additions cannot change it).
+//
+// PACKED: a wavefront takes 64 synapses of any rows; each lane loads its own trigger,
+// whose spike word, the window count and the multiplier then come in one round.
+template <bool PACKED>
 __global__ void __launch_bounds__(256) k_plastic(ScInstance I, ScPlastic P, int k)
 {
     const int c = uniform((int)blockIdx.x * 4 + (int)(threadIdx.x / SC_WAVE));
     const int lane = threadIdx.x & (SC_WAVE - 1);
     if (c < P.n_chunks) {
-        const int32_t trig = uniform(P.ch_trig[c]);
-        const uint32_t b0 = (uint32_t)uniform((int)P.ch_begin[c]), b1 = (uint32_t)uniform((int)P.ch_begin[c + 1]);
+        const uint32_t b0 = PACKED ? (uint32_t)c * SC_WAVE : (uint32_t)uniform((int)P.ch_begin[c]);
+        const uint32_t b1 = PACKED ? min(b0 + SC_WAVE, P.n_syn) : (uint32_t)uniform((int)P.ch_begin[c + 1]);
+        const int32_t trig = PACKED ? P.ch_trig[min(b0 + lane, b1 - 1u)] : uniform(P.ch_trig[c]);
         const int R = I.R;
         const int row = (I.ctl->row + k) % R;
         int s_post = 0;
@@ -2176,9 +2181,9 @@ __global__ void __launch_bounds__(256) k_plastic(ScInstance I, ScPlastic P, int 
             const int r = P.rule == SC_STDP_HEBB ? row : row_back(row, P.t_delay, R);
             s_post = (int)((I.ring[(int64_t)r * I.Wr + (trig >> 6)] >> (trig & 63)) & 1ull);
         }
-        s_post = uniform(s_post);
-        if (!P.skip_quiet || s_post) {
-            constexpr int U = SC_PLASTIC_CHUNK / SC_WAVE;
+        if (!PACKED) s_post = uniform(s_post);
+        if (PACKED || !P.skip_quiet || s_post) {
+            constexpr int U = PACKED ? 1 : SC_PLASTIC_CHUNK / SC_WAVE;
             uint32_t vi[U], pr[U], h[U];
             float w[U];
 #pragma unroll
@@ -2216,7 +2221,7 @@ __global__ void __launch_bounds__(256) k_plastic(ScInstance I, ScPlastic P, int 
             }
 #pragma unroll
             for (int u = 0; u < U; ++u)
-                if (b0 + lane + u * SC_WAVE < b1) P.val[vi[u]] = w[u];
+                if (b0 + lane + u * SC_WAVE < b1 && (!PACKED || !P.skip_quiet || s_post)) P.val[vi[u]] = w[u];
         }
     }
     // the window counts of this step are complete (the step kernel ran before this
@@ -2414,7 +2419,9 @@ void launch_plastic(hipStream_t s, const ScInstance &I, const DevWork &w, int k)
 {
     for (const ScPlastic &P : w.plastic) {
         if (P.n_chunks <= 0) continue;
-        k_plastic<<<(unsigned)((P.n_chunks + 3) / 4), 256, 0, s>>>(I, P, k);
+        const unsigned blocks = (unsigned)((P.n_chunks + 3) / 4);
+        if (P.packed) k_plastic<true><<<blocks, 256, 0, s>>>(I, P, k);
+        else k_plastic<false><<<blocks, 256, 0, s>>>(I, P, k);
     }
 }
 

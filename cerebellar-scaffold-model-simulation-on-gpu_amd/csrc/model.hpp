@@ -161,6 +161,7 @@ struct PlasticPlan {
     std::vector<uint32_t> pre, vidx;
     std::vector<uint32_t> ch_begin;  // chunks of <= SC_PLASTIC_CHUNK synapses of one row
     std::vector<int32_t> ch_trig;    // per chunk: post bit (Hebb) / teacher bit (Teacher), -1: none
+    bool packed = false;             // short rows: no chunks, ch_trig per synapse
 };
 
 struct Plan {

@@ -854,6 +854,10 @@ int plan_build(scaffold_env *env, Plan &P)
             quiet_keeps = quiet_keeps && !std::signbit(x) && (r.rule != SC_STDP_HEBB || x <= 1.f);
         X.skip_quiet = quiet_keeps;
         const ScPop &post = P.pops[src.post];
+        // a wavefront per row idles the lanes a short row does not fill: with 2.3
+        // synapses a row (22k rows) k_plastic took 7.3 us a step, packed 2.8; rows as
+        // long as a wavefront are better off with one trigger (and one early exit) a chunk
+        X.packed = nnz < (int64_t)SC_WAVE * (int64_t)(src.row_ptr.size() - 1);
         for (size_t j = 0; j + 1 < src.row_ptr.size(); ++j) {
             int32_t pb = (int32_t)(post.dev_base + (int)j);  // the row's trigger
             if (tp) {  // the teacher: the first entry of the teacher projection's row (SynapticPlasticity.cu:93)
@@ -869,7 +873,8 @@ int plan_build(scaffold_env *env, Plan &P)
                 X.pre[e] = (uint32_t)src.col[e];
                 X.vidx[e] = (uint32_t)v;
             }
-            for (int64_t b = src.row_ptr[j]; b < src.row_ptr[j + 1]; b += SC_PLASTIC_CHUNK) {
+            if (X.packed) X.ch_trig.insert(X.ch_trig.end(), (size_t)(src.row_ptr[j + 1] - src.row_ptr[j]), pb);
+            for (int64_t b = src.row_ptr[j]; !X.packed && b < src.row_ptr[j + 1]; b += SC_PLASTIC_CHUNK) {
                 X.ch_trig.push_back(pb);
                 X.ch_begin.push_back((uint32_t)std::min<int64_t>(b + SC_PLASTIC_CHUNK, src.row_ptr[j + 1]));
             }

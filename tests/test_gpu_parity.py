@@ -1073,3 +1073,34 @@ def test_plasticity_across_trials(pkg, orc):
         env.reset(trial)
         ref.reset()
     env.finalize()
+
+
+@pytest.mark.parametrize("granules,rule", [(1, "teacher"), (16, "teacher"), (17, "hebb"), (333, "teacher"),
+                                           (333, "hebb")])
+def test_short_row_plasticity_bit_exact(pkg, orc, granules, rule):
+    """Rules on rows of a few synapses, whose synapses share wavefronts across rows:
+    a wavefront not full, full, one synapse over, many; a Teacher rule whose quiet
+    synapses keep their multipliers, and a Hebb rule that moves every synapse."""
+    env = pkg.NetworkEnvironment(1, 7, 16, 2, 1)
+    cfg = pkg.synth_preset(0)
+    for i, n in enumerate((granules, 60, 3, 8, 6, 6, 2, 24)):
+        cfg.counts[i] = n
+    cfg.mf_rate_hz = 60.0
+    env.describe_synthetic(cfg)
+    idx = {env.projection(i).type: i for i in range(env.info().n_projections)}
+    target = idx[13]  # glomerulus to granule, up to four synapses a row
+    if rule == "teacher":
+        r = dict(rule=pkg.STDP_TEACHER, target=target, teacher=idx[15],
+                 coefficients={pkg.A1_J: 0.0, pkg.A2_JI: -0.01}, time_window=50)
+    else:
+        r = dict(rule=pkg.STDP_HEBB, target=target, teacher=-1,
+                 coefficients={pkg.A0: -1e-4, pkg.A1_J: 2e-3, pkg.A1_I: -1e-3, pkg.A2_JI: 5e-4}, time_window=20)
+    env.set_plasticity(**r)
+    env.initialize(50, 25)
+    p = env.projection(target)
+    ref = orc.OracleSim.from_env(env)
+    ref.initialize()
+    ref.add_plasticity(r["rule"], target, r["teacher"], r["coefficients"], r["time_window"], p.grid_exp)
+    run_and_compare(env, ref, 0, 100, check_counts=False)
+    assert np.array_equal(bits(env.projection_csr(target)[2]), bits(ref.multipliers(target)))
+    env.finalize()
