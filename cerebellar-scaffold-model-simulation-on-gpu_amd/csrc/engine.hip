@@ -151,8 +151,8 @@ struct Engine {
     struct PlasticView {
         int proj;
         const float *val;
-        int64_t n_val;
-        std::vector<uint32_t> vidx;
+        const uint32_t *vidx;  // on the device
+        int64_t n;
     };
     std::vector<PlasticView> plastic_views;
 };
@@ -831,7 +831,7 @@ int engine_create(Engine **out, Plan &P)
         }
         d.affine = (int32_t)(X.rule.affine & 15u);
         e->w.plastic.push_back(d);
-        e->plastic_views.push_back(Engine::PlasticView{X.rule.target, d.val, X.n_val, X.vidx});
+        e->plastic_views.push_back(Engine::PlasticView{X.rule.target, d.val, vidx, (int64_t)X.vidx.size()});
     }
     if (!e->w.plastic.empty()) {
         ScPlastic *dp;
@@ -928,19 +928,6 @@ void engine_destroy(Engine *e)
     for (hipEvent_t x : e->kt.pool) (void)hipEventDestroy(x);
     if (e->stream) (void)hipStreamDestroy(e->stream);
     delete e;
-}
-
-int engine_read_plastic(Engine *e, int proj, float *out)
-{
-    for (const Engine::PlasticView &v : e->plastic_views) {
-        if (v.proj != proj) continue;
-        std::vector<float> buf((size_t)v.n_val);
-        HIP_TRY(hipStreamSynchronize(e->stream));
-        if (v.n_val > 0) HIP_TRY(hipMemcpy(buf.data(), v.val, sizeof(float) * (size_t)v.n_val, hipMemcpyDeviceToHost));
-        for (size_t i = 0; i < v.vidx.size(); ++i) out[i] = buf[v.vidx[i]];
-        return SCAFFOLD_OK;
-    }
-    return -1;
 }
 
 int64_t engine_device_bytes(Engine *e) { return e ? e->bytes : 0; }
@@ -1341,88 +1328,6 @@ int engine_time(Engine *e, int n_steps, int use_graph, int graph_steps, double *
     return engine_finish(e, graph_steps, kNoSignal);  // the step-kernel timer's events of this run
 }
 
-// The state in reference order.  A kernel reorders it on its way into the hand-off
-// buffer, part by part (kParts of them in the buffer), and the host copies each part
-// to the caller's arrays while the next ones come; above kCopyAlone neurons a few
-// threads share the copying, which the page faults of newly allocated arrays bound.
-// One copy of the records, reordered by the host, took 4.0 ms at 1.55M neurons; 1.5 ms
-// this way.
-constexpr int kParts = 4, kCopyAlone = 1 << 17, kCopyThreads = 4;
-
-int engine_get_state(Engine *e, float *V, float *g, int32_t *refr)
-{
-    const int N = e->total_ref;
-    if (N <= 0) return SCAFFOLD_OK;
-    // (the buffer holds at least 4096 neurons, and all of a network of up to 65536)
-    const int room = (int)(e->hand_bytes / sizeof(ScState)), parts = N <= std::min(room, 16384) ? 1 : kParts;
-    const int cap = parts == 1 ? (N + 1) & ~1 : room / kParts & ~1, n_chunks = (N + cap - 1) / cap;
-    const size_t part_bytes = (size_t)cap * sizeof(ScState);
-    const unsigned long long seq0 = e->seq + 1;  // signal of chunk c: seq0 + c
-    const auto launch = [&](int c) {
-        launch_state(e->stream, e->hi, c * cap, std::min(cap, N - c * cap), cap, e->data_d + (c % parts) * part_bytes,
-                     e->w.end_done, hand_signal(e));
-        return hipGetLastError();
-    };
-    const auto copy = [&](int c) {
-        const size_t r0 = (size_t)c * cap, n = std::min((size_t)cap, (size_t)N - r0);
-        const float *from = reinterpret_cast<const float *>(e->data + (c % parts) * part_bytes);
-        if (V) memcpy(V + r0, from, n * sizeof(float));
-        if (g) memcpy(g + 2 * r0, from + cap, 2 * n * sizeof(float));
-        if (refr) memcpy(refr + r0, from + 3 * (size_t)cap, n * sizeof(int32_t));
-    };
-    int launched = 0;
-    for (; launched < std::min(parts, n_chunks); ++launched) HIP_TRY(launch(launched));
-    if (N < kCopyAlone) {
-        for (int c = 0; c < n_chunks; ++c) {
-            int rc = hand_wait(e, seq0 + c);
-            if (rc) return rc;
-            copy(c);
-            if (launched < n_chunks) HIP_TRY(launch(launched++));
-        }
-        return SCAFFOLD_OK;
-    }
-    // chunks are taken in order; copied[p]: chunks that left part p
-    std::atomic<int> next{0}, copied[kParts] = {};
-    std::atomic<bool> stop{false};
-    const auto arrived = [&](int c) { return __atomic_load_n(&e->hand->ready, __ATOMIC_ACQUIRE) >= seq0 + c; };
-    const auto work = [&] {
-        for (int c = next++; c < n_chunks; c = next++) {
-            for (int i = 0; !arrived(c); ++i) {
-                if (stop) return;
-                if (i < 4096) __builtin_ia32_pause();
-                else std::this_thread::yield();
-            }
-            copy(c);
-            copied[c % kParts].fetch_add(1);
-        }
-    };
-    std::thread helpers[kCopyThreads];
-    int n_helpers = 0;
-    try {
-        for (; n_helpers < kCopyThreads; ++n_helpers) helpers[n_helpers] = std::thread(work);
-    } catch (...) {  // no more threads: the ones that started do
-    }
-    hipError_t err = hipSuccess;
-    while (n_helpers && err == hipSuccess && launched < n_chunks) {
-        for (int i = 1; err == hipSuccess && copied[launched % kParts] < launched / kParts; ++i) {
-            __builtin_ia32_pause();
-            if ((i & 0xFFFFF) == 0 && (err = hipStreamQuery(e->stream)) == hipErrorNotReady) err = hipSuccess;
-        }
-        if (err == hipSuccess) err = launch(launched++);
-    }
-    if (err == hipSuccess && n_helpers) err = hipStreamSynchronize(e->stream);
-    if (err != hipSuccess) stop = true;
-    for (int i = 0; i < n_helpers; ++i) helpers[i].join();
-    if (err != hipSuccess) return fail(SCAFFOLD_ERR_HIP, "state read-back: %s", hipGetErrorString(err));
-    for (int c = next; c < n_chunks; ++c) {  // no thread could be started
-        int rc = hand_wait(e, seq0 + c);
-        if (rc) return rc;
-        copy(c);
-        if (launched < n_chunks) HIP_TRY(launch(launched++));
-    }
-    return SCAFFOLD_OK;
-}
-
 int engine_set_state(Engine *e, const float *V, const float *g, const int32_t *refr)
 {
     HIP_TRY(hipStreamSynchronize(e->stream));
@@ -1462,6 +1367,114 @@ int engine_get_totals(Engine *e, unsigned long long *totals)
     if (rc) return rc;
     memcpy(totals, e->totals_h, sizeof(unsigned long long) * (e->n_pops + 1));
     return SCAFFOLD_OK;
+}
+
+// A result that is handed over in parts: launch(c) queues the kernel that writes chunk c
+// into part c % parts of the hand-off buffer and asks for one signal; copy(c) takes it out.
+// Chunks are copied while the next ones come; for results above kCopyAlone bytes a few
+// threads share the copying, which the page faults of newly allocated arrays bound.
+constexpr int kParts = 4, kCopyThreads = 4;
+constexpr size_t kCopyAlone = 2 << 20;
+
+template <typename Launch, typename Copy>
+static int hand_parts(Engine *e, int n_chunks, int parts, size_t bytes, const Launch &launch, const Copy &copy)
+{
+    const unsigned long long seq0 = e->seq + 1;  // signal of chunk c: seq0 + c
+    int launched = 0;
+    const auto launch_next = [&] {
+        launch(launched++);
+        return hipGetLastError();
+    };
+    while (launched < std::min(parts, n_chunks)) HIP_TRY(launch_next());
+    const auto alone = [&](int c) {
+        for (; c < n_chunks; ++c) {
+            int rc = hand_wait(e, seq0 + c);
+            if (rc) return rc;
+            copy(c);
+            if (launched < n_chunks) HIP_TRY(launch_next());
+        }
+        return (int)SCAFFOLD_OK;
+    };
+    if (bytes < kCopyAlone || parts < kParts) return alone(0);
+    // chunks are taken in order; copied[p]: chunks that left part p
+    std::atomic<int> next{0}, copied[kParts] = {};
+    std::atomic<bool> stop{false};
+    const auto arrived = [&](int c) { return __atomic_load_n(&e->hand->ready, __ATOMIC_ACQUIRE) >= seq0 + c; };
+    const auto work = [&] {
+        for (int c = next++; c < n_chunks; c = next++) {
+            for (int i = 0; !arrived(c); ++i) {
+                if (stop) return;
+                if (i < 4096) __builtin_ia32_pause();
+                else std::this_thread::yield();
+            }
+            copy(c);
+            copied[c % kParts].fetch_add(1);
+        }
+    };
+    std::thread helpers[kCopyThreads];
+    int n_helpers = 0;
+    try {
+        for (; n_helpers < kCopyThreads; ++n_helpers) helpers[n_helpers] = std::thread(work);
+    } catch (...) {  // no more threads: the ones that started do
+    }
+    if (!n_helpers) return alone(0);
+    hipError_t err = hipSuccess;
+    while (err == hipSuccess && launched < n_chunks) {
+        for (int i = 1; err == hipSuccess && copied[launched % kParts] < launched / kParts; ++i) {
+            __builtin_ia32_pause();
+            if ((i & 0xFFFFF) == 0 && (err = hipStreamQuery(e->stream)) == hipErrorNotReady) err = hipSuccess;
+        }
+        if (err == hipSuccess) err = launch_next();
+    }
+    if (err == hipSuccess) err = hipStreamSynchronize(e->stream);
+    if (err != hipSuccess) stop = true;
+    for (int i = 0; i < n_helpers; ++i) helpers[i].join();
+    if (err != hipSuccess) return fail(SCAFFOLD_ERR_HIP, "hand-over in parts: %s", hipGetErrorString(err));
+    return SCAFFOLD_OK;
+}
+
+// The state in reference order, which a kernel brings it into.  One copy of the records,
+// reordered by the host, took 4.0 ms at 1.55M neurons; 1.5 ms this way.
+int engine_get_state(Engine *e, float *V, float *g, int32_t *refr)
+{
+    const int N = e->total_ref;
+    if (N <= 0) return SCAFFOLD_OK;
+    // (the buffer holds at least 4096 neurons, and all of a network of up to 65536)
+    const int room = (int)(e->hand_bytes / sizeof(ScState)), parts = N <= std::min(room, 16384) ? 1 : kParts;
+    const int cap = parts == 1 ? (N + 1) & ~1 : room / kParts & ~1, n_chunks = (N + cap - 1) / cap;
+    const size_t part_bytes = (size_t)cap * sizeof(ScState);
+    const auto launch = [&](int c) {
+        launch_state(e->stream, e->hi, c * cap, std::min(cap, N - c * cap), cap, e->data_d + (c % parts) * part_bytes,
+                     e->w.end_done, hand_signal(e));
+    };
+    const auto copy = [&](int c) {
+        const size_t r0 = (size_t)c * cap, n = std::min((size_t)cap, (size_t)N - r0);
+        const float *from = reinterpret_cast<const float *>(e->data + (c % parts) * part_bytes);
+        if (V) memcpy(V + r0, from, n * sizeof(float));
+        if (g) memcpy(g + 2 * r0, from + cap, 2 * n * sizeof(float));
+        if (refr) memcpy(refr + r0, from + 3 * (size_t)cap, n * sizeof(int32_t));
+    };
+    return hand_parts(e, n_chunks, parts, (size_t)N * sizeof(ScState), launch, copy);
+}
+
+// The multipliers of a plastic projection in source order, handed over like the state.
+// -1: `proj` is not plastic.
+int engine_read_plastic(Engine *e, int proj, float *out)
+{
+    for (const Engine::PlasticView &v : e->plastic_views) {
+        if (v.proj != proj) continue;
+        const int64_t cap = (int64_t)(e->hand_bytes / kParts / sizeof(float)), n_chunks = (v.n + cap - 1) / cap;
+        const auto launch = [&](int c) {
+            launch_multipliers(e->stream, v.val, v.vidx + c * cap, (int)std::min(cap, v.n - c * cap),
+                               reinterpret_cast<float *>(e->data_d) + (c % kParts) * cap, e->w.end_done, hand_signal(e));
+        };
+        const auto copy = [&](int c) {
+            memcpy(out + c * cap, reinterpret_cast<const float *>(e->data) + (c % kParts) * cap,
+                   sizeof(float) * (size_t)std::min(cap, v.n - c * cap));
+        };
+        return hand_parts(e, (int)n_chunks, kParts, (size_t)v.n * sizeof(float), launch, copy);
+    }
+    return -1;
 }
 
 int engine_get_fired(Engine *e, int row, int32_t *ids, int32_t cap, int32_t *n)

@@ -2104,6 +2104,17 @@ __global__ void k_init_params(const ScInstance *__restrict__ ip, uint32_t k0, ui
     I.st[d].refr = 0;
 }
 
+// The end of every block of a kernel that wrote host memory: the last one signals.
+__device__ __forceinline__ void part_complete(unsigned int *done, const ScSignal &sig)
+{
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0 && atomicAdd(done, 1u) == gridDim.x - 1) {
+        *done = 0u;
+        signal_host(sig);
+    }
+}
+
 // State of the neurons of reference ids [r0, r0 + n), in that order, into host memory:
 // `cap` potentials, 2 cap conductances, cap counters at `out`.  Each thread finds its
 // neuron through the few populations.  Bound by the bus (16 bytes a neuron).
@@ -2129,12 +2140,18 @@ __global__ void __launch_bounds__(256) k_state(const ScState *__restrict__ st, c
             reinterpret_cast<int32_t *>(V + 3 * cap)[i] = refr;
         }
     }
-    __threadfence_system();
-    __syncthreads();
-    if (threadIdx.x == 0 && atomicAdd(done, 1u) == gridDim.x - 1) {
-        *done = 0u;
-        signal_host(sig);
-    }
+    part_complete(done, sig);
+}
+
+// Multipliers of n synapses in source order (vidx: their places in the layout) into
+// host memory.
+__global__ void __launch_bounds__(256) k_multipliers(const float *__restrict__ val, const uint32_t *__restrict__ vidx,
+                                                     int n, float *__restrict__ out, unsigned int *__restrict__ done,
+                                                     ScSignal sig)
+{
+    const int i = blockIdx.x * (int)blockDim.x + (int)threadIdx.x;
+    if (i < n) out[i] = val[vidx[i]];
+    part_complete(done, sig);
 }
 
 // Conductances of every device neuron set to zero (the other fields kept).
@@ -2408,6 +2425,12 @@ void launch_state(hipStream_t s, const ScInstance &I, int r0, int n, int cap, vo
                   const ScSignal &sig)
 {
     if (n > 0) k_state<<<(n + 255) / 256, 256, 0, s>>>(I.st, I.pops, I.n_pops, r0, n, cap, out, done, sig);
+}
+
+void launch_multipliers(hipStream_t s, const float *val, const uint32_t *vidx, int n, float *out, unsigned int *done,
+                        const ScSignal &sig)
+{
+    if (n > 0) k_multipliers<<<(n + 255) / 256, 256, 0, s>>>(val, vidx, n, out, done, sig);
 }
 
 void launch_zero_g(hipStream_t s, ScState *st, int n)

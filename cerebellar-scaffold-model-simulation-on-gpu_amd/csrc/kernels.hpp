@@ -76,6 +76,9 @@ void launch_zero_g(hipStream_t s, ScState *st, int n);
 // counter (left zero).
 void launch_state(hipStream_t s, const ScInstance &I, int r0, int n, int cap, void *out, unsigned int *done,
                   const ScSignal &sig);
+// out[i] = val[vidx[i]] for n > 0 synapses, out in mapped host memory; `done` as above.
+void launch_multipliers(hipStream_t s, const float *val, const uint32_t *vidx, int n, float *out, unsigned int *done,
+                        const ScSignal &sig);
 // The plasticity rules of one network after step k of a run (single instance).
 void launch_plastic(hipStream_t s, const ScInstance &I, const DevWork &w, int k);
 

@@ -128,3 +128,18 @@ def test_state_read_back_in_parts(pkg, n_input):
         for got, want in zip(env.state(), (V, g, refr)):
             assert np.array_equal(got, want)
     env.finalize()
+
+
+@pytest.mark.parametrize("preset", [0, 1])
+def test_multipliers_read_back_in_parts(pkg, preset):
+    """A plastic projection's multipliers as they were set, read back in parts and (1.97M
+    synapses) in parts copied by threads."""
+    env = new_env(pkg, preset, plasticities=1)
+    idx = {env.projection(i).type: i for i in range(env.info().n_projections)}
+    want = env.projection_csr(idx[0])[2].copy()
+    env.set_plasticity(rule=pkg.STDP_TEACHER, target=idx[0], teacher=idx[11],
+                       coefficients={pkg.A1_J: 0.0, pkg.A2_JI: -0.01}, time_window=50)
+    env.initialize(50, 25)
+    for _ in range(2):
+        assert np.array_equal(env.projection_csr(idx[0])[2], want)
+    env.finalize()
