@@ -363,5 +363,7 @@ struct ScInstance {
     // copies of counts, events and totals in mapped host memory, as of the last run
     int32_t *h_counts;
     unsigned long long *h_events, *h_totals;
-    int32_t R, Wr, n_groups, n_pops, n_stims, Ndev, pad0, pad1;
+    int32_t R, Wr, n_groups, n_pops, n_stims, Ndev;
+    int32_t batch_row;         // in a batch's instance table: ctl->row (kept by the batch's own launches)
+    int32_t pad_;
 };

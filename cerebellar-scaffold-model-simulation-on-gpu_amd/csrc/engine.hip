@@ -992,7 +992,7 @@ static void launch_step_kernels(hipStream_t s, const ScInstance *single, const S
     }
 }
 
-static void launch_end(hipStream_t s, const ScInstance *single, const ScInstance *insts, int n_inst, const DevWork &w,
+static void launch_end(hipStream_t s, const ScInstance *single, ScInstance *insts, int n_inst, const DevWork &w,
                        int K, const ScOut *out, const ScSignal &stats = ScSignal{}, const RunSync *res = nullptr)
 {
     launch_run_end(s, single, insts, n_inst, K, w.max_groups, out, stats, w.end_done, res ? res->done : nullptr);
@@ -1005,7 +1005,7 @@ static bool same_out(const ScOut &a, const ScOut &b)
 
 // Captures `chunk` steps as a graph: the step kernels, and with `end` the run's
 // end as well (with the output train when out is set).
-static hipError_t capture_run(hipStream_t s, hipGraphExec_t *gexec, const ScInstance *single, const ScInstance *insts,
+static hipError_t capture_run(hipStream_t s, hipGraphExec_t *gexec, const ScInstance *single, ScInstance *insts,
                               int n_inst, const DevWork &w, int chunk, bool end, const ScOut *out)
 {
     hipGraph_t g = nullptr;
@@ -1021,7 +1021,7 @@ static hipError_t capture_run(hipStream_t s, hipGraphExec_t *gexec, const ScInst
 }
 
 // The graph `which` of G for runs of `chunk` steps, captured on first use.
-static int graph_for(hipStream_t s, RunGraphs &G, int which, const ScInstance *single, const ScInstance *insts,
+static int graph_for(hipStream_t s, RunGraphs &G, int which, const ScInstance *single, ScInstance *insts,
                      int n_inst, const DevWork &w, int chunk, const ScOut *out, hipGraphExec_t *ge)
 {
     RunGraphs::Slot &x = G.slot[which];
@@ -1084,7 +1084,7 @@ static int hand_wait(Engine *e, unsigned long long seq)
 // launched directly, signals the train (*train_seq; 0: no signal) and then the run's
 // statistics (e->stats_seq), so a caller that waits for the train alone does not wait
 // for the statistics.
-static int run_steps(hipStream_t s, RunGraphs &G, const ScInstance *single, const ScInstance *insts, int n_inst,
+static int run_steps(hipStream_t s, RunGraphs &G, const ScInstance *single, ScInstance *insts, int n_inst,
                      const DevWork &w, int n_steps, int use_graph, int chunk, KTimer *kt = nullptr,
                      Engine *e = nullptr, const ScOut *out = nullptr, bool *out_taken = nullptr,
                      unsigned long long *train_seq = nullptr, bool resident = true)
@@ -1646,6 +1646,7 @@ int batch_run(Batch *b, int n_steps, int graph_steps, double *ms)
     // what calls on the networks themselves left queued: new rates, the end of a run
     for (hipStream_t x : b->inst_streams) HIP_TRY(hipStreamSynchronize(x));
     HIP_TRY(hipEventRecord(e0, b->stream));
+    launch_batch_rows(b->stream, b->di, b->n_inst);
     rc = run_steps(b->stream, b->graphs, nullptr, b->di, b->n_inst, b->w, n_steps, 1,
                    chunk_for(graph_steps, b->min_R));
     if (rc) return rc;

@@ -284,6 +284,16 @@ __device__ __forceinline__ int run_row(const ScInstance &I, int k)
     return r >= I.R ? r - I.R : r;
 }
 
+// The same for an instance of a batch's table in its step kernel: the row lies in the
+// table itself, so a task reaches its ring row one dependent access to memory sooner than
+// through the step counters (8 networks, 532k cells bf16: 47.4 us a step through the
+// counters, 46.0 this way).
+__device__ __forceinline__ int batch_row(const ScInstance &I, int k)
+{
+    const int r = I.batch_row + k;
+    return r >= I.R ? r - I.R : r;
+}
+
 // Ring row of the step `back` steps before the step whose row is `row` (back < R).
 __device__ __forceinline__ int row_back(int row, int back, int R)
 {
@@ -960,7 +970,7 @@ __device__ __forceinline__ void do_team(const ScInstance &I0, const ScInstance *
     const bool gather_updates = count > 1;
     const ScInstance &I = inst_of<SINGLE>(I0, insts, h.inst);
     int row_n = row_single;
-    if (!SINGLE && active) row_n = uniform(run_row(I, k));
+    if (!SINGLE && active) row_n = uniform(batch_row(I, k));
     float u = 0.f;
     float2 gg = {0.f, 0.f};
     int32_t rf = 0;
@@ -1160,7 +1170,7 @@ __device__ __forceinline__ const uint32_t *stage_windows(uint32_t sd, uint32_t *
         const int n4 = __builtin_amdgcn_readlane((int)sd, base + F_NW) >> 2;
         const int o4 = __builtin_amdgcn_readlane((int)sd, base + F_OFF) >> 2;
         const ScInstance &I = inst_of<SINGLE>(I0, insts, inst);
-        const int rn = SINGLE ? row_single : run_row(I, k);
+        const int rn = SINGLE ? row_single : batch_row(I, k);
         const u32x4 *src = reinterpret_cast<const u32x4 *>(
             reinterpret_cast<const uint32_t *>(I.ring + (int64_t)row_back(rn, delay, I.R) * I.Wr) + w0);
         for (int cb = wave * SC_WAVE; cb < n4; cb += SC_BLOCK)
@@ -1232,14 +1242,14 @@ __device__ __forceinline__ void step_body(const ScInstance &I0, const ScInstance
     if (c == SC_CLASS_LANE) {
         const ScLaneTask &t = lanes[idx];
         const ScInstance &I = inst_of<SINGLE>(I0, insts, t.inst);
-        const int row_n = SINGLE ? row_single : uniform(run_row(I, k));
+        const int row_n = SINGLE ? row_single : uniform(batch_row(I, k));
         const ScPop &P = I.pops[t.pop];
         if (staged) lane_dispatch<IDX16, true, NT>(t, I, P, row_n, stage, lane);
         else lane_dispatch<IDX16, false, NT>(t, I, P, row_n, stage, lane);
     } else {  // stimulus blocks (never staged)
         const ScStimTask t = stt[idx];
         const ScInstance &I = inst_of<SINGLE>(I0, insts, t.inst);
-        const int row_n = SINGLE ? row_single : run_row(I, k);
+        const int row_n = SINGLE ? row_single : batch_row(I, k);
         const int d = t.group * SC_WAVE + lane;
         int spk = 0;
         if (lane < t.nvalid) {
@@ -1996,7 +2006,7 @@ __device__ __forceinline__ void stats_block(const ScInstance &I0, const ScInstan
 // the statistics on request took a one-step exchange of a 9.9k-cell network 72 us (the
 // rates' copy included), this way 27.
 template <bool SINGLE>
-__global__ void __launch_bounds__(SC_STATS_CHUNK / 2) k_run_end(ScInstance I0, const ScInstance *__restrict__ insts,
+__global__ void __launch_bounds__(SC_STATS_CHUNK / 2) k_run_end(ScInstance I0, ScInstance *insts,
                                                                  int n_inst, int K, int nchunk, int n_out, ScOut O,
                                                                  ScSignal stats, unsigned int *__restrict__ done,
                                                                  unsigned int *__restrict__ run_done)
@@ -2060,12 +2070,20 @@ __global__ void __launch_bounds__(SC_STATS_CHUNK / 2) k_run_end(ScInstance I0, c
         c->m += K;
         c->row = (c->row + K) % I.R;
         c->recount = 0;
+        if (!SINGLE) insts[i].batch_row = c->row;
     }
     if (threadIdx.x == 0) {
         done[0] = 0u;
         if (run_done) *run_done = 0u;
         if (stats.ready) signal_host(stats);
     }
+}
+
+// The rows of a batch's instance table, as its networks' own calls left them.
+__global__ void k_batch_rows(ScInstance *insts, int n_inst)
+{
+    const int i = blockIdx.x * (int)blockDim.x + (int)threadIdx.x;
+    if (i < n_inst) insts[i].batch_row = insts[i].ctl->row;
 }
 
 // New stimulus descriptors, brought as a kernel argument: the launch takes its place in
@@ -2383,7 +2401,7 @@ void launch_run(hipStream_t s, const ScInstance &I, const DevWork &w, const ScRu
     else k_run<false><<<w.n_blocks, SC_BLOCK, 0, s>>>(I, w.layout, w.lanes, w.stims, w.teams, w.stages, r);
 }
 
-void launch_run_end(hipStream_t s, const ScInstance *single, const ScInstance *insts, int n_inst, int K,
+void launch_run_end(hipStream_t s, const ScInstance *single, ScInstance *insts, int n_inst, int K,
                     int max_groups, const ScOut *out, const ScSignal &stats, unsigned int *done, unsigned int *run_done)
 {
     if (K <= 0 || n_inst <= 0) return;
@@ -2403,6 +2421,11 @@ void launch_run_end(hipStream_t s, const ScInstance *single, const ScInstance *i
         if (nchunk > 1) k_stats_zero<false><<<K * n_inst, 256, 0, s>>>(ScInstance{}, insts, K);
         k_run_end<false><<<n_stats, bs, 0, s>>>(ScInstance{}, insts, n_inst, K, nchunk, 0, o, stats, done, nullptr);
     }
+}
+
+void launch_batch_rows(hipStream_t s, ScInstance *insts, int n_inst)
+{
+    k_batch_rows<<<(n_inst + 255) / 256, 256, 0, s>>>(insts, n_inst);
 }
 
 void launch_set_stims(hipStream_t s, ScStim *dst, const ScStim *src, int n)

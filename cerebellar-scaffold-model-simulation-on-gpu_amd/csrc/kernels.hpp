@@ -51,9 +51,11 @@ void launch_step(hipStream_t s, const ScInstance *single, const ScInstance *inst
 // `stats`) and the advance of every instance's step counters by K.
 // `done` are two zeroed device counters kept for this launch sequence (the kernel
 // leaves them zero again).
-void launch_run_end(hipStream_t s, const ScInstance *single, const ScInstance *insts, int n_inst, int K,
+void launch_run_end(hipStream_t s, const ScInstance *single, ScInstance *insts, int n_inst, int K,
                     int max_groups, const ScOut *out, const ScSignal &stats, unsigned int *done,
                     unsigned int *run_done = nullptr);
+// The batch rows of an instance table, before a batch's first step after other calls.
+void launch_batch_rows(hipStream_t s, ScInstance *insts, int n_inst);
 // The stimulus descriptors dst[0..n) := src[0..n) (host memory, read by the call).
 void launch_set_stims(hipStream_t s, ScStim *dst, const ScStim *src, int n);
 // Blocks of a resident run that the current device holds at once, and the run (one

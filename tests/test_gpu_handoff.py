@@ -143,3 +143,22 @@ def test_multipliers_read_back_in_parts(pkg, preset):
     for _ in range(2):
         assert np.array_equal(env.projection_csr(idx[0])[2], want)
     env.finalize()
+
+
+def test_batch_after_a_call_on_one_of_its_networks(pkg):
+    """The batch's steps follow on from where a network's own calls left its ring."""
+    one, other, alone = (new_env(pkg, 0) for _ in range(3))
+    for e in (one, other, alone):
+        e.initialize(50, 25)
+    batch = pkg.Batch([one, other])
+    batch.run(25)
+    one.loop_n_steps(25, 17, want_output=False)
+    batch.run(60)
+    alone.loop_n_steps(0, 102, want_output=False)
+    for s in range(90, 102):
+        assert np.array_equal(one.spike_row(s), alone.spike_row(s))
+    for x, y in zip(one.state(), alone.state()):
+        assert np.array_equal(x.view(np.uint32), y.view(np.uint32))
+    batch.destroy()
+    for e in (one, other, alone):
+        e.finalize()
