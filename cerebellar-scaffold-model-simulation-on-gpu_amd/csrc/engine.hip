@@ -1029,6 +1029,9 @@ static int graph_for(hipStream_t s, RunGraphs &G, int which, const ScInstance *s
     if (!x.exec || x.chunk != chunk || !same_out(x.out, o)) {
         if (x.exec) (void)hipGraphExecDestroy(x.exec);
         x.exec = nullptr;
+        // a resident run of another engine may record an event on this stream (run_order):
+        // not while the stream is being captured
+        std::lock_guard<std::mutex> lock(g_run_mu);
         hipError_t err = capture_run(s, &x.exec, single, insts, n_inst, w, chunk, which != RunGraphs::STEPS, out);
         if (err != hipSuccess) return fail(SCAFFOLD_ERR_HIP, "graph capture: %s", hipGetErrorString(err));
         x.chunk = chunk;
