@@ -561,6 +561,8 @@ int scaffold_get_option(scaffold_env *env, const char *key, int64_t *value)
     else if (!strcmp(key, "nontemporal")) *value = o.nontemporal;
     else if (!strcmp(key, "resident")) *value = o.resident;
     else if (!strcmp(key, "run_polls")) *value = o.run_polls;
+    else if (!strcmp(key, "resident_runs")) engine_run_counts(env->eng, value, nullptr);
+    else if (!strcmp(key, "runs_given_up")) engine_run_counts(env->eng, nullptr, value);
     else return fail(SCAFFOLD_ERR_INVALID_ARG, "unknown option %s", key);
     return SCAFFOLD_OK;
 }

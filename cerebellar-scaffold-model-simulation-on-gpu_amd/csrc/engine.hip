@@ -91,6 +91,7 @@ struct RunSync {
     uint32_t *failed_h = nullptr, *failed_hd = nullptr;  // host word a given-up run sets, and its device address
     int max_steps = 0;                   // longest run whose rows the ring holds beside those it reads
     int polls = 0;                       // most polls of one wait
+    int64_t launched = 0, given_up = 0;  // runs so far (engine_run_counts)
 };
 
 // Mapped host memory that kernels of one engine hand results over in (its calls are
@@ -938,6 +939,12 @@ void engine_blocks(Engine *e, int *n_blocks, int *n_staged)
     *n_staged = e ? e->w.n_staged : 0;
 }
 
+void engine_run_counts(Engine *e, int64_t *launched, int64_t *given_up)
+{
+    if (launched) *launched = e ? e->run.launched : 0;
+    if (given_up) *given_up = e ? e->run.given_up : 0;
+}
+
 int engine_sync(Engine *e)
 {
     HIP_TRY(hipStreamSynchronize(e->stream));
@@ -1126,6 +1133,7 @@ static int run_steps(hipStream_t s, RunGraphs &G, const ScInstance *single, ScIn
             int rc = run_order(s);
             if (rc) return rc;
             launch_run(s, *single, w, ScRun{res->deps, res->tags, res->done, res->failed_hd, K, res->polls});
+            ++e->run.launched;
         } else {
             launch_step_kernels(s, single, insts, w, K);
         }
@@ -1171,6 +1179,7 @@ static int engine_recover(Engine *e, int graph_steps)
     HIP_TRY(hipDeviceSynchronize());  // the fills above, before the engine's (non-blocking) stream goes on
     *e->run.failed_h = 0u;
     e->run.deps = nullptr;
+    ++e->run.given_up;
     int rc = run_steps(e->stream, e->graphs, &e->hi, e->di, 1, e->w, steps, 0, chunk_for(graph_steps, e->hi.R));
     if (rc) return rc;
     HIP_TRY(hipStreamSynchronize(e->stream));

@@ -241,6 +241,9 @@ int engine_time(Engine *e, int n_steps, int use_graph, int graph_steps,
                 double *ms_total, double *ms_kernel_mean);
 int64_t engine_device_bytes(Engine *e);
 void engine_blocks(Engine *e, int *n_blocks, int *n_staged);
+// Resident runs launched since initialization, and how often one was given up (the
+// engine launches a kernel per step from then on).
+void engine_run_counts(Engine *e, int64_t *launched, int64_t *given_up);
 int engine_copy_probe(int64_t bytes, int iters, double *ms);
 // Current multipliers of a plastic projection in source order; returns -1 if no
 // plasticity rule targets the projection.

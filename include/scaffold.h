@@ -254,10 +254,25 @@ int scaffold_set_input_stim_ids(scaffold_env *env, int neuron_index,
  *   "graph_steps"       exchange steps per run: a run's statistics and counter
  *                       advance are one launch at its end (the length of a
  *                       captured graph with "graph" 1; a batch's runs are always
- *                       replayed as graphs).  The output train of a call is
- *                       gathered by that launch in a graph, else by a launch of
- *                       its own after the call's last step, and the call returns
- *                       once the train is written.
+ *                       replayed as graphs).  The output train of a call that
+ *                       ends with a window is gathered by the last run's end,
+ *                       else (the window ends earlier, or the last run is shorter
+ *                       than it) by a launch of its own; the call returns once
+ *                       the train is written.
+ *   "resident"          1 (default): runs of networks that fit the chip (a block
+ *                       per compute unit; no plasticity rules; a ring with room
+ *                       for 16 rows beside those a step reads) are one launch
+ *                       whose blocks stay on the chip from step to step, in calls
+ *                       of at least 16 steps without "graph" and recording; 0: a
+ *                       launch per step.  Results are identical either way
+ *   "run_polls"         most polls of one wait inside a resident run, 0 .. 2^30
+ *                       (default 2^20, about a second).  A run that exceeds it (its
+ *                       blocks were not on the chip together, e.g. beside another
+ *                       process's) is given up, nothing of it is kept, its steps are
+ *                       launched one by one, as are all later ones of the network
+ *   "resident_runs", "runs_given_up"   (scaffold_get_option only) resident runs
+ *                       launched since initialization, and how many were given up
+ *                       (after one, none is launched any more)
  *   "reset_g"           1: also zero conductances in scaffold_reset_network_env
  *                       (the reference keeps them, GPUScaffoldSimulation.cu:802-854)
  *   "stage_spikes"      1 (default): blocks whose gathers scatter over a bounded
