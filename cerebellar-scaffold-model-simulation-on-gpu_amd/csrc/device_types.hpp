@@ -256,10 +256,14 @@ struct ScLayout {
 // of the ring row (32-bit words [w0, w1) are staged) stands at LDS word lds + w.
 #define SC_DEP_ONCE  (-1)
 #define SC_RUN_BLOCKS 256  // blocks of a resident run on a whole MI355X (one per CU)
-// Fewest steps of a call worth a resident run: its start (tables, the first fetch of its
-// code, the cleared rows) and its end (every block waits for all) cost some 25 us, 2.2
-// us a step are gained (48k cells: 8 steps 217 against 207 us, 25 steps 144 against 200).
+// Fewest steps of a call whose runs are resident, and of such a run.  A run's start
+// (tables, the first fetch of its code, the cleared rows) and end (every block waits for
+// all) take 14 us at 9.9k cells (79 blocks) and 22 at 48k (253), those of a run launched
+// step by step 8; 2.1 and 1.7 us a step are gained: even at 3 and 8 steps.  50 steps in
+// runs of 5: 376 against 396 us at 9.9k cells, 426 against 405 at 24k (216 blocks), 505
+// against 461 at 48k; in runs of 13 and 12 at 48k 377 against 418.
 #define SC_RUN_MIN   16
+#define SC_RUN_LEAST(blocks) ((blocks) <= SC_RUN_BLOCKS / 2 ? 4 : 8)
 #define SC_MAX_DEP   20
 #define SC_MAIL      4
 #define SC_MAIL_MOST 192  // most blocks whose mail a block reads

@@ -1085,6 +1085,17 @@ static int hand_wait(Engine *e, unsigned long long seq)
     return SCAFFOLD_OK;
 }
 
+// Resident runs that a call of n steps is cut into, of about `chunk` steps each and
+// equally long (0: none, a launch per step).  A remainder too short for a call of its own
+// goes to the other runs where the ring has room, so 26 steps at a chunk of 25 are one
+// run.  A run below SC_RUN_LEAST steps is slower than its steps one by one.
+static int resident_runs(int n, int chunk, int max_steps, int n_blocks)
+{
+    int runs = (n + chunk - 1) / chunk;
+    if (runs > 1 && n - (runs - 1) * chunk < SC_RUN_MIN && (n + runs - 2) / (runs - 1) <= max_steps) --runs;
+    return n >= SC_RUN_MIN && n / runs >= SC_RUN_LEAST(n_blocks) ? runs : 0;
+}
+
 // n_steps steps in runs: graph replays of `chunk` steps, then direct launches for
 // the rest (every run direct without graphs).  With the timer on, each run's step
 // kernels lie between two events and its end is launched after them.  `out`: the
@@ -1103,14 +1114,17 @@ static int run_steps(hipStream_t s, RunGraphs &G, const ScInstance *single, ScIn
     if (train_seq) *train_seq = 0;
     if (n_steps <= 0) return SCAFFOLD_OK;
     const bool timer = kt && kt->on;
-    const RunSync *res =
-        e && resident && e->run.deps && !use_graph && n_steps >= SC_RUN_MIN ? &e->run : nullptr;
-    if (res) chunk = std::min(chunk, res->max_steps);
-    const int last_k = n_steps % chunk ? n_steps % chunk : chunk;  // steps of the last run
+    int n_runs = 0;  // resident runs left
+    if (e && resident && e->run.deps && !use_graph)
+        n_runs = resident_runs(n_steps, std::min(chunk, e->run.max_steps), e->run.max_steps, w.n_blocks);
+    const RunSync *res = n_runs ? &e->run : nullptr;
+    // steps of the last run
+    const int last_k = res ? n_steps / n_runs : n_steps % chunk ? n_steps % chunk : chunk;
     const ScOut *last_out = out && out->out && out->T > 0 && out->T <= last_k ? out : nullptr;
     int done = 0;
     while (done < n_steps) {
-        const int K = std::min(chunk, n_steps - done);
+        const int left = n_steps - done, K = res ? (left + n_runs - 1) / n_runs : std::min(chunk, left);
+        if (res) --n_runs;
         const bool last = done + K == n_steps;
         const ScOut *o = last ? last_out : nullptr;
         const bool graph = use_graph && K == chunk;

@@ -254,11 +254,12 @@ int scaffold_set_input_stim_ids(scaffold_env *env, int neuron_index,
  *   "graph_steps"       exchange steps per run: a run's statistics and counter
  *                       advance are one launch at its end (the length of a
  *                       captured graph with "graph" 1; a batch's runs are always
- *                       replayed as graphs).  The output train of a call that
- *                       ends with a window is gathered by the last run's end,
- *                       else (the window ends earlier, or the last run is shorter
- *                       than it) by a launch of its own; the call returns once
- *                       the train is written.
+ *                       replayed as graphs; resident runs are up to 15 steps
+ *                       longer where that saves a short last one).  The output
+ *                       train of a call that ends with a window is gathered by the
+ *                       last run's end, else (the window ends earlier, or the last
+ *                       run is shorter than it) by a launch of its own; the call
+ *                       returns once the train is written.
  *   "resident"          1 (default): runs of networks that fit the chip (a block
  *                       per compute unit; no plasticity rules; a ring with room
  *                       for 16 rows beside those a step reads) are one launch

@@ -94,3 +94,40 @@ def test_given_up_run_is_counted(pkg, orc):
     compare(env, orc.OracleSim.from_env(env), [25, 50], 25)
     assert runs(env) == (1, 1)
     env.finalize()
+
+
+@pytest.mark.parametrize("T_print,T,graph_steps,calls", [
+    # calls of (steps, resident runs): short last runs joined to the others, equal cuts
+    (50, 25, 25, [(15, 0), (16, 1), (26, 1), (40, 1), (41, 2), (51, 2), (100, 4), (1, 0)]),
+    (50, 25, 3, [(25, 0), (16, 0), (50, 0)]),        # runs too short to pay
+    (50, 25, 5, [(25, 4), (16, 3), (50, 9)]),
+    (50, 25, 10, [(25, 2), (50, 4), (16, 1)]),
+    (12, 12, 25, [(18, 1), (19, 2), (36, 2), (40, 3)]),  # a ring with room for 18 steps
+])
+def test_call_lengths_in_runs(pkg, orc, T_print, T, graph_steps, calls):
+    env = small_env(pkg, 2, graph_steps=graph_steps)
+    env.initialize(T_print, T)
+    counts, loop = [], env.loop_n_steps
+    def counted(t, n):
+        before = runs(env)[0]
+        out = loop(t, n)
+        counts.append((n, runs(env)[0] - before))
+        return out
+    env.loop_n_steps = counted
+    compare(env, orc.OracleSim.from_env(env), [n for n, _ in calls], T)
+    assert counts == calls and runs(env)[1] == 0
+    env.finalize()
+
+
+def test_short_runs_of_a_large_grid(pkg):
+    """24k cells in runs of 6 or 7 steps: a launch per step is faster there."""
+    env = new_env(pkg, 1, scale=0.25, burst_n_mf=12)
+    env.set_option("graph_steps", 5)
+    env.initialize(50, 25)
+    assert env.info().n_blocks > 128
+    env.loop_n_steps(0, 50, want_output=False)
+    assert runs(env) == (0, 0)
+    env.set_option("graph_steps", 8)
+    env.loop_n_steps(50, 50, want_output=False)
+    assert runs(env) == (6, 0)
+    env.finalize()
