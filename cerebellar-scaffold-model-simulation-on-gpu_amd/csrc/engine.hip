@@ -1179,9 +1179,14 @@ static int chunk_for(int graph_steps, int R) { return std::max(1, std::min(graph
 // After a resident run was given up (its blocks were not on the device together in
 // time, e.g. beside another process's): nothing of it or of the runs behind it was
 // stored or counted.  Launches their steps again, a kernel per step, as all later
-// ones of this engine will be.
-static int engine_recover(Engine *e, int graph_steps)
+// ones of this engine will be.  *ms_per_step: what they took.
+static int engine_recover(Engine *e, int graph_steps, double *ms_per_step)
 {
+    LocalEvents L;
+    hipEvent_t a, b;
+    int rc = L.make(&a);
+    if (!rc) rc = L.make(&b);
+    if (rc) return rc;
     HIP_TRY(hipStreamSynchronize(e->stream));
     ScCtl c;
     HIP_TRY(hipMemcpy(&c, e->hi.ctl, sizeof(c), hipMemcpyDeviceToHost));
@@ -1194,34 +1199,40 @@ static int engine_recover(Engine *e, int graph_steps)
     *e->run.failed_h = 0u;
     e->run.deps = nullptr;
     ++e->run.given_up;
-    int rc = run_steps(e->stream, e->graphs, &e->hi, e->di, 1, e->w, steps, 0, chunk_for(graph_steps, e->hi.R));
+    HIP_TRY(hipEventRecord(a, e->stream));
+    rc = run_steps(e->stream, e->graphs, &e->hi, e->di, 1, e->w, steps, 0, chunk_for(graph_steps, e->hi.R));
     if (rc) return rc;
+    HIP_TRY(hipEventRecord(b, e->stream));
     HIP_TRY(hipStreamSynchronize(e->stream));
+    float ms = 0.f;
+    HIP_TRY(hipEventElapsedTime(&ms, a, b));
+    if (ms_per_step) *ms_per_step = ms / std::max(1, steps);
     return SCAFFOLD_OK;
 }
 
 // Waits for signal `upto` (kNoSignal: for the engine's stream), then adds what the
 // step-kernel timer measured.  *recovered: a resident run was given up and its steps
-// were launched again.
-static int engine_finish(Engine *e, int graph_steps, unsigned long long upto, bool *recovered = nullptr)
+// were launched again, in *ms_per_step each; the timer leaves that call out (its events
+// lie around runs that ended early).
+static int engine_finish(Engine *e, int graph_steps, unsigned long long upto, bool *recovered = nullptr,
+                         double *ms_per_step = nullptr)
 {
     int rc = hand_wait(e, upto);
     if (rc) return rc;
+    const bool failed = __atomic_load_n(&e->hand->run_failed, __ATOMIC_ACQUIRE) != 0;
     KTimer &kt = e->kt;
     float x = 0.f;
     for (size_t i = 0; i < kt.piece_k.size(); ++i) {
         HIP_TRY(hipEventSynchronize(kt.pool[2 * i + 1]));
+        if (failed) continue;
         HIP_TRY(hipEventElapsedTime(&x, kt.pool[2 * i], kt.pool[2 * i + 1]));
         kt.ms += x;
         kt.launches += kt.piece_k[i];
     }
     kt.piece_k.clear();
     kt.used = 0;
-    if (__atomic_load_n(&e->hand->run_failed, __ATOMIC_ACQUIRE)) {
-        if (recovered) *recovered = true;
-        return engine_recover(e, graph_steps);
-    }
-    return SCAFFOLD_OK;
+    if (recovered) *recovered = failed;
+    return failed ? engine_recover(e, graph_steps, ms_per_step) : (int)SCAFFOLD_OK;
 }
 
 int engine_run(Engine *e, int n_steps, int use_graph, int graph_steps)
@@ -1350,8 +1361,12 @@ int engine_time(Engine *e, int n_steps, int use_graph, int graph_steps, double *
     HIP_TRY(hipEventSynchronize(b));
     float ms = 0.f;
     HIP_TRY(hipEventElapsedTime(&ms, a, b));
-    if (ms_total) *ms_total = ms;
-    return engine_finish(e, graph_steps, kNoSignal);  // the step-kernel timer's events of this run
+    bool recovered = false;
+    double ms_per_step = 0.0;
+    rc = engine_finish(e, graph_steps, kNoSignal, &recovered, &ms_per_step);  // (the step-kernel timer's events, too)
+    // a given-up run says nothing about the steps: those launched again do
+    if (ms_total) *ms_total = recovered ? ms_per_step * n_steps : ms;
+    return rc;
 }
 
 int engine_set_state(Engine *e, const float *V, const float *g, const int32_t *refr)

@@ -131,3 +131,22 @@ def test_short_runs_of_a_large_grid(pkg):
     env.loop_n_steps(50, 50, want_output=False)
     assert runs(env) == (6, 0)
     env.finalize()
+
+
+def test_given_up_run_is_not_timed(pkg):
+    """What is timed are the steps launched again, and the step timer leaves the call out."""
+    env = small_env(pkg, 3, run_polls=0)
+    env.initialize(50, 25)
+    env.step_timer(1)
+    env.loop_n_steps(0, 25, want_output=False)
+    assert env.step_timer() == (0.0, 0)
+    env.loop_n_steps(25, 25, want_output=False)
+    ms, launches = env.step_timer(0)
+    assert ms > 0.0 and launches == 25
+    env.finalize()
+    env = small_env(pkg, 3, run_polls=0)
+    env.initialize(50, 25)
+    given_up, later = env.time_steps(200), env.time_steps(200)
+    assert runs(env)[1] == 1 and env.info().current_step == 400
+    assert 0.5 * later < given_up < 2.0 * later
+    env.finalize()
