@@ -143,6 +143,8 @@ struct Engine {
     uint8_t *data = nullptr, *data_d = nullptr;  // behind that: hand_bytes of data
     size_t hand_bytes = 0;
     unsigned long long seq = 0;  // of the last signal asked for
+    uint64_t moved = 0;   // what has moved the step counters (runs, jumps of the step count), for batches
+    bool queued = false;  // work of a call that returned may still be on the stream (new rates, the end of a run)
     // the statistics of the last run are in host memory once this signal is in
     // (kNoSignal: once the stream is idle)
     unsigned long long stats_seq = 0;
@@ -497,7 +499,7 @@ static int upload_work(std::vector<void *> &allocs, int64_t *bytes, DevWork &w, 
                        std::vector<ScLaneTask> lanes, const std::vector<ScStimTask> &stims,
                        std::vector<ScTeamTask> teams, const std::vector<TaskWin> &lane_win,
                        const std::vector<TaskWin> &team_win, bool stage, int ratio, int n_hist,
-                       int most_blocks)
+                       int most_blocks, int n_inst)
 {
     for (size_t i = 1; i < team_t.size(); ++i)
         if (team_t[i] > team_t[i - 1]) return fail(SCAFFOLD_ERR_STATE, "team descriptors not ordered by width");
@@ -538,7 +540,7 @@ static int upload_work(std::vector<void *> &allocs, int64_t *bytes, DevWork &w, 
     w.lanes = l;
     w.stims = s;
     w.teams = t;
-    if ((rc = dalloc(allocs, bytes, &w.end_done, 2))) return rc;  // zeroed
+    if ((rc = dalloc(allocs, bytes, &w.end_done, (size_t)2 + n_inst))) return rc;  // zeroed
     w.idx16 = false;
     for (const ScLaneTask &x : lanes) w.idx16 = w.idx16 || x.idx16;
     for (const ScTeamTask &x : teams) w.idx16 = w.idx16 || x.hdr;
@@ -788,7 +790,7 @@ int engine_create(Engine **out, Plan &P)
     int most_blocks = 0;
     if ((rc = run_capacity(P.index_bits == 16, &most_blocks))) return bail(rc);
     if ((rc = upload_work(A, B, e->w, e->h_team_t, e->h_lanes, e->h_stims, e->h_teams, e->h_lane_win, e->h_team_win,
-                          P.stage != 0, P.stage_ratio, n_hist, most_blocks)))
+                          P.stage != 0, P.stage_ratio, n_hist, most_blocks, 0)))
         return bail(rc);
     // plasticity rules: per-synapse arrays; the multipliers they update are the
     // f32 arrays of the target's lane slices or merged rows
@@ -969,6 +971,7 @@ int engine_zero_g(Engine *e)
 // it is rewritten during step n, and team-mode words are assembled by atomicOr.
 int engine_set_ctl(Engine *e, int64_t n, int64_t m)
 {
+    ++e->moved;
     const int row = (int)(((n % e->hi.R) + e->hi.R) % e->hi.R);
     HIP_TRY(hipMemsetAsync(e->hi.ring + (size_t)row * e->hi.Wr, 0, sizeof(uint64_t) * e->hi.Wr, e->stream));
     launch_set_ctl(e->stream, e->hi.ctl, n, m, row);
@@ -980,6 +983,7 @@ int engine_upload_stims(Engine *e, const std::vector<ScStim> &stims)
 {
     if ((int)stims.size() != e->n_stims) return fail(SCAFFOLD_ERR_STATE, "stimulus table size changed");
     if (stims.empty()) return SCAFFOLD_OK;
+    e->queued = true;
     launch_set_stims(e->stream, e->stims, stims.data(), (int)stims.size());
     HIP_TRY(hipGetLastError());
     return SCAFFOLD_OK;
@@ -1113,6 +1117,10 @@ static int run_steps(hipStream_t s, RunGraphs &G, const ScInstance *single, ScIn
     if (out_taken) *out_taken = false;
     if (train_seq) *train_seq = 0;
     if (n_steps <= 0) return SCAFFOLD_OK;
+    if (e) {
+        e->queued = true;
+        ++e->moved;
+    }
     const bool timer = kt && kt->on;
     int n_runs = 0;  // resident runs left
     if (e && resident && e->run.deps && !use_graph)
@@ -1326,6 +1334,7 @@ int engine_time(Engine *e, int n_steps, int use_graph, int graph_steps, double *
         if (rc) return rc;
         HIP_TRY(hipEventRecord(b, e->stream));
     } else {
+        ++e->moved;
         // direct launches; one event pair brackets each run of back-to-back step
         // kernels, so the mean is per step kernel without per-launch event overhead
         std::vector<hipEvent_t> ev;
@@ -1595,7 +1604,8 @@ int engine_copy_probe(int64_t bytes, int iters, double *ms)
 struct Batch {
     hipStream_t stream = nullptr;
     std::vector<void *> allocs;
-    std::vector<hipStream_t> inst_streams;  // the engines' own
+    std::vector<Engine *> engines;
+    std::vector<uint64_t> moved;  // of each engine, after the batch's own last run (its rows are in the table)
     ScInstance *di = nullptr;
     int n_inst = 0;
     int min_R = 0;
@@ -1643,8 +1653,9 @@ int batch_build(Batch **out, std::vector<Engine *> &engines, const std::vector<c
     b->min_R = 1 << 30;
     for (size_t i = 0; i < engines.size(); ++i) {
         const Engine *e = engines[i];
+        b->engines.push_back(engines[i]);
+        b->moved.push_back(~0ull);
         insts.push_back(e->hi);
-        b->inst_streams.push_back(e->stream);
         b->min_R = std::min(b->min_R, e->hi.R);
         for (ScLaneTask t : e->h_lanes) { t.inst = (int)i; lanes.push_back(t); }
         lane_win.insert(lane_win.end(), e->h_lane_win.begin(), e->h_lane_win.end());
@@ -1668,7 +1679,7 @@ int batch_build(Batch **out, std::vector<Engine *> &engines, const std::vector<c
     int rc;
     if ((rc = dupload(b->allocs, nullptr, &b->di, insts))) return bail(rc);
     if ((rc = upload_work(b->allocs, nullptr, b->w, tw, lanes, stims, tt, lane_win, team_win, stage != 0,
-                          plans[0]->stage_ratio, 0, 0)))
+                          plans[0]->stage_ratio, 0, 0, (int)insts.size())))
         return bail(rc);
     for (const ScInstance &x : insts) b->w.max_groups = std::max(b->w.max_groups, x.n_groups);
     b->w.nontemporal = nt_all || algo > ((int64_t)64 << 20);
@@ -1685,9 +1696,16 @@ int batch_run(Batch *b, int n_steps, int graph_steps, double *ms)
     if (!rc) rc = L.make(&e1);
     if (rc) return rc;
     // what calls on the networks themselves left queued: new rates, the end of a run
-    for (hipStream_t x : b->inst_streams) HIP_TRY(hipStreamSynchronize(x));
+    for (Engine *e : b->engines) {
+        if (!e->queued) continue;
+        HIP_TRY(hipStreamSynchronize(e->stream));
+        e->queued = false;
+    }
     HIP_TRY(hipEventRecord(e0, b->stream));
-    launch_batch_rows(b->stream, b->di, b->n_inst);
+    bool moved = false;
+    for (size_t i = 0; i < b->engines.size(); ++i)
+        if (b->engines[i]->moved++ != b->moved[i]) moved = true;
+    if (moved) launch_batch_rows(b->stream, b->di, b->n_inst);
     rc = run_steps(b->stream, b->graphs, nullptr, b->di, b->n_inst, b->w, n_steps, 1,
                    chunk_for(graph_steps, b->min_R));
     if (rc) return rc;
@@ -1696,6 +1714,7 @@ int batch_run(Batch *b, int n_steps, int graph_steps, double *ms)
     float t = 0.f;
     HIP_TRY(hipEventElapsedTime(&t, e0, e1));
     if (ms) *ms = t;
+    for (size_t i = 0; i < b->engines.size(); ++i) b->moved[i] = b->engines[i]->moved;
     return SCAFFOLD_OK;
 }
 

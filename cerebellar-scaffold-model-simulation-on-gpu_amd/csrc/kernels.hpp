@@ -29,7 +29,8 @@ struct DevWork {
     int max_groups = 0;               // most 64-neuron groups of one instance (statistics grid)
     std::vector<ScPlastic> plastic;   // plasticity rules, applied in order after each step
     const ScPlastic *d_plastic = nullptr;  // the rules on the device (window-count blocks of the step kernel)
-    unsigned int *end_done = nullptr;      // arrival counters of the run-end kernel (zero between launches)
+    unsigned int *end_done = nullptr;      // arrival counters of the run-end kernel (zero between launches): 2, and
+                                           // one per instance of a batch
 };
 
 // Output spike train of a run's last T steps: n_out output neurons at device bits
@@ -49,8 +50,8 @@ void launch_step(hipStream_t s, const ScInstance *single, const ScInstance *inst
 // the run's rows, the output spike train of its last out->T steps when out is set
 // (one instance only), then the statistics' copies in host memory (signalled by
 // `stats`) and the advance of every instance's step counters by K.
-// `done` are two zeroed device counters kept for this launch sequence (the kernel
-// leaves them zero again).
+// `done` are zeroed device counters kept for this launch sequence, two and in a batch one
+// per instance (the kernel leaves them zero again).
 void launch_run_end(hipStream_t s, const ScInstance *single, ScInstance *insts, int n_inst, int K,
                     int max_groups, const ScOut *out, const ScSignal &stats, unsigned int *done,
                     unsigned int *run_done = nullptr);

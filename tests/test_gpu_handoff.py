@@ -2,6 +2,7 @@
 that splits: fired-neuron lists, output trains and counts against the spike rows, rates
 against the spikes they set."""
 import math
+import time
 
 import numpy as np
 import pytest
@@ -160,5 +161,88 @@ def test_batch_after_a_call_on_one_of_its_networks(pkg):
     for x, y in zip(one.state(), alone.state()):
         assert np.array_equal(x.view(np.uint32), y.view(np.uint32))
     batch.destroy()
+    for e in (one, other, alone):
+        e.finalize()
+
+
+def test_statistics_of_uneven_batches(pkg):
+    """Counts, events and totals of every network of a batch, as its own calls give them:
+    networks of one and of several statistics blocks a row, of few and of many rows."""
+    def nets():
+        envs = [input_env(pkg, n, hz) for n, hz in ((140000, 20.0), (3, 900.0), (131073, 0.0))]
+        for k in range(9):
+            e = new_env(pkg, 0, stim_seed=300 + k)
+            e.initialize(50, 25)
+            envs.append(e)
+        return envs
+
+    one, alone = nets(), nets()
+    batch = pkg.Batch(one)
+    t = 0
+    for n in (1, 60, 25):
+        batch.run(n)
+        for e in alone:
+            e.loop_n_steps(t, n, want_output=False)
+        t += n
+        for a, b in zip(one, alone):
+            assert np.array_equal(a.totals()[0], b.totals()[0]) and a.totals()[1] == b.totals()[1]
+            for s in range(t - n, t):
+                ca, ea = a.counts(s)
+                cb, eb = b.counts(s)
+                assert np.array_equal(ca, cb) and ea == eb
+    assert all(e.totals()[1] > 0 for e in one[3:])
+    batch.destroy()
+    for e in one + alone:
+        e.finalize()
+
+
+def test_batch_run_does_not_grow_with_every_network(pkg):
+    """A one-step run of 64 small networks is bound by launches, like one of 8: their
+    statistics are closed side by side (one after another, 3.3 times as long)."""
+    def median(n):
+        envs = [new_env(pkg, 1, scale=0.03, burst_n_mf=2, seed=400 + k) for k in range(n)]
+        for e in envs:
+            e.initialize(50, 25)
+        batch = pkg.Batch(envs)
+        for _ in range(20):
+            batch.run(1)
+        times = []
+        for _ in range(101):
+            t0 = time.perf_counter()
+            batch.run(1)
+            times.append(time.perf_counter() - t0)
+        batch.destroy()
+        for e in envs:
+            e.finalize()
+        return sorted(times)[50]
+
+    assert median(64) < 2.4 * median(8)
+
+
+def test_batches_that_share_a_network(pkg):
+    """Each batch follows on from what the other, the network's own calls, jumps of the step
+    count and timed steps made of its ring."""
+    one, other, alone = (new_env(pkg, 0) for _ in range(3))
+    for e in (one, other, alone):
+        e.initialize(50, 25)
+    both, single = pkg.Batch([one, other]), pkg.Batch([one])
+    both.run(7)
+    both.run(7)
+    single.run(5)
+    both.run(6)
+    one.time_steps(9, kernel_mean=True)
+    both.run(4)
+    one.loop_n_steps(1000, 3, want_output=False)
+    both.run(8)
+    alone.loop_n_steps(0, 38, want_output=False)
+    alone.loop_n_steps(1000, 11, want_output=False)
+    assert one.info().current_step == alone.info().current_step == 1011
+    for s in range(1000, 1011):
+        assert np.array_equal(one.spike_row(s), alone.spike_row(s))
+        assert np.array_equal(one.counts(s)[0], alone.counts(s)[0])
+    for x, y in zip(one.state(), alone.state()):
+        assert np.array_equal(x.view(np.uint32), y.view(np.uint32))
+    both.destroy()
+    single.destroy()
     for e in (one, other, alone):
         e.finalize()
