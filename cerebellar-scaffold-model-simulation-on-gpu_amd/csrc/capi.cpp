@@ -56,9 +56,17 @@ static double poisson_thr(float hz) { return (double)hz / kSec * kDT; }
 
 // The draws v whose uniform number 2^-32 + v * 2^-32 (rounded to float as the kernel
 // rounds it) lies below thr: it does not fall as v grows, so they are 0 .. *cut.
-// False when there are none.
+// False when there are none.  The number is exact up to 2^-8 (v + 1 <= 2^24); beyond,
+// rounding moves it by at most 2^-23 of itself, so the cut lies within a few 2^-23 of
+// thr * 2^32 - 1 and a few bisections find it (a network of thousands of stimuli has
+// them all recomputed with every change of rates).
 static bool draws_below(double thr, uint32_t *cut)
 {
+    if (thr <= 0x1p-8) {
+        const double n = std::max(0.0, std::ceil(thr * 0x1p32) - 1.0);
+        *cut = n > 0.0 ? (uint32_t)n - 1u : 0u;
+        return n > 0.0;
+    }
     const float inv = 2.3283064365386963e-10f;
     auto below = [&](uint32_t v) {
         const float p = (float)v * inv;
@@ -66,8 +74,11 @@ static bool draws_below(double thr, uint32_t *cut)
     };
     *cut = 0;
     if (!below(0u)) return false;
-    uint32_t lo = 0u, hi = 0xFFFFFFFFu;  // below(lo); the answer lies in [lo, hi]
-    while (lo < hi) {
+    const double most = 4294967295.0, x = std::min(most, thr * 4294967296.0 - 1.0), d = x * 0x1p-22 + 2.0;
+    uint32_t lo = (uint32_t)std::max(0.0, x - d), hi = (uint32_t)std::min(most, x + d);
+    if (!below(lo)) lo = 0u;
+    if (below(hi)) hi = UINT32_MAX;
+    while (lo < hi) {  // below(lo); the answer lies in [lo, hi]
         const uint32_t mid = lo + (hi - lo) / 2 + 1;
         if (below(mid)) lo = mid;
         else hi = mid - 1;

@@ -102,6 +102,8 @@ struct ScStim {
 
 // Stimulus descriptors that one launch of the upload kernel carries (kernel argument).
 #define SC_STIMS_PER_LAUNCH 8
+// Most stimuli whose descriptors are brought by launches; more are copied.
+#define SC_STIMS_BY_LAUNCH 40
 struct ScStimBlock {
     ScStim s[SC_STIMS_PER_LAUNCH];
 };

@@ -246,3 +246,53 @@ def test_batches_that_share_a_network(pkg):
     single.destroy()
     for e in (one, other, alone):
         e.finalize()
+
+
+def many_stimuli(pkg, n):
+    """n stimuli of one neuron each, over 20 INPUT populations, in index order."""
+    n_pops, per = 20, -(-n // 20)
+    env = pkg.NetworkEnvironment(1, n_pops + 1, 0, n)
+    env.set_neuron_params(0, "cell", 0, 1, 10.0, -65.0, 2.0, 0.0, -70.0, -50.0, 1.0, pkg.NORMAL,
+                          [1.0, 0.0, 0.1, 5.0])
+    pops = [env.set_neuron_params(1 + i, f"in{i}", 0, per, 0, 0, 0, 0, 0, 0, 0, pkg.INPUT, []) for i in range(n_pops)]
+    for k in range(n):
+        f = pkg.StimFunc()
+        f.poisson_hz, f.poisson_on, f.poisson_off, f.seed = 0.0, 0.0, math.inf, 5 + k
+        f.poisson_hz_from_freq = 1
+        env.set_input_stim_ids(pops[k // per], np.array([k % per]), f)
+    env.initialize(50, 25)
+    base = [env.population(p).base_id for p in pops]
+    return env, np.array([base[k // per] + k % per for k in range(n)])
+
+
+@pytest.mark.parametrize("n", [40, 41, 300])
+def test_rates_of_many_stimuli(pkg, n):
+    env, ids = many_stimuli(pkg, n)
+    rng = np.random.default_rng(n)
+    t = 0
+    for _ in range(4):
+        on = rng.integers(0, 2, n)
+        env.set_input_freq([10000.0 * x for x in on])
+        env.loop_n_steps(t, 2, want_output=False)
+        t += 2
+        for step in (t - 2, t - 1):
+            assert np.array_equal(env.spike_row(step)[ids], on)
+    env.finalize()
+
+
+def test_rates_do_not_grow_with_every_stimulus(pkg):
+    """New rates before a one-step exchange: 1024 stimuli took 23 times as long as 8 when
+    each 8 of them were a launch."""
+    def median(n):
+        env, _ = many_stimuli(pkg, n)
+        times = []
+        for t in range(101):
+            freqs = [4.0 + t % 2] * n
+            t0 = time.perf_counter()
+            env.set_input_freq(freqs)
+            env.loop_n_steps(t, 1, want_output=False)
+            times.append(time.perf_counter() - t0)
+        env.finalize()
+        return sorted(times)[50]
+
+    assert median(1024) < 10.0 * median(8)
