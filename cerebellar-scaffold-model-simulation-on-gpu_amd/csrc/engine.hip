@@ -91,6 +91,7 @@ struct RunSync {
     uint32_t *failed_h = nullptr, *failed_hd = nullptr;  // host word a given-up run sets, and its device address
     int max_steps = 0;                   // longest run whose rows the ring holds beside those it reads
     int polls = 0;                       // most polls of one wait
+    int cus = 0;                         // compute units of the device
     int64_t launched = 0, given_up = 0;  // runs so far (engine_run_counts)
 };
 
@@ -111,6 +112,7 @@ static_assert(sizeof(HandOff) == 64, "the data starts on a line of its own");
 
 struct Engine {
     hipStream_t stream = nullptr;
+    int device = 0;
     RunSync run;
     std::vector<void *> allocs;
     int64_t bytes = 0;
@@ -558,7 +560,7 @@ static int engine_plan_run(Engine *e, const Plan &P)
     e->run.max_steps = P.R - P.max_delay - 2;
     if (e->run.max_steps < SC_RUN_MIN) return SCAFFOLD_OK;
     int rc, most = 0;
-    if ((rc = run_capacity(e->w.idx16, &most))) return rc;
+    if ((rc = run_capacity(e->w.idx16, &most, &e->run.cus))) return rc;
     if (e->w.n_blocks > most) return SCAFFOLD_OK;
     e->run.failed_h = &e->hand->run_failed;
     e->run.failed_hd = &e->hand_d->run_failed;
@@ -584,6 +586,8 @@ int engine_create(Engine **out, Plan &P)
     auto bail = [&](int code) { engine_destroy(e); return code; };
     auto &A = e->allocs;
     int64_t *B = &e->bytes;
+    if (hipGetDevice(&e->device) != hipSuccess || e->device < 0 || e->device >= kMaxDevices)
+        return bail(fail(SCAFFOLD_ERR_CAPACITY, "device %d beyond the table of calls", e->device));
     if (hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking) != hipSuccess)
         return bail(fail(SCAFFOLD_ERR_HIP, "hipStreamCreate failed"));
     ScInstance &I = e->hi;
@@ -888,36 +892,60 @@ int engine_create(Engine **out, Plan &P)
     return SCAFFOLD_OK;
 }
 
-// Resident runs of different streams of one device follow each other: two of them
-// side by side could each hold CUs the other's blocks need.  The stream of the last
-// run on each device; another stream's next run first waits for the work that stream
-// holds then.
-static std::mutex g_run_mu;
-static hipStream_t g_run_last[kMaxDevices] = {};
-
-static int run_order(hipStream_t s)
+// Resident runs that a call of n steps is cut into, of about `chunk` steps each and
+// equally long (0: none, a launch per step).  A remainder too short for a call of its own
+// goes to the other runs where the ring has room, so 26 steps at a chunk of 25 are one
+// run.  A run below SC_RUN_LEAST steps is slower than its steps one by one.
+static int resident_runs(int n, int chunk, int max_steps, int n_blocks)
 {
-    int dev = 0;
-    HIP_TRY(hipGetDevice(&dev));
-    if (dev < 0 || dev >= kMaxDevices) return fail(SCAFFOLD_ERR_CAPACITY, "device %d beyond the run table", dev);
-    if (g_run_last[dev] && g_run_last[dev] != s) {
-        LocalEvents L;
-        hipEvent_t ev;
-        int rc = L.make(&ev);
-        if (rc) return rc;
-        HIP_TRY(hipEventRecord(ev, g_run_last[dev]));
-        HIP_TRY(hipStreamWaitEvent(s, ev, 0));
-    }
-    g_run_last[dev] = s;
-    return SCAFFOLD_OK;
+    int runs = (n + chunk - 1) / chunk;
+    if (runs > 1 && n - (runs - 1) * chunk < SC_RUN_MIN && (n + runs - 2) / (runs - 1) <= max_steps) --runs;
+    return n >= SC_RUN_MIN && n / runs >= SC_RUN_LEAST(n_blocks) ? runs : 0;
 }
 
-// The stream is idle and about to be destroyed.
-static void run_order_forget(hipStream_t s)
+// The calls under way on a device and what they hold of it.  Resident runs of two streams
+// side by side could each hold CUs the other's blocks need, so a call's runs are resident
+// only if its blocks fit beside those of every other call under way; a call returns when
+// its resident runs are done, so those that run together always fit together.  A call
+// that launches step by step waits for nobody; its kernels, two blocks to a CU, count
+// half.  Blocks are counted in whole 32nds: the hardware deals them out to 8 XCDs and 4
+// shader engines each in turn.  Two networks on two threads, us a window of 25 steps: 9.9k
+// cells (96 blocks counted) 98 by single steps, 145 with runs one after another, 72 side
+// by side; 24k cells (224) 104, 146, 96.  96.7k cells beside 24k ones whose runs hold
+// their CUs: 29k steps a second, 82k this way.
+static std::mutex g_share_mu;
+static int g_share[kMaxDevices] = {};
+
+struct ChipShare {
+    int dev, held = 0;
+    int n_runs = 0;  // resident runs of the call (0: a launch per step)
+    // A call whose kernels have n_blocks blocks and whose steps would be `runs` resident
+    // runs (0: cannot be) on a device of `cus` CUs.
+    ChipShare(int device, int n_blocks, int runs, int cus) : dev(device)
+    {
+        const auto counted = [](int n) { return (n + 31) / 32 * 32; };
+        std::lock_guard<std::mutex> lock(g_share_mu);
+        // (alone, the grid fits: engine_plan_run)
+        if (g_share[dev] == 0 || g_share[dev] + counted(n_blocks) <= cus) n_runs = runs;
+        held = n_runs ? counted(n_blocks) : counted((n_blocks + 1) / 2);
+        g_share[dev] += held;
+    }
+    ~ChipShare()
+    {
+        std::lock_guard<std::mutex> lock(g_share_mu);
+        g_share[dev] -= held;
+    }
+    ChipShare(const ChipShare &) = delete;
+    ChipShare &operator=(const ChipShare &) = delete;
+};
+
+// The share of a call of n_steps steps on engine e; `resident`: its runs may be.
+static ChipShare share_for(const Engine *e, int n_steps, int chunk, bool resident)
 {
-    std::lock_guard<std::mutex> lock(g_run_mu);
-    for (hipStream_t &x : g_run_last)
-        if (x == s) x = nullptr;
+    const int most = e->run.max_steps;
+    return ChipShare(e->device, e->w.n_blocks,
+                     resident && e->run.deps ? resident_runs(n_steps, std::min(chunk, most), most, e->w.n_blocks) : 0,
+                     e->run.cus);
 }
 
 void engine_destroy(Engine *e)
@@ -927,7 +955,6 @@ void engine_destroy(Engine *e)
     e->graphs.destroy();
     for (void *p : e->allocs) (void)hipFree(p);
     if (e->out_h) (void)hipHostFree(e->out_h);
-    run_order_forget(e->stream);
     for (hipEvent_t x : e->kt.pool) (void)hipEventDestroy(x);
     if (e->stream) (void)hipStreamDestroy(e->stream);
     delete e;
@@ -1048,9 +1075,6 @@ static int graph_for(hipStream_t s, RunGraphs &G, int which, const ScInstance *s
     if (!x.exec || x.chunk != chunk || !same_out(x.out, o)) {
         if (x.exec) (void)hipGraphExecDestroy(x.exec);
         x.exec = nullptr;
-        // a resident run of another engine may record an event on this stream (run_order):
-        // not while the stream is being captured
-        std::lock_guard<std::mutex> lock(g_run_mu);
         hipError_t err = capture_run(s, &x.exec, single, insts, n_inst, w, chunk, which != RunGraphs::STEPS, out);
         if (err != hipSuccess) return fail(SCAFFOLD_ERR_HIP, "graph capture: %s", hipGetErrorString(err));
         x.chunk = chunk;
@@ -1097,30 +1121,20 @@ static int hand_wait(Engine *e, unsigned long long seq)
     return SCAFFOLD_OK;
 }
 
-// Resident runs that a call of n steps is cut into, of about `chunk` steps each and
-// equally long (0: none, a launch per step).  A remainder too short for a call of its own
-// goes to the other runs where the ring has room, so 26 steps at a chunk of 25 are one
-// run.  A run below SC_RUN_LEAST steps is slower than its steps one by one.
-static int resident_runs(int n, int chunk, int max_steps, int n_blocks)
-{
-    int runs = (n + chunk - 1) / chunk;
-    if (runs > 1 && n - (runs - 1) * chunk < SC_RUN_MIN && (n + runs - 2) / (runs - 1) <= max_steps) --runs;
-    return n >= SC_RUN_MIN && n / runs >= SC_RUN_LEAST(n_blocks) ? runs : 0;
-}
-
 // n_steps steps in runs: graph replays of `chunk` steps, then direct launches for
 // the rest (every run direct without graphs).  With the timer on, each run's step
 // kernels lie between two events and its end is launched after them.  `out`: the
 // output train of the last out->T steps, gathered by the last run's end when that
 // run holds them all (*out_taken then set; otherwise the caller gathers it).
-// `e` (one instance, resident runs where it has them): the end of its last run, if
+// `n_runs`: the steps are that many resident runs (0: a launch per step).
+// `e` (one instance): the end of its last run, if
 // launched directly, signals the train (*train_seq; 0: no signal) and then the run's
 // statistics (e->stats_seq), so a caller that waits for the train alone does not wait
 // for the statistics.
 static int run_steps(hipStream_t s, RunGraphs &G, const ScInstance *single, ScInstance *insts, int n_inst,
                      const DevWork &w, int n_steps, int use_graph, int chunk, KTimer *kt = nullptr,
                      Engine *e = nullptr, const ScOut *out = nullptr, bool *out_taken = nullptr,
-                     unsigned long long *train_seq = nullptr, bool resident = true)
+                     unsigned long long *train_seq = nullptr, int n_runs = 0)
 {
     if (out_taken) *out_taken = false;
     if (train_seq) *train_seq = 0;
@@ -1130,9 +1144,6 @@ static int run_steps(hipStream_t s, RunGraphs &G, const ScInstance *single, ScIn
         ++e->moved;
     }
     const bool timer = kt && kt->on;
-    int n_runs = 0;  // resident runs left
-    if (e && resident && e->run.deps && !use_graph)
-        n_runs = resident_runs(n_steps, std::min(chunk, e->run.max_steps), e->run.max_steps, w.n_blocks);
     const RunSync *res = n_runs ? &e->run : nullptr;
     // steps of the last run
     const int last_k = res ? n_steps / n_runs : n_steps % chunk ? n_steps % chunk : chunk;
@@ -1159,9 +1170,6 @@ static int run_steps(hipStream_t s, RunGraphs &G, const ScInstance *single, ScIn
             if (rc) return rc;
             HIP_TRY(hipGraphLaunch(ge, s));
         } else if (res) {
-            std::lock_guard<std::mutex> lock(g_run_mu);
-            int rc = run_order(s);
-            if (rc) return rc;
             launch_run(s, *single, w, ScRun{res->deps, res->tags, res->done, res->failed_hd, K, res->polls});
             ++e->run.launched;
         } else {
@@ -1253,8 +1261,10 @@ static int engine_finish(Engine *e, int graph_steps, unsigned long long upto, bo
 
 int engine_run(Engine *e, int n_steps, int use_graph, int graph_steps)
 {
-    int rc = run_steps(e->stream, e->graphs, &e->hi, e->di, 1, e->w, n_steps, use_graph,
-                       chunk_for(graph_steps, e->hi.R), &e->kt, e);
+    const int chunk = chunk_for(graph_steps, e->hi.R);
+    const ChipShare share = share_for(e, n_steps, chunk, !use_graph);
+    int rc = run_steps(e->stream, e->graphs, &e->hi, e->di, 1, e->w, n_steps, use_graph, chunk, &e->kt, e, nullptr,
+                       nullptr, nullptr, share.n_runs);
     if (rc) return rc;
     return engine_finish(e, graph_steps, e->stats_seq);
 }
@@ -1263,6 +1273,7 @@ int engine_run_output(Engine *e, int n_steps, int use_graph, int graph_steps, in
                       const uint8_t **train, Recorder *rec, int rec_T, int64_t step0)
 {
     const int chunk = chunk_for(graph_steps, e->hi.R);
+    const ChipShare share = share_for(e, n_steps, chunk, !use_graph && !rec);
     int rc = SCAFFOLD_OK;
     // the train of steps [first_out_step, first_out_step + T_out) is gathered by
     // the end of the call's last run when the window closes the call and that run
@@ -1281,7 +1292,7 @@ int engine_run_output(Engine *e, int n_steps, int use_graph, int graph_steps, in
     unsigned long long early = 0;
     if (!rec) {
         rc = run_steps(e->stream, e->graphs, &e->hi, e->di, 1, e->w, n_steps, use_graph, chunk, &e->kt,
-                       e, closes ? &out : nullptr, &taken, &early);
+                       e, closes ? &out : nullptr, &taken, &early, share.n_runs);
         if (rc) return rc;
     }
     for (int done = 0; rec && done < n_steps;) {
@@ -1289,7 +1300,7 @@ int engine_run_output(Engine *e, int n_steps, int use_graph, int graph_steps, in
         const int K = (int)std::min<int64_t>(n_steps - done, (s / rec_T + 1) * rec_T - s);
         if ((rc = recorder_before(rec, e->stream, s + K))) return rc;
         rc = run_steps(e->stream, e->graphs, &e->hi, e->di, 1, e->w, K, use_graph, chunk, &e->kt,
-                       e, closes && done + K == n_steps ? &out : nullptr, &taken, &early, false);
+                       e, closes && done + K == n_steps ? &out : nullptr, &taken, &early);
         if (rc) return rc;
         if ((s + K) % rec_T == 0 && (rc = recorder_window(rec, e->stream, e->hi.ring, s + K))) return rc;
         done += K;
@@ -1336,9 +1347,11 @@ int engine_time(Engine *e, int n_steps, int use_graph, int graph_steps, double *
     if (!rc) rc = L.make(&b);
     if (rc) return rc;
     const int chunk = chunk_for(graph_steps, e->hi.R);
+    const ChipShare share = share_for(e, n_steps, chunk, !use_graph && !ms_kernel_mean);
     if (!ms_kernel_mean) {
         HIP_TRY(hipEventRecord(a, e->stream));
-        rc = run_steps(e->stream, e->graphs, &e->hi, e->di, 1, e->w, n_steps, use_graph, chunk, &e->kt, e);
+        rc = run_steps(e->stream, e->graphs, &e->hi, e->di, 1, e->w, n_steps, use_graph, chunk, &e->kt, e, nullptr,
+                       nullptr, nullptr, share.n_runs);
         if (rc) return rc;
         HIP_TRY(hipEventRecord(b, e->stream));
     } else {
@@ -1703,6 +1716,7 @@ int batch_run(Batch *b, int n_steps, int graph_steps, double *ms)
     int rc = L.make(&e0);
     if (!rc) rc = L.make(&e1);
     if (rc) return rc;
+    const ChipShare share(b->engines[0]->device, b->w.n_blocks, 0, 0);
     // what calls on the networks themselves left queued: new rates, the end of a run
     for (Engine *e : b->engines) {
         if (!e->queued) continue;

@@ -2404,7 +2404,7 @@ void launch_step(hipStream_t s, const ScInstance *single, const ScInstance *inst
     else launch_step_nt<false>(s, single, insts, w, k);
 }
 
-int run_capacity(bool idx16, int *blocks)
+int run_capacity(bool idx16, int *blocks, int *n_cus)
 {
     int dev = 0, cus = 0, per_cu = 0;
     HIP_TRY(hipGetDevice(&dev));
@@ -2412,6 +2412,7 @@ int run_capacity(bool idx16, int *blocks)
     HIP_TRY(idx16 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_run<true>, SC_BLOCK, 0)
                   : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_run<false>, SC_BLOCK, 0));
     *blocks = per_cu * cus;
+    if (n_cus) *n_cus = cus;
     return SCAFFOLD_OK;
 }
 

@@ -61,7 +61,7 @@ void launch_batch_rows(hipStream_t s, ScInstance *insts, int n_inst);
 void launch_set_stims(hipStream_t s, ScStim *dst, const ScStim *src, int n);
 // Blocks of a resident run that the current device holds at once, and the run (one
 // network, no plasticity rules).  launch_run_end follows with run_done = r.done.
-int run_capacity(bool idx16, int *blocks);
+int run_capacity(bool idx16, int *blocks, int *n_cus = nullptr);  // and the device's CUs
 void launch_run(hipStream_t s, const ScInstance &I, const DevWork &w, const ScRun &r);
 void launch_set_ctl(hipStream_t s, ScCtl *ctl, int64_t n, int64_t m, int row);
 void launch_init_params(hipStream_t s, const ScInstance *di, int n_threads, uint64_t seed, uint64_t off);

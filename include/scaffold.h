@@ -264,8 +264,10 @@ int scaffold_set_input_stim_ids(scaffold_env *env, int neuron_index,
  *                       per compute unit; no plasticity rules; a ring with room
  *                       for 16 rows beside those a step reads) are one launch
  *                       whose blocks stay on the chip from step to step, in calls
- *                       of at least 16 steps without "graph" and recording; 0: a
- *                       launch per step.  Results are identical either way
+ *                       of at least 16 steps without "graph" and recording, unless
+ *                       calls of other networks are under way (on other threads)
+ *                       whose blocks leave no room for this one's; 0: a launch per
+ *                       step.  Results are identical either way
  *   "run_polls"         most polls of one wait inside a resident run, 0 .. 2^30
  *                       (default 2^20, about a second).  A run that exceeds it (its
  *                       blocks were not on the chip together, e.g. beside another
