@@ -881,9 +881,7 @@ int engine_create(Engine **out, Plan &P)
         e->totals_h = st + P.R;
         e->counts_h = reinterpret_cast<const int32_t *>(st + n64);
         st = reinterpret_cast<unsigned long long *>(e->data_d + e->hand_bytes);
-        I.h_events = st;
-        I.h_totals = st + P.R;
-        I.h_counts = reinterpret_cast<int32_t *>(st + n64);
+        e->w.host = ScHostStats{reinterpret_cast<int32_t *>(st + n64), st, st + P.R};
     }
     if ((rc = engine_plan_run(e, P))) return bail(rc);
     std::vector<ScInstance> one{I};
@@ -1041,7 +1039,7 @@ static void launch_step_kernels(hipStream_t s, const ScInstance *single, const S
 static void launch_end(hipStream_t s, const ScInstance *single, ScInstance *insts, int n_inst, const DevWork &w,
                        int K, const ScOut *out, const ScSignal &stats = ScSignal{}, const RunSync *res = nullptr)
 {
-    launch_run_end(s, single, insts, n_inst, K, w.max_groups, out, stats, w.end_done, res ? res->done : nullptr);
+    launch_run_end(s, single, insts, n_inst, w, K, out, stats, res ? res->done : nullptr);
 }
 
 static bool same_out(const ScOut &a, const ScOut &b)
@@ -1662,6 +1660,7 @@ int batch_build(Batch **out, std::vector<Engine *> &engines, const std::vector<c
     if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess)
         return bail(fail(SCAFFOLD_ERR_HIP, "hipStreamCreate failed"));
     std::vector<ScInstance> insts;
+    std::vector<ScHostStats> stats;
     std::vector<ScLaneTask> lanes;
     std::vector<ScStimTask> stims;
     struct TeamEntry {
@@ -1677,6 +1676,7 @@ int batch_build(Batch **out, std::vector<Engine *> &engines, const std::vector<c
         b->engines.push_back(engines[i]);
         b->moved.push_back(~0ull);
         insts.push_back(e->hi);
+        stats.push_back(e->w.host);
         b->min_R = std::min(b->min_R, e->hi.R);
         for (ScLaneTask t : e->h_lanes) { t.inst = (int)i; lanes.push_back(t); }
         lane_win.insert(lane_win.end(), e->h_lane_win.begin(), e->h_lane_win.end());
@@ -1699,6 +1699,9 @@ int batch_build(Batch **out, std::vector<Engine *> &engines, const std::vector<c
     }
     int rc;
     if ((rc = dupload(b->allocs, nullptr, &b->di, insts))) return bail(rc);
+    ScHostStats *hosts;
+    if ((rc = dupload(b->allocs, nullptr, &hosts, stats))) return bail(rc);
+    b->w.hosts = hosts;
     if ((rc = upload_work(b->allocs, nullptr, b->w, tw, lanes, stims, tt, lane_win, team_win, stage != 0,
                           plans[0]->stage_ratio, 0, 0, (int)insts.size())))
         return bail(rc);

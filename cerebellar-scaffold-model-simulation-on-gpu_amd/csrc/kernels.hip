@@ -1990,19 +1990,19 @@ __device__ __forceinline__ void stats_block(const ScInstance &I0, const ScInstan
 // The counts and events of a run's K rows and the totals of instance I, copied to their
 // places in host memory by the block's first STATS_COPY threads.
 constexpr int STATS_COPY = 256;
-__device__ __forceinline__ void copy_stats(const ScInstance &I, int K)
+__device__ __forceinline__ void copy_stats(const ScInstance &I, const ScHostStats &H, int K)
 {
     if (threadIdx.x >= STATS_COPY) return;
     const int np = I.n_pops;
     for (int i = threadIdx.x; i < K * np; i += STATS_COPY) {
         const int kk = i / np, at = run_row(I, kk) * np + (i - kk * np);
-        I.h_counts[at] = (int32_t)ld_agent(reinterpret_cast<const uint32_t *>(I.counts) + at);
+        H.counts[at] = (int32_t)ld_agent(reinterpret_cast<const uint32_t *>(I.counts) + at);
     }
     for (int kk = threadIdx.x; kk < K; kk += STATS_COPY) {
         const int row = run_row(I, kk);
-        I.h_events[row] = ld_agent(I.events + row);
+        H.events[row] = ld_agent(I.events + row);
     }
-    if ((int)threadIdx.x <= np) I.h_totals[threadIdx.x] = ld_agent(I.totals + threadIdx.x);
+    if ((int)threadIdx.x <= np) H.totals[threadIdx.x] = ld_agent(I.totals + threadIdx.x);
 }
 
 // The end of a run of K steps in one launch: blocks [0, n_out) (one instance, O.out
@@ -2028,6 +2028,7 @@ __device__ __forceinline__ void copy_stats(const ScInstance &I, int K)
 // rates' copy included), this way 27.
 template <bool SINGLE>
 __global__ void __launch_bounds__(SC_STATS_CHUNK / 2) k_run_end(ScInstance I0, ScInstance *insts,
+                                                                 ScHostStats H0, const ScHostStats *__restrict__ hosts,
                                                                  int n_inst, int K, int nchunk, int n_out, ScOut O,
                                                                  ScSignal stats, unsigned int *__restrict__ done,
                                                                  unsigned int *__restrict__ run_done)
@@ -2054,7 +2055,7 @@ __global__ void __launch_bounds__(SC_STATS_CHUNK / 2) k_run_end(ScInstance I0, S
             __syncthreads();
             if (!inst_last) return;
             if (threadIdx.x == 0) done[2 + inst] = 0u;
-            copy_stats(insts[inst], K);
+            copy_stats(insts[inst], hosts[inst], K);
         }
     } else {
         const int i = b * (int)blockDim.x + (int)threadIdx.x;
@@ -2080,7 +2081,7 @@ __global__ void __launch_bounds__(SC_STATS_CHUNK / 2) k_run_end(ScInstance I0, S
     }
     __syncthreads();
     if (!last) return;
-    if (SINGLE) copy_stats(I0, K);
+    if (SINGLE) copy_stats(I0, H0, K);
     if (stats.ready && threadIdx.x < STATS_COPY) __threadfence_system();  // by each wavefront that copied
     __syncthreads();
     for (int i = threadIdx.x; i < n_inst; i += blockDim.x) {
@@ -2422,11 +2423,11 @@ void launch_run(hipStream_t s, const ScInstance &I, const DevWork &w, const ScRu
     else k_run<false><<<w.n_blocks, SC_BLOCK, 0, s>>>(I, w.layout, w.lanes, w.stims, w.teams, w.stages, r);
 }
 
-void launch_run_end(hipStream_t s, const ScInstance *single, ScInstance *insts, int n_inst, int K,
-                    int max_groups, const ScOut *out, const ScSignal &stats, unsigned int *done, unsigned int *run_done)
+void launch_run_end(hipStream_t s, const ScInstance *single, ScInstance *insts, int n_inst, const DevWork &w, int K,
+                    const ScOut *out, const ScSignal &stats, unsigned int *run_done)
 {
     if (K <= 0 || n_inst <= 0) return;
-    const int nchunk = std::max(1, (max_groups + SC_STATS_CHUNK - 1) / SC_STATS_CHUNK);
+    const int nchunk = std::max(1, (w.max_groups + SC_STATS_CHUNK - 1) / SC_STATS_CHUNK);
     const int n_stats = K * n_inst * nchunk;
     constexpr int bs = SC_STATS_CHUNK / 2;
     ScOut o{};
@@ -2437,10 +2438,12 @@ void launch_run_end(hipStream_t s, const ScInstance *single, ScInstance *insts, 
     }
     if (single) {
         if (nchunk > 1) k_stats_zero<true><<<K, 256, 0, s>>>(*single, insts, K);
-        k_run_end<true><<<n_stats + n_out, bs, 0, s>>>(*single, insts, 1, K, nchunk, n_out, o, stats, done, run_done);
+        k_run_end<true><<<n_stats + n_out, bs, 0, s>>>(*single, insts, w.host, nullptr, 1, K, nchunk, n_out, o,
+                                                         stats, w.end_done, run_done);
     } else {
         if (nchunk > 1) k_stats_zero<false><<<K * n_inst, 256, 0, s>>>(ScInstance{}, insts, K);
-        k_run_end<false><<<n_stats, bs, 0, s>>>(ScInstance{}, insts, n_inst, K, nchunk, 0, o, stats, done, nullptr);
+        k_run_end<false><<<n_stats, bs, 0, s>>>(ScInstance{}, insts, ScHostStats{}, w.hosts, n_inst, K, nchunk, 0, o, stats,
+                                                  w.end_done, nullptr);
     }
 }
 

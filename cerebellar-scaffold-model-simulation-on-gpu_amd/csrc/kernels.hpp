@@ -31,6 +31,8 @@ struct DevWork {
     const ScPlastic *d_plastic = nullptr;  // the rules on the device (window-count blocks of the step kernel)
     unsigned int *end_done = nullptr;      // arrival counters of the run-end kernel (zero between launches): 2, and
                                            // one per instance of a batch
+    ScHostStats host{};                    // places of the statistics' copies (one network)
+    const ScHostStats *hosts = nullptr;    // per instance of a batch, on the device
 };
 
 // Output spike train of a run's last T steps: n_out output neurons at device bits
@@ -50,11 +52,8 @@ void launch_step(hipStream_t s, const ScInstance *single, const ScInstance *inst
 // the run's rows, the output spike train of its last out->T steps when out is set
 // (one instance only), then the statistics' copies in host memory (signalled by
 // `stats`) and the advance of every instance's step counters by K.
-// `done` are zeroed device counters kept for this launch sequence, two and in a batch one
-// per instance (the kernel leaves them zero again).
-void launch_run_end(hipStream_t s, const ScInstance *single, ScInstance *insts, int n_inst, int K,
-                    int max_groups, const ScOut *out, const ScSignal &stats, unsigned int *done,
-                    unsigned int *run_done = nullptr);
+void launch_run_end(hipStream_t s, const ScInstance *single, ScInstance *insts, int n_inst, const DevWork &w, int K,
+                    const ScOut *out, const ScSignal &stats, unsigned int *run_done = nullptr);
 // The batch rows of an instance table, before a batch's first step after other calls.
 void launch_batch_rows(hipStream_t s, ScInstance *insts, int n_inst);
 // The stimulus descriptors dst[0..n) := src[0..n) (host memory, read by the call).
