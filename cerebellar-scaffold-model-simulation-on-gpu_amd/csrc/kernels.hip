@@ -639,10 +639,11 @@ __device__ __forceinline__ float wone(const void *val, uint32_t i)
 // first index plus the number of mask bits below it.  The sums of up to SC_GROUP_LOADS
 // spiking entries go to the team's f64 LDS accumulator of the projection: atomics on one
 // LDS word follow each other, and with one for every spiking entry a step at strong drive
-// (96.7k cells f32, 60 Hz mossy rate) took 15.5 us, 14.1 this way.  A group's single spike,
-// the usual one at low rates, skips the additions: without that branch a step took 9.6 us
-// at 4 Hz (9.3 with it, 9.4 with an atomic per entry; 13.8 at 60 Hz) and 10.0 with bf16
-// multipliers and 16-bit columns (9.6).
+// (96.7k cells f32, 60 Hz mossy rate) took 15.5 us, 13.1 this way (14.1 with the four
+// added one after another instead of in pairs).  A group's single spike, the usual one at
+// low rates, skips the additions: without that branch a step took 9.6 us at 4 Hz (9.25
+// with it, 9.4 with an atomic per entry) and 10.0 with bf16 multipliers and 16-bit columns
+// (9.6).
 // Longer sums -- one per lane and projection, combined across the wavefront at the end --
 // took 13.4 us at 60 Hz where this took 13.0, 10.1 at 4 Hz (9.8), and 80 on rows without
 // groups (70).
@@ -700,11 +701,9 @@ __device__ __forceinline__ void team_groups(const TeamHead &T, const TeamPart &p
                 float wv[SC_GROUP_LOADS];
 #pragma unroll
                 for (int k = 0; k < SC_GROUP_LOADS; ++k) wv[k] = wone<WP>(val, idx[k]);
+                static_assert(SC_GROUP_LOADS == 4, "two pairs");
                 double t = (double)wv[0];
-                if (on[1]) {
-#pragma unroll
-                    for (int k = 1; k < SC_GROUP_LOADS; ++k) t += (double)(on[k] ? wv[k] : 0.f);
-                }
+                if (on[1]) t = (t + (double)wv[1]) + ((double)(on[2] ? wv[2] : 0.f) + (double)(on[3] ? wv[3] : 0.f));
                 atomicAdd(a, t);
             }
         }
