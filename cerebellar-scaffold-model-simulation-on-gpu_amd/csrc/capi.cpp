@@ -1124,7 +1124,8 @@ static int trial_time(scaffold_env *env, int T_print, int n_steps, double *ms, d
     P.R = 2 * T_print;
     int rc = plan_build(env, P);
     if (rc) return rc;
-    if (lane_synapses) *lane_synapses = P.lane_synapses;  // the values the options resolve to
+    // the values the options resolve to (0 where no number gives the same widths)
+    if (lane_synapses) *lane_synapses = P.wide_teams ? 0 : P.lane_synapses;
     if (word_groups) *word_groups = P.group_min;
     Engine *e = nullptr;
     rc = engine_create(&e, P);

@@ -184,6 +184,7 @@ struct Plan {
     int stage = 1;  // stage spike windows in LDS where the plan finds it pays
     int stage_ratio = 8;
     int lane_synapses = 8;  // team width target in effect
+    bool wide_teams = false;  // ... but teams of three quarters of it (resident runs)
     int group_min = 0;      // word-group threshold in effect (0: none)
     bool nontemporal = false;  // load the synapse streams nontemporal
     int index_bits = 32;

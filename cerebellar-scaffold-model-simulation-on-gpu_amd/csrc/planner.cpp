@@ -739,12 +739,12 @@ int plan_build(scaffold_env *env, Plan &P)
         return t;
     };
     // A network whose runs can stay resident (a block per CU, 256 at most) takes wider
-    // teams where they still fit, at three quarters of the synapses per lane: 6
-    // instead of 8 measured 141 against 149 us per 25-step call at 9.9k cells, 139
+    // teams where they still fit, at three quarters of the synapses per lane (unless the
+    // option names a number): 6 instead of 8 measured 141 against 149 us per 25-step call at 9.9k cells, 139
     // against 149 at 24k, 146 against 166 at 39k (rule-text density), 125 against 125
     // at 5.8k.
     double per_lane = P.lane_synapses;
-    if (!large && opt.resident && env->plast.empty()) {
+    if (opt.lane_synapses == 0 && !large && opt.resident && env->plast.empty()) {
         int blocks = 0;
         for (const TeamPop &T : P.teams) {
             const int per = SC_MAX_TEAM / width_for(T, 0.75 * per_lane);
@@ -758,7 +758,8 @@ int plan_build(scaffold_env *env, Plan &P)
         }
         blocks += (lanes + SC_LANE_PER_BLOCK - 1) / SC_LANE_PER_BLOCK;
         blocks += (stims + SC_STIM_PER_BLOCK - 1) / SC_STIM_PER_BLOCK;
-        if (blocks <= SC_RUN_BLOCKS) per_lane *= 0.75;
+        P.wide_teams = blocks <= SC_RUN_BLOCKS;
+        if (P.wide_teams) per_lane *= 0.75;
     }
     for (TeamPop &T : P.teams) {
         T.team_waves = width_for(T, per_lane);

@@ -243,9 +243,8 @@ int scaffold_set_input_stim_ids(scaffold_env *env, int neuron_index,
  *   "lane_synapses"     team mode: target synapses per lane (sets the team width);
  *                       0 (default): 8 when one step's synapse and state streams
  *                       fit in 64 MB (the step is latency-bound: wide teams),
- *                       else 64 (throughput-bound: more synapses per block).
- *                       Three quarters of the value where the network's runs then
- *                       still stay resident (see "resident")
+ *                       else 64 (throughput-bound: more synapses per block); 6
+ *                       where the network's runs then still stay resident
  *   "graph"             0 (default): launch every step kernel directly; 1: replay
  *                       captured hipGraphs of whole runs (on ROCm 7 the direct
  *                       launches measured as fast or faster at every size: the
@@ -552,7 +551,8 @@ int scaffold_step_timer(scaffold_env *env, int on, double *ms, int64_t *launches
  * options on env (17 trials; ms_default is the time with the environment's own
  * options, and a lane_synapses or word_groups of -1 / 0 picking by size is
  * reported as the value it resolves to for this network, so the result can be
- * applied to other networks as is).  The network's own state, seeds and
+ * applied to other networks as is; a lane_synapses of 0 stays 0 where the
+ * default widens the teams of resident runs).  The network's own state, seeds and
  * counters are untouched. */
 typedef struct {
     int32_t lane_max_fanin, lane_synapses, graph_steps;

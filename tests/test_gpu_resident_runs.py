@@ -150,3 +150,18 @@ def test_given_up_run_is_not_timed(pkg):
     assert runs(env)[1] == 1 and env.info().current_step == 400
     assert 0.5 * later < given_up < 2.0 * later
     env.finalize()
+
+
+def test_lane_synapses_as_given(pkg):
+    """A given team width holds whether runs may be resident or not; the default is wider
+    where they are."""
+    def blocks(**options):
+        env = small_env(pkg, 1, **options)
+        env.initialize(50, 25)
+        n = env.info().n_blocks
+        env.finalize()
+        return n
+
+    assert blocks(lane_synapses=8) == blocks(lane_synapses=8, resident=0)
+    assert blocks(lane_synapses=2) == blocks(lane_synapses=2, resident=0)
+    assert blocks() > blocks(resident=0) == blocks(lane_synapses=8)
