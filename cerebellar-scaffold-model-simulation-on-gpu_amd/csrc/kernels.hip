@@ -638,17 +638,18 @@ __device__ __forceinline__ float wone(const void *val, uint32_t i)
 // bits -- then one multiplier per set bit of (spikes & mask), at the group's
 // first index plus the number of mask bits below it.  The sums of up to SC_GROUP_LOADS
 // spiking entries go to the team's f64 LDS accumulator of the projection: atomics on one
-// LDS word follow each other, and with one for every spiking entry a step at strong drive
-// (96.7k cells f32, 60 Hz mossy rate) took 15.5 us, 13.1 this way (14.1 with the four
-// added one after another instead of in pairs).  A group's single spike, the usual one at
-// low rates, skips the additions: without that branch a step took 9.6 us at 4 Hz (9.25
-// with it, 9.4 with an atomic per entry) and 10.0 with bf16 multipliers and 16-bit columns
-// (9.6).
+// LDS word follow each other.  How many: more loads a batch lengthen the chain of a step
+// that is bound by latency (96.7k cells) and save rounds of one bound by throughput.
+// Loads a batch: us a step at 96.7k cells f32 4 Hz, 60 Hz / 145k / 387k / 1.55M fp8 16-bit:
+//   2: 9.5, 14.0 / 15.7 / 25.6 / 69.6     3: 9.6, 14.0 / 15.4 / 25.4 / 69.0
+//   4: 9.9, 14.5 / 15.2 / 25.4 / 68.7     5: 10.2, 15.0 / 15.0 / 25.3 / 68.7
+//   4, an atomic for every entry: 9.6, 16.2 / 15.5 / 25.4 / 70.4
+// (skipping the additions of a single spike acts like 2.)
 // Longer sums -- one per lane and projection, combined across the wavefront at the end --
 // took 13.4 us at 60 Hz where this took 13.0, 10.1 at 4 Hz (9.8), and 80 on rows without
 // groups (70).
 #define SC_GROUP_BATCH 1
-#define SC_GROUP_LOADS 4
+#define SC_GROUP_LOADS 3
 template <int WP, bool STAGED, bool NT, bool COH>
 __device__ __forceinline__ void team_groups(const TeamHead &T, const TeamPart &part, gptr<uint32_t> ring32,
                                             const uint32_t *win, const uint32_t *rowoff, uint32_t gmask, int tid,
@@ -701,10 +702,8 @@ __device__ __forceinline__ void team_groups(const TeamHead &T, const TeamPart &p
                 float wv[SC_GROUP_LOADS];
 #pragma unroll
                 for (int k = 0; k < SC_GROUP_LOADS; ++k) wv[k] = wone<WP>(val, idx[k]);
-                static_assert(SC_GROUP_LOADS == 4, "two pairs");
-                double t = (double)wv[0];
-                if (on[1]) t = (t + (double)wv[1]) + ((double)(on[2] ? wv[2] : 0.f) + (double)(on[3] ? wv[3] : 0.f));
-                atomicAdd(a, t);
+                static_assert(SC_GROUP_LOADS == 3, "the sum");
+                atomicAdd(a, (double)wv[0] + ((double)(on[1] ? wv[1] : 0.f) + (double)(on[2] ? wv[2] : 0.f)));
             }
         }
     }
