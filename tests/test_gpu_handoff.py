@@ -296,3 +296,23 @@ def test_rates_do_not_grow_with_every_stimulus(pkg):
         return sorted(times)[50]
 
     assert median(1024) < 10.0 * median(8)
+
+
+@pytest.mark.parametrize("n_input,hz", [
+    (65600, 10000.0),     # two words a thread, every bit set, the last thread's words past the end
+    (262144, 3000.0),     # four words a thread, one whole tile
+    (262209, 50.0),       # a word past it
+    (600000, 4.0),        # three tiles
+])
+def test_fired_lists_by_parts_of_a_tile(pkg, n_input, hz):
+    """Lists cut short inside a tile, at its end and in the next, both ways of asking."""
+    env = input_env(pkg, n_input, hz)
+    env.loop_n_steps(0, 2, want_output=False)
+    want = np.flatnonzero(env.spike_row(1))
+    for cap in sorted({0, 1, 5, 4095, 8192, 8193, want.size - 1, want.size, want.size + 7}):
+        if cap < 0:
+            continue
+        for query in (env.fired, env.fired_noalloc):
+            got, n = query(1, cap)
+            assert n == want.size and np.array_equal(got, want[:cap])
+    env.finalize()
