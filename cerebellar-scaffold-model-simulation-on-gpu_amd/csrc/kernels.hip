@@ -636,26 +636,25 @@ __device__ __forceinline__ float wone(const void *val, uint32_t i)
 // group's spike word -- both halves from LDS in a staged block unless its
 // projection was left in memory (gmask), each half read only where the mask has
 // bits -- then one multiplier per set bit of (spikes & mask), at the group's
-// first index plus the number of mask bits below it.  The sums of up to SC_GROUP_LOADS
-// spiking entries go to the team's f64 LDS accumulator of the projection: atomics on one
-// LDS word follow each other.  How many: more loads a batch lengthen the chain of a step
-// that is bound by latency (96.7k cells) and save rounds of one bound by throughput.
+// first index plus the number of mask bits below it.  The sums of up to 3 or 4 spiking
+// entries go to the team's f64 LDS accumulator of the projection: atomics on one LDS word
+// follow each other.  How many: more loads a batch lengthen the chain of a step that is
+// bound by latency (96.7k cells) and save rounds of one bound by throughput (networks whose
+// streams are loaded nontemporal).
 // Loads a batch: us a step at 96.7k cells f32 4 Hz, 60 Hz / 145k / 387k / 1.55M fp8 16-bit:
 //   2: 9.5, 14.0 / 15.7 / 25.6 / 69.6     3: 9.6, 14.0 / 15.4 / 25.4 / 69.0
 //   4: 9.9, 14.5 / 15.2 / 25.4 / 68.7     5: 10.2, 15.0 / 15.0 / 25.3 / 68.7
 //   4, an atomic for every entry: 9.6, 16.2 / 15.5 / 25.4 / 70.4
-// (skipping the additions of a single spike acts like 2.)
 // Longer sums -- one per lane and projection, combined across the wavefront at the end --
 // took 13.4 us at 60 Hz where this took 13.0, 10.1 at 4 Hz (9.8), and 80 on rows without
 // groups (70).
 #define SC_GROUP_BATCH 1
-#define SC_GROUP_LOADS 3
 template <int WP, bool STAGED, bool NT, bool COH>
 __device__ __forceinline__ void team_groups(const TeamHead &T, const TeamPart &part, gptr<uint32_t> ring32,
                                             const uint32_t *win, const uint32_t *rowoff, uint32_t gmask, int tid,
                                             int TT, double *acc, u32x4 rec0)
 {
-    constexpr int GB = SC_GROUP_BATCH;
+    constexpr int GB = SC_GROUP_BATCH, LOADS = NT ? 4 : 3;
     gptr<u32x4> grp = gbl(reinterpret_cast<const u32x4 *>(T.grp));
     const void *val = T.val;
     const int n = part.g1;
@@ -686,24 +685,26 @@ __device__ __forceinline__ void team_groups(const TeamHead &T, const TeamPart &p
             const uint64_t mask = ((uint64_t)g[u].w << 32) | g[u].z;
             uint64_t act = (((uint64_t)hi[u] << 32) | lo[u]) & mask;
             double *a = &acc[g[u].x >> SC_Q_SHIFT];
-            // the multipliers of up to SC_GROUP_LOADS spiking neurons are loaded
+            // the multipliers of up to LOADS spiking neurons are loaded
             // together (a slot without one reloads the group's first multiplier,
             // which exists), then added
             while (act) {
-                uint32_t idx[SC_GROUP_LOADS];
-                bool on[SC_GROUP_LOADS];
+                uint32_t idx[LOADS];
+                bool on[LOADS];
 #pragma unroll
-                for (int k = 0; k < SC_GROUP_LOADS; ++k) {
+                for (int k = 0; k < LOADS; ++k) {
                     on[k] = act != 0ull;
                     const int bit = on[k] ? __ffsll((long long)act) - 1 : 0;
                     idx[k] = g[u].y + (on[k] ? (uint32_t)__popcll(mask & ((1ull << bit) - 1ull)) : 0u);
                     act &= act - 1;
                 }
-                float wv[SC_GROUP_LOADS];
+                float wv[LOADS];
 #pragma unroll
-                for (int k = 0; k < SC_GROUP_LOADS; ++k) wv[k] = wone<WP>(val, idx[k]);
-                static_assert(SC_GROUP_LOADS == 3, "the sum");
-                atomicAdd(a, (double)wv[0] + ((double)(on[1] ? wv[1] : 0.f) + (double)(on[2] ? wv[2] : 0.f)));
+                for (int k = 0; k < LOADS; ++k) wv[k] = wone<WP>(val, idx[k]);
+                const auto w = [&](int k) { return (double)(on[k] ? wv[k] : 0.f); };
+                double t = w(0) + w(1), r = w(2);
+                if constexpr (LOADS == 4) r += w(3);
+                atomicAdd(a, t + r);
             }
         }
     }
