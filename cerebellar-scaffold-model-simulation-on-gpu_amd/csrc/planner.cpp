@@ -856,8 +856,8 @@ int plan_build(scaffold_env *env, Plan &P)
         X.skip_quiet = quiet_keeps;
         const ScPop &post = P.pops[src.post];
         // a wavefront per row idles the lanes a short row does not fill: with 2.3
-        // synapses a row (22k rows) k_plastic took 7.3 us a step, packed 2.8; rows as
-        // long as a wavefront are better off with one trigger (and one early exit) a chunk
+        // synapses a row (22k rows) k_plastic took 7.3 us a step, packed 2.8; rows nearly as
+        // long as a wavefront are even (2M synapses, 60 a row: 33.9 us a step against 33.2)
         X.packed = nnz < (int64_t)SC_WAVE * (int64_t)(src.row_ptr.size() - 1);
         for (size_t j = 0; j + 1 < src.row_ptr.size(); ++j) {
             int32_t pb = (int32_t)(post.dev_base + (int)j);  // the row's trigger
