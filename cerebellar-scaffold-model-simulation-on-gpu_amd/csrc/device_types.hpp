@@ -260,7 +260,7 @@ struct ScLayout {
 #define SC_RUN_BLOCKS 256  // blocks of a resident run on a whole MI355X (one per CU)
 // Fewest steps of a call whose runs are resident, and of such a run.  A run's start
 // (tables, the first fetch of its code, the cleared rows) and end (every block waits for
-// all) take 14 us at 9.9k cells (79 blocks) and 22 at 48k (253), those of a run launched
+// all) take 14 us at 9.9k cells (79 blocks) and 22 at 48k (225), those of a run launched
 // step by step 8; 2.1 and 1.7 us a step are gained: even at 3 and 8 steps.  50 steps in
 // runs of 5: 376 against 396 us at 9.9k cells, 426 against 405 at 24k (216 blocks), 505
 // against 461 at 48k; in runs of 13 and 12 at 48k 377 against 418.

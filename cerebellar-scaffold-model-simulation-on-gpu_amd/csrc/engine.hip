@@ -1308,7 +1308,7 @@ int engine_run_output(Engine *e, int n_steps, int use_graph, int graph_steps, in
             launch_out_train(e->stream, e->hi.ring, e->hi.Wr, R, row0, e->T_out, e->out_bits, e->n_out, out.out);
             HIP_TRY(hipGetLastError());
         }
-        *train = e->out_h;  // complete once engine_finish has synchronized the stream
+        *train = e->out_h;  // complete once engine_finish has waited for its signal or the stream
     }
     bool recovered = false;
     const unsigned long long upto = !train ? e->stats_seq : early ? early : kNoSignal;

@@ -1318,9 +1318,9 @@ __global__ void __launch_bounds__(SC_BLOCK) __attribute__((amdgpu_waves_per_eu(8
 // the gathers.  Hence the split: the longer delays' windows are copied by one
 // wavefront while another updates the neurons, one-step spikes travel in the line
 // that is polled for them instead of through the ring, each lane keeps its first
-// synapse record.  Measured per call of 25 steps, against a launch per step of the
-// same build: 125 against 180 us at 5.8k cells, 149 against 184 at 9.9k, 149 against
-// 198 at 24k, 145 against 200 at 48k (253 blocks).
+// synapse record.  Measured per call of 25 steps (loop_n_steps alone, no hand-off),
+// against a launch per step of the same build: 128 against 165 us at 5.8k cells, 142
+// against 177 at 9.9k, 141 against 191 at 24k, 143 against 192 at 48k (253 blocks).
 #define SC_RUN_GIVEN_UP 0x80000000u
 __device__ __forceinline__ uint32_t ld_agent(const uint32_t *p)
 {
@@ -1805,8 +1805,8 @@ __device__ __forceinline__ void run_lane_dispatch(const ScLaneTask *t, bool has,
 // 128 VGPRs and one block per CU (256 blocks).  With 64 VGPRs two blocks share a CU
 // and networks of up to 512 blocks fit, but the loop-carried values spill and the
 // blocks of a CU share its issue slots: at 96.7k cells (501 blocks) such a run took
-// 241 us per 25-step call against 248 with a launch per step, not worth a second
-// instantiation; at 9.9k cells 172 against 154 with 128 VGPRs.
+// 297 us per 25-step call against 248 with a launch per step; at 9.9k cells 182 against
+// 142 with 128 VGPRs.
 template <bool IDX16>
 __global__ void __launch_bounds__(SC_BLOCK) __attribute__((amdgpu_waves_per_eu(4, 4)))
 k_run(ScInstance I0, ScLayout L, const ScLaneTask *__restrict__ lanes,
@@ -2314,7 +2314,7 @@ __global__ void __launch_bounds__(256) k_plastic(ScInstance I, ScPlastic P, int 
 // and leave in whole lines, as `out` is host memory: stored one by one by the words'
 // owners they would be a bus transaction each.  Bound by the launch and the bus: a query
 // of a 97k-cell network takes 17 us; with the ids in allocated device memory, copied out,
-// it took 56.
+// it took 50.
 constexpr int kFiredIds = 8192, kFiredWords = 4;
 __global__ void __launch_bounds__(1024) k_fired(const uint64_t *__restrict__ row, int n_groups,
                                                 const ScGroup *__restrict__ groups, int32_t *__restrict__ out,

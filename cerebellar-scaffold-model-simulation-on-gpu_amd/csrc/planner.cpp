@@ -740,9 +740,9 @@ int plan_build(scaffold_env *env, Plan &P)
     };
     // A network whose runs can stay resident (a block per CU, 256 at most) takes wider
     // teams where they still fit, at three quarters of the synapses per lane (unless the
-    // option names a number): 6 instead of 8 measured 141 against 149 us per 25-step call at 9.9k cells, 139
-    // against 149 at 24k, 146 against 166 at 39k (rule-text density), 125 against 125
-    // at 5.8k.
+    // option names a number): 6 instead of 8 measured 142
+    // against 153 us per 25-step call at 9.9k cells, 141 against 150 at 24k, 147 against
+    // 165 at 39k (rule-text density), 128 against 127 at 5.8k.
     double per_lane = P.lane_synapses;
     if (opt.lane_synapses == 0 && !large && opt.resident && env->plast.empty()) {
         int blocks = 0;
